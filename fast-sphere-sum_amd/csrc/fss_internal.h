@@ -230,6 +230,12 @@ struct Sal {
     int64_t adam_t = 0;
 };
 
+// Workspace of the remesh: missed targets, counters, and the triangle bins of
+// the full search.
+struct Remesh {
+    DevBuf miss, cnt, tri, count, start, scan, place, cap, bin, odd;
+};
+
 struct Timing {
     static constexpr int RING = 256;
     hipEvent_t ev[RING][5] = {}; // + [4]: start of the far-field (proxy) kernel
@@ -257,6 +263,7 @@ struct fss_ctx {
     fss::Tree tree;
     fss::Timing timing;
     fss::Sal sal;
+    fss::Remesh remesh;
 
     // device constants
     fss::DevBuf d_lu, d_perm, d_vinv, d_pts;

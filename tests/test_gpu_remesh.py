@@ -61,3 +61,44 @@ def test_remesh_after_rk4_steps_conserves_circulation_roughly(fsslib):
     m0 = np.sum((adv + 2 * om * st[2].cpu().numpy()) * area)
     m1 = np.sum((vo + 2 * om * z) * area)
     assert abs(m1 - m0) < 1e-2 * np.sum(np.abs(adv) * area)
+
+
+def _distorted(fsslib, kind):
+    """Advected meshes whose triangles leave the bins of the full search: folded
+    over (large displacement), collapsed and nearly collapsed edges (singular and
+    ill-conditioned triangles), one patch shrunk so that its neighbours are
+    stretched over many cells."""
+    x, y, z, tris = fsslib.grid_icosahedral(4)
+    p = np.stack((x, y, z), 1)
+    rng = np.random.default_rng(11)
+    p = p + 0.004 * rng.normal(size=p.shape)  # targets off the mesh edges
+    if kind == "fold":
+        p = p + 0.12 * rng.normal(size=p.shape)
+    elif kind == "collapse":
+        for k, t in enumerate(rng.choice(len(tris), 60, replace=False)):
+            a, b, _ = tris[t]
+            p[a] = p[b] + (0, 1e-14, 1e-9)[k % 3] * rng.normal(size=3)
+    else:
+        near = p @ p[0] > 0.9
+        p[near] = p[0] + 0.02 * (p[near] - p[0])
+    return (x, y, z), p / np.linalg.norm(p, axis=1)[:, None], tris
+
+
+@pytest.mark.parametrize("kind", ["fold", "collapse", "stretch"])
+def test_remesh_full_search_of_distorted_meshes(fsslib, kind):
+    """No adjacency at all, so every target takes the full search: the same
+    (lowest-index) triangle as the oracle's scan."""
+    import torch
+    (x, y, z), p, tris = _distorted(fsslib, kind)
+    n = len(x)
+    off, idx = np.zeros(n + 1, np.int32), np.zeros(1, np.int32)
+    ax, ay, az = (np.ascontiguousarray(c) for c in p.T)
+    av = np.sin(3 * ax) + 0.3 * ay
+    want_v, _, want_tri, want_nf = oracle.remesh(ax, ay, az, av, tris, off, idx, x, y, z)
+    print(f"remesh {kind}: n={n} fallbacks={want_nf}", flush=True)
+    d = lambda a: torch.from_numpy(np.ascontiguousarray(a)).cuda()
+    got_v, _, got_tri, nf = fsslib.Context().remesh(d(ax), d(ay), d(az), d(av), d(tris.astype(np.int32)), d(off),
+                                                    d(idx), d(x), d(y), d(z), tri_out=True)
+    assert nf == want_nf == n
+    np.testing.assert_array_equal(got_tri.cpu().numpy(), want_tri)
+    np.testing.assert_allclose(got_v.cpu().numpy(), want_v, rtol=0, atol=1e-15 * np.abs(want_v).max())
