@@ -60,10 +60,32 @@ __device__ inline void interp(const int32_t *tv, const double *c, const double *
     if (atr) *tr_out = b0 * atr[tv[0]] + b1 * atr[tv[1]] + b2 * atr[tv[2]];
 }
 
-// Adjacent triangles of the target's vertex, eight lanes per target: every lane
-// solves one triangle of the list and the first hit in list order wins, so a
-// target waits for one solve in place of up to six in a row (a thread per
-// target: 24 us at 163,842 targets).  Misses go to the fallback list.
+// False only where the solve cannot make p a non-negative combination of the
+// vertices.  Its coordinates are exact for vertices perturbed by a small
+// multiple of 1e-16 of the largest one (LU with pivoting is backward stable), and
+// coordinate m times the determinant is p . (v_{m+1} x v_{m+2}): two of these
+// with opposite signs beyond 1e-12 |p| max|v|^2 keep opposite signs under any such
+// perturbation.  A matrix that could be singular under one (its solve stops at a
+// zero pivot and leaves p in place of coordinates) and anything not finite are
+// left to the solve.
+__device__ inline bool may_hold(const double *v, const double *p)
+{
+    double f[3], vv = 0, det = 0;
+    for (int m = 0; m < 3; m++) {
+        const double *a = v + 3 * ((m + 1) % 3), *b = v + 3 * ((m + 2) % 3);
+        const double c0 = a[1] * b[2] - a[2] * b[1], c1 = a[2] * b[0] - a[0] * b[2], c2 = a[0] * b[1] - a[1] * b[0];
+        f[m] = p[0] * c0 + p[1] * c1 + p[2] * c2;
+        vv = fmax(vv, a[0] * a[0] + a[1] * a[1] + a[2] * a[2]);
+        if (m == 0) det = v[0] * c0 + v[1] * c1 + v[2] * c2;
+    }
+    const double tol = 1e-12 * vv * (fabs(p[0]) + fabs(p[1]) + fabs(p[2]));
+    return !(det * det > 1e-24 * vv * vv * vv && fmin(f[0], fmin(f[1], f[2])) < -tol && fmax(f[0], fmax(f[1], f[2])) > tol);
+}
+
+// Adjacent triangles of the target's vertex; misses go to the fallback list.
+// A target first walks to a triangle that may hold it and then solves, so the
+// targets of a wave solve together and nearly always once (163,842 targets: 21.7
+// us; solving every triangle on the way 24.3, eight lanes a target 25.9).
 __global__ void __launch_bounds__(256) k_remesh_adjacent(
     int64_t n, const double *__restrict__ ax, const double *__restrict__ ay, const double *__restrict__ az,
     const double *__restrict__ avort, const double *__restrict__ atr, const int32_t *__restrict__ tris,
@@ -71,30 +93,27 @@ __global__ void __launch_bounds__(256) k_remesh_adjacent(
     const double *__restrict__ y, const double *__restrict__ z, double omega, double *vort, double *tr,
     int32_t *tri_out, int32_t *miss, unsigned long long *nmiss)
 {
-    const int64_t i = ((int64_t)blockIdx.x * blockDim.x + threadIdx.x) >> 3;
-    const int l = threadIdx.x & 7, sh = threadIdx.x & 56;
+    const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
     if (i >= n) return;
     const double p[3] = {x[i], y[i], z[i]};
+    double v[9], c[3];
+    int32_t tv[3], t = -1;
+    int32_t j = vt_off[i];
     const int32_t end = vt_off[i + 1];
-    for (int32_t j = vt_off[i]; j < end; j += 8) {
-        double v[9], c[3];
-        int32_t tv[3], t = -1;
-        bool hit = false;
-        if (j + l < end) {
-            t = vt_idx[j + l];
+    for (;;) {
+        bool may = false;
+        while (j < end && !may) {
+            t = vt_idx[j++];
             load_tri(tris, t, ax, ay, az, tv, v);
-            hit = in_tri(v, p, c);
+            may = may_hold(v, p);
         }
-        const uint32_t m = (uint32_t)(__ballot(hit) >> sh) & 255u;
-        if (m) {
-            if (l == __ffs(m) - 1) {
-                interp(tv, c, az, avort, atr, p[2], omega, &vort[i], tr ? &tr[i] : nullptr);
-                tri_out[i] = t;
-            }
+        if (!may) break;
+        if (in_tri(v, p, c)) {
+            interp(tv, c, az, avort, atr, p[2], omega, &vort[i], tr ? &tr[i] : nullptr);
+            tri_out[i] = t;
             return;
         }
     }
-    if (l) return;
     tri_out[i] = -1;
     unsigned long long q = atomicAdd(nmiss, 1ull);
     miss[q] = (int32_t)i;
@@ -113,69 +132,81 @@ __global__ void __launch_bounds__(256) k_remesh_adjacent(
 //
 // The solve rounds: a triangle also "contains" a target that rounding puts
 // there.  With condition number k of the vertex matrix the coordinates are off
-// by a small multiple of 1e-16 k relative to the largest, so below k = 1e8
-// coordinates that come out non-negative are above -1e-6 of the largest one and the
-// target is within 1.00001 of the triangle's size of its centre: the caps are
-// 1.05 times as large.  Triangles that are worse conditioned, not finite, or
+// by a small multiple of 1e-16 k relative to the largest, so below k = 1e6
+// coordinates that come out non-negative are above -1e-8 of the largest one and the
+// target is within 1.0000001 of the triangle's size of its centre: the caps are
+// 1.05 times as large, and 2e-6 for their rounding to FP32.  Triangles that are worse conditioned, not finite, or
 // larger than the cells (RM_CAP) stay on a list that every target solves.
 struct RmGrid {
     int G;       // cells per dimension
-    double inv;  // cells per unit length
-    double rmax; // largest chord radius that is binned
+    float inv;   // cells per unit length
+    float rmax;  // largest chord radius that is binned
 };
 
-__device__ inline int rm_cell1(const RmGrid &g, double x)
+__device__ inline int rm_cell1(const RmGrid &g, float x)
 {
-    const int k = (int)((x + 1.0) * g.inv);
+    const int k = (int)((x + 1.0f) * g.inv);
     return k < 0 ? 0 : k < g.G ? k : g.G - 1;
 }
 
 // unit vector of p; false where there is none
-__device__ inline bool rm_unit(const double *p, double *u)
+__device__ inline bool rm_unit(const double *p, float *u)
 {
-    const double r = sqrt(p[0] * p[0] + p[1] * p[1] + p[2] * p[2]);
-    for (int k = 0; k < 3; k++) u[k] = p[k] / r;
-    return r > 0 && r < 1e150;
+    const double q = p[0] * p[0] + p[1] * p[1] + p[2] * p[2];
+    const float r = rsqrtf((float)q);
+    for (int k = 0; k < 3; k++) u[k] = (float)p[k] * r;
+    return q > 1e-30 && q < 1e30;
 }
 
-// cap of a triangle: unit axis and the chord from it to the furthest vertex
-// direction; false where the triangle is not to be binned
-__device__ inline bool rm_cap(const double *v, double *axis, double &chord)
+// Cap of a triangle in FP32: unit axis and the chord from it to the furthest
+// vertex direction, each off by less than 1e-6 (the searches add that); false
+// where the triangle is not to be binned.  The condition number is estimated
+// from edge differences formed in FP64; the line is drawn at 1e6, where their
+// FP32 products still tell.
+__device__ inline bool rm_cap(const double *v, float *axis, float &chord)
 {
-    double u[9], s[3];
+    float u[9], s[3];
     bool ok = rm_unit(v, u) && rm_unit(v + 3, u + 3) && rm_unit(v + 6, u + 6);
     for (int k = 0; k < 3; k++) s[k] = u[k] + u[3 + k] + u[6 + k];
-    ok = ok && rm_unit(s, axis);
-    double d2 = 0, cmax = 0, det = 0, len = 0;
+    const float q = s[0] * s[0] + s[1] * s[1] + s[2] * s[2], r = rsqrtf(q);
+    float d2 = 0, e[9];
+    for (int k = 0; k < 3; k++) axis[k] = s[k] * r;
     for (int m = 0; m < 3; m++) {
-        double q = 0;
-        for (int k = 0; k < 3; k++) q += (u[3 * m + k] - axis[k]) * (u[3 * m + k] - axis[k]);
-        d2 = fmax(d2, q);
-        // rows of the inverse vertex matrix, times the determinant
-        const double *a = v + 3 * ((m + 1) % 3), *b = v + 3 * ((m + 2) % 3), *w = v + 3 * m;
-        const double c0 = a[1] * b[2] - a[2] * b[1], c1 = a[2] * b[0] - a[0] * b[2], c2 = a[0] * b[1] - a[1] * b[0];
-        cmax = fmax(cmax, sqrt(c0 * c0 + c1 * c1 + c2 * c2));
-        len = fmax(len, sqrt(w[0] * w[0] + w[1] * w[1] + w[2] * w[2]));
-        if (m == 0) det = w[0] * c0 + w[1] * c1 + w[2] * c2;
+        float d = 0;
+        for (int k = 0; k < 3; k++) {
+            d += (u[3 * m + k] - axis[k]) * (u[3 * m + k] - axis[k]);
+            e[3 * m + k] = (float)(v[(3 * m + 3 + k) % 9] - v[3 * m + k]);
+        }
+        d2 = fmaxf(d2, d);
     }
-    chord = sqrt(d2);
-    return ok && 3.0 * len * cmax < 1e8 * fabs(det); // false for anything not finite
+    chord = sqrtf(d2);
+    // |v_j x v_k| <= |v| |edge|, det = v_0 . (e_0 x e_1)
+    float len2 = 0, edge2 = 0;
+    for (int m = 0; m < 3; m++) {
+        const float w0 = (float)v[3 * m], w1 = (float)v[3 * m + 1], w2 = (float)v[3 * m + 2];
+        len2 = fmaxf(len2, w0 * w0 + w1 * w1 + w2 * w2);
+        edge2 = fmaxf(edge2, e[3 * m] * e[3 * m] + e[3 * m + 1] * e[3 * m + 1] + e[3 * m + 2] * e[3 * m + 2]);
+    }
+    const float det = (float)v[0] * (e[1] * e[5] - e[2] * e[4]) + (float)v[1] * (e[2] * e[3] - e[0] * e[5]) +
+                      (float)v[2] * (e[0] * e[4] - e[1] * e[3]);
+    return ok && q > 0.1f && 3.0f * len2 * sqrtf(edge2) < 1e6f * fabsf(det); // false for anything not finite
 }
 
 __global__ void __launch_bounds__(256) k_remesh_bin(int64_t ntri, const double *__restrict__ ax,
                                                     const double *__restrict__ ay, const double *__restrict__ az,
                                                     const int32_t *__restrict__ tris, RmGrid g, int32_t *count,
-                                                    int2 *place, double4 *cap, int32_t *odd, unsigned int *nodd)
+                                                    int2 *place, float4 *cap, int32_t *odd, unsigned int *nodd)
 {
     const int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
     if (t >= ntri) return;
     int32_t tv[3];
-    double v[9], a[3] = {0, 0, 0}, chord = 0;
+    double v[9];
+    float a[3], chord;
     load_tri(tris, t, ax, ay, az, tv, v);
     if (rm_cap(v, a, chord) && chord <= g.rmax) {
         const int c = (rm_cell1(g, a[2]) * g.G + rm_cell1(g, a[1])) * g.G + rm_cell1(g, a[0]);
         place[t] = make_int2(c, atomicAdd(&count[c], 1));
-        cap[t] = make_double4(a[0], a[1], a[2], chord);
+        cap[t] = make_float4(a[0], a[1], a[2], chord);
     } else {
         place[t] = make_int2(-1, 0);
         odd[atomicAdd(nodd, 1u)] = (int32_t)t;
@@ -194,7 +225,7 @@ __global__ void __launch_bounds__(256) k_remesh_full(
     const int32_t *__restrict__ miss, int64_t nmiss, const double *__restrict__ ax, const double *__restrict__ ay,
     const double *__restrict__ az, const double *__restrict__ avort, const double *__restrict__ atr,
     const int32_t *__restrict__ tris, RmGrid g, const int32_t *__restrict__ start, const int32_t *__restrict__ bin,
-    const double4 *__restrict__ cap, const int32_t *__restrict__ odd, const unsigned int *__restrict__ nodd,
+    const float4 *__restrict__ cap, const int32_t *__restrict__ odd, const unsigned int *__restrict__ nodd,
     const double *__restrict__ x, const double *__restrict__ y, const double *__restrict__ z, double omega,
     double *vort, double *tr, int32_t *tri_out, unsigned long long *nbad)
 {
@@ -203,15 +234,16 @@ __global__ void __launch_bounds__(256) k_remesh_full(
     const int lane = threadIdx.x & 63;
     const int64_t i = miss[w];
     const double p[3] = {x[i], y[i], z[i]};
-    double v[9], c[3], u[3];
+    double v[9], c[3];
+    float u[3];
     int32_t tv[3], best = INT32_MAX;
     auto test = [&](int32_t t) {
         if (t >= best) return;
         load_tri(tris, t, ax, ay, az, tv, v);
-        if (in_tri(v, p, c)) best = t;
+        if (may_hold(v, p) && in_tri(v, p, c)) best = t;
     };
     if (rm_unit(p, u)) {
-        const double q = 1.05 * g.rmax + 1e-9;
+        const float q = 1.05f * g.rmax + 4e-6f;
         int lo[3], hi[3];
         for (int k = 0; k < 3; k++) {
             lo[k] = rm_cell1(g, u[k] - q);
@@ -224,8 +256,8 @@ __global__ void __launch_bounds__(256) k_remesh_full(
                 const int32_t e = start[row + hi[0] + 1];
                 for (int32_t k = start[row + lo[0]] + lane; k < e; k += 64) {
                     const int32_t t = bin[k];
-                    const double4 a = cap[t];
-                    const double dx = u[0] - a.x, dy = u[1] - a.y, dz = u[2] - a.z, r = 1.05 * a.w + 1e-9;
+                    const float4 a = cap[t];
+                    const float dx = u[0] - a.x, dy = u[1] - a.y, dz = u[2] - a.z, r = 1.05f * a.w + 2e-6f;
                     if (dx * dx + dy * dy + dz * dz <= r * r) test(t);
                 }
             }
@@ -257,8 +289,8 @@ static RmGrid rm_grid(int64_t ntri)
     const double r0 = std::sqrt(4 * M_PI / (1.3 * (double)ntri)), rmax = std::min(0.5, 4 * r0);
     RmGrid g;
     g.G = (int)std::max(1.0, std::min((double)RM_MAX_G, std::floor(2.0 / (2.1 * rmax))));
-    g.inv = g.G / 2.0;
-    g.rmax = rmax;
+    g.inv = g.G / 2.0f;
+    g.rmax = (float)rmax;
     return g;
 }
 
@@ -282,7 +314,7 @@ fss_status remesh(fss_ctx *ctx, const double *ax, const double *ay, const double
     FSS_HIP(hipMemsetAsync(W.cnt.p, 0, sizeof(unsigned long long) * 3, s));
     unsigned long long *c = W.cnt.as<unsigned long long>();
     int32_t *miss = W.miss.as<int32_t>();
-    hipLaunchKernelGGL(k_remesh_adjacent, dim3((unsigned)div_up(8 * n, 256)), dim3(256), 0, s, n, ax, ay, az, avort,
+    hipLaunchKernelGGL(k_remesh_adjacent, dim3((unsigned)div_up(n, 256)), dim3(256), 0, s, n, ax, ay, az, avort,
                        atr, tris, vt_off, vt_idx, x, y, z, omega, vort, tr, to, miss, c);
     FSS_HIP(hipGetLastError());
     unsigned long long h[2] = {0, 0};
@@ -297,21 +329,21 @@ fss_status remesh(fss_ctx *ctx, const double *ax, const double *ay, const double
         FSS_TRY(W.start.ensure(sizeof(int32_t) * (nc + 1)));
         FSS_TRY(W.scan.ensure(tmp));
         FSS_TRY(W.place.ensure(sizeof(int2) * ntri));
-        FSS_TRY(W.cap.ensure(sizeof(double4) * ntri));
+        FSS_TRY(W.cap.ensure(sizeof(float4) * ntri));
         FSS_TRY(W.bin.ensure(sizeof(int32_t) * ntri));
         FSS_TRY(W.odd.ensure(sizeof(int32_t) * ntri));
         unsigned int *nodd = reinterpret_cast<unsigned int *>(c + 2);
         const dim3 gt((unsigned)div_up(ntri, 256));
         FSS_HIP(hipMemsetAsync(W.count.p, 0, sizeof(int32_t) * (nc + 1), s));
         hipLaunchKernelGGL(k_remesh_bin, gt, dim3(256), 0, s, ntri, ax, ay, az, tris, g, W.count.as<int32_t>(),
-                           W.place.as<int2>(), W.cap.as<double4>(), W.odd.as<int32_t>(), nodd);
+                           W.place.as<int2>(), W.cap.as<float4>(), W.odd.as<int32_t>(), nodd);
         FSS_HIP(hipcub::DeviceScan::ExclusiveSum(W.scan.p, tmp, W.count.as<int32_t>(), W.start.as<int32_t>(),
                                                  (int)(nc + 1), s));
         hipLaunchKernelGGL(k_remesh_sort, gt, dim3(256), 0, s, ntri, W.place.as<int2>(), W.start.as<int32_t>(),
                            W.bin.as<int32_t>());
         hipLaunchKernelGGL(k_remesh_full, dim3((unsigned)div_up((int64_t)h[0], 4)), dim3(256), 0, s, miss, (int64_t)h[0],
                            ax, ay, az, avort, atr, tris, g, W.start.as<int32_t>(), W.bin.as<int32_t>(),
-                           W.cap.as<double4>(), W.odd.as<int32_t>(), nodd, x, y, z, omega, vort, tr, to, c + 1);
+                           W.cap.as<float4>(), W.odd.as<int32_t>(), nodd, x, y, z, omega, vort, tr, to, c + 1);
         FSS_HIP(hipGetLastError());
         FSS_HIP(hipMemcpyAsync(h + 1, c + 1, sizeof(unsigned long long), hipMemcpyDeviceToHost, s));
         FSS_HIP(hipStreamSynchronize(s));
