@@ -129,11 +129,11 @@ template <class T> struct Merged {
         used += add;
         return FSS_OK;
     }
-    fss_status copy(const DevBuf &src, int64_t n, hipStream_t s)
+    fss_status copy(const T *src, int64_t n, hipStream_t s)
     {
         T *d;
         FSS_TRY(reserve(n, s, &d));
-        if (n > 0) FSS_HIP(hipMemcpyAsync(d, src.p, sizeof(T) * n, hipMemcpyDeviceToDevice, s));
+        if (n > 0) FSS_HIP(hipMemcpyAsync(d, src, sizeof(T) * n, hipMemcpyDeviceToDevice, s));
         return FSS_OK;
     }
 };
@@ -159,8 +159,9 @@ fss_status batch_build(fss_ctx *ctx, int ninst, const int64_t *ns, const int *le
     Merged<Range> ra, rb;
     std::vector<Instance> inst(ninst);
     fss_tree_stats tot{};
-    // running bases: particles, records, nodes, near output slots, L x n
-    int64_t pb = 0, P0 = 0, NN = 0, NO = 0, LN = 0;
+    // running bases: particles, records, nodes, near output slots, L x n, entries
+    // of the near and far source lists
+    int64_t pb = 0, P0 = 0, NN = 0, NO = 0, LN = 0, NSn = 0, NSf = 0;
     int Lmax = 0;
     for (int k = 0; k < ninst; k++) {
         if (ns[k] < 1) return set_error("batch: every instance needs n >= 1"), FSS_ERR_INVALID;
@@ -182,7 +183,7 @@ fss_status batch_build(fss_ctx *ctx, int ninst, const int64_t *ns, const int *le
         FSS_TRY(recnode.reserve(T.p0, s, &d32));
         hipLaunchKernelGGL(k_app_i32, dim3(grid_of(T.p0)), dim3(256), 0, s, T.recnode.as<int32_t>(), T.p0, nbase, 0,
                            d32);
-        FSS_TRY(rinfo.copy(T.rinfo, T.p0, s));
+        FSS_TRY(rinfo.copy(T.rinfo.as<uint8_t>(), T.p0, s));
         FSS_TRY(ipos.reserve(T.n, s, &d32));
         hipLaunchKernelGGL(k_app_i32, dim3(grid_of(T.n)), dim3(256), 0, s, T.ipos.as<int32_t>(), T.n, sbase, 0, d32);
         FSS_TRY(oslot.reserve(T.nn, s, &d32));
@@ -191,13 +192,17 @@ fss_status batch_build(fss_ctx *ctx, int ninst, const int64_t *ns, const int *le
         int4 *d4;
         FSS_TRY(nrange.reserve(T.nn, s, &d4));
         hipLaunchKernelGGL(k_app_nrange, dim3(grid_of(T.nn)), dim3(256), 0, s, T.nrange.as<int4>(), T.nn, sbase, d4);
-        FSS_TRY(counts.copy(T.counts, T.nn, s));
-        const int64_t ln = (int64_t)T.L * T.n;
-        FSS_TRY(inv.reserve(ln, s, &d32));
-        hipLaunchKernelGGL(k_app_i32, dim3(grid_of(ln)), dim3(256), 0, s, T.inv_active.as<int32_t>(), ln, obase, 1,
-                           d32);
-        FSS_TRY(nodeof.reserve(ln, s, &d32));
-        hipLaunchKernelGGL(k_app_i32, dim3(grid_of(ln)), dim3(256), 0, s, T.nodeof.as<int32_t>(), ln, nbase, 1, d32);
+        FSS_TRY(counts.copy(T.counts.as<int32_t>(), T.nn, s));
+        // maps of the memberships outside the main paths, where there are any
+        const int64_t ln = T.p0 > T.n ? (int64_t)T.L * T.n : 0, loff = inv.used;
+        if (ln > 0) {
+            FSS_TRY(inv.reserve(ln, s, &d32));
+            hipLaunchKernelGGL(k_app_i32, dim3(grid_of(ln)), dim3(256), 0, s, T.inv_active.as<int32_t>(), ln, obase, 1,
+                               d32);
+            FSS_TRY(nodeof.reserve(ln, s, &d32));
+            hipLaunchKernelGGL(k_app_i32, dim3(grid_of(ln)), dim3(256), 0, s, T.nodeof.as<int32_t>(), ln, nbase, 1,
+                               d32);
+        }
         FSS_TRY(node_slot.reserve(T.nn, s, &d32));
         hipLaunchKernelGGL(k_app_i32, dim3(grid_of(T.nn)), dim3(256), 0, s, T.node_slot.as<int32_t>(), T.nn, slbase,
                            1, d32);
@@ -205,9 +210,9 @@ fss_status batch_build(fss_ctx *ctx, int ninst, const int64_t *ns, const int *le
         if (T.n_charge > 0)
             hipLaunchKernelGGL(k_app_i32, dim3(grid_of(T.n_charge)), dim3(256), 0, s, T.charge_nodes.as<int32_t>(),
                                T.n_charge, nbase, 0, d32);
-        FSS_TRY(tri_info.copy(T.tri_info, 4 * T.nn, s));
-        FSS_TRY(tri_xyz.copy(T.tri_xyz, 9 * T.nn, s));
-        FSS_TRY(proxy.copy(T.proxy_xyz, T.nn * p, s));
+        FSS_TRY(tri_info.copy(T.d_info, 4 * T.nn, s));
+        FSS_TRY(tri_xyz.copy(T.d_xyz, 9 * T.nn, s));
+        FSS_TRY(proxy.copy(T.proxy_xyz.as<double4>(), T.nn * p, s));
         NearItem *dn;
         FSS_TRY(near.reserve(T.n_near, s, &dn));
         if (T.n_near > 0)
@@ -233,7 +238,7 @@ fss_status batch_build(fss_ctx *ctx, int ninst, const int64_t *ns, const int *le
             hipLaunchKernelGGL(k_app_range, dim3(grid_of(T.n_rb)), dim3(256), 0, s, T.ranges_b.as<Range>(), T.n_rb,
                                T.p0, p, sbase, nbase, dr);
         FSS_HIP(hipGetLastError());
-        inst[k] = Instance{pb, T.n, LN, T.L, 0, sbase, nbase};
+        inst[k] = Instance{pb, T.n, loff, T.L, 0, sbase, nbase};
         const fss_tree_stats &ps = T.stats;
         tot.n_interactions += ps.n_interactions;
         for (int t = 0; t < 4; t++) tot.n_type[t] += ps.n_type[t];
@@ -245,7 +250,9 @@ fss_status batch_build(fss_ctx *ctx, int ninst, const int64_t *ns, const int *le
         P0 += T.p0;
         NN += T.nn;
         NO += T.nslot_out;
-        LN += ln;
+        LN += (int64_t)T.L * T.n;
+        NSn += T.n_near_src;
+        NSf += T.n_far_src;
         // the next instance's build reuses the tree buffers: the appends above
         // are on the same stream, so they read this instance's data first
     }
@@ -271,6 +278,8 @@ fss_status batch_build(fss_ctx *ctx, int ninst, const int64_t *ns, const int *le
     T.n_ra = ra.used;
     T.n_rb = rb.used;
     T.n_charge = charge.used;
+    T.n_near_src = NSn;
+    T.n_far_src = NSf;
     T.pairs_near = tot.pairs_near;
     T.pairs_far = tot.pairs_far;
     T.ninst = ninst;
@@ -303,10 +312,9 @@ fss_status batch_build(fss_ctx *ctx, int ninst, const int64_t *ns, const int *le
     T.loc.release();
     T.found.release();
     T.inter.release();
-    T.ids.release();
-    T.offsets.release();
     FSS_HIP(hipStreamSynchronize(s));
     FSS_TRY(plan_finish(ctx));
+    build_scratch_trim(ctx->build);
     T.built = true;
     return FSS_OK;
 }

@@ -1186,12 +1186,12 @@ static fss_status upward(fss_ctx *ctx, typename Rec<Real>::T4 *src)
     const int64_t ns = T.n_up_small, nl = T.n_up - ns;
     if (ns > 0)
         hipLaunchKernelGGL((k_upward_pair<Real, D>), dim3((unsigned)div_up(div_up(ns, 2), 4)), dim3(256), 0, s,
-                           T.up_items.as<int4>(), ns, T.recnode.as<int32_t>(), T.tri_info.as<double>(),
-                           T.tinv.as<double>(), ctx->d_vinv.as<double>(), p0, src, part);
+                           T.up_items.as<int4>(), ns, T.recnode.as<int32_t>(), T.d_info,
+                           T.d_tinv, ctx->d_vinv.as<double>(), p0, src, part);
     if (nl > 0)
         hipLaunchKernelGGL((k_upward<Real, D>), dim3((unsigned)div_up(nl, 4)), dim3(256), 0, s,
-                           T.up_items.as<int4>() + ns, nl, T.recnode.as<int32_t>(), T.tri_info.as<double>(),
-                           T.tinv.as<double>(), ctx->d_vinv.as<double>(), p0, src, part);
+                           T.up_items.as<int4>() + ns, nl, T.recnode.as<int32_t>(), T.d_info,
+                           T.d_tinv, ctx->d_vinv.as<double>(), p0, src, part);
     if (T.n_up_multi > 0)
         hipLaunchKernelGGL((k_upward_finish<Real, D>), dim3((unsigned)div_up(T.n_up_multi, 4)), dim3(256), 0, s,
                            T.up_multi.as<int4>(), T.n_up_multi, part, ctx->d_vinv.as<double>(), p0, src);
@@ -1226,7 +1226,7 @@ static fss_status run_degree(fss_ctx *ctx, const fss_particles *pp, fss_velocity
         {
             hipLaunchKernelGGL((k_proxy_list<double, D>), dim3((unsigned)div_up(T.n_proxy, 4)), dim3(256), 0, s,
                                T.proxy_items.as<ProxyItem>(), T.n_proxy, T.far_off.as<int64_t>(), T.far_src.as<int32_t>(), src,
-                               T.recnode.as<int32_t>(), (const float *)nullptr, p0, T.tri_info.as<double>(),
+                               T.recnode.as<int32_t>(), (const float *)nullptr, p0, T.d_info,
                                T.proxy_xyz.as<double4>(), ctx->phi.as<double>());
         }
         if (ev) FSS_HIP(hipEventRecord(ev[1], s));
@@ -1236,7 +1236,7 @@ static fss_status run_degree(fss_ctx *ctx, const fss_particles *pp, fss_velocity
                            : (ctx->near_r == 2 ? k_near<double, 2, false> : k_near<double, 4, false>);
             hipLaunchKernelGGL(kn, dim3((unsigned)T.n_near), dim3(64), 0, s, T.near_items.as<NearItem>(),
                                T.near_src.as<int32_t>(), src, T.recid.as<int32_t>(), T.recnode.as<int32_t>(), p0, p,
-                               T.tri_info.as<double>(), pp->x, pp->y, pp->z, ost, ctx->out3.as<double>());
+                               T.d_info, pp->x, pp->y, pp->z, ost, ctx->out3.as<double>());
         }
         if (ev) FSS_HIP(hipEventRecord(ev[2], s));
     } else {
@@ -1245,7 +1245,7 @@ static fss_status run_degree(fss_ctx *ctx, const fss_particles *pp, fss_velocity
         float *aoff = reinterpret_cast<float *>(src + nsrc);
         hipLaunchKernelGGL(k_gather32, dim3(gs), dim3(256), 0, s, pp->x, pp->y, pp->z, pp->vort,
                            pp->area, T.recid.as<int32_t>(), p0, T.proxy_xyz.as<double4>(), nprox, p,
-                           T.recnode.as<int32_t>(), T.tri_info.as<double>(), bltc ? 0 : 1, src,
+                           T.recnode.as<int32_t>(), T.d_info, bltc ? 0 : 1, src,
                            aoff);
         if (bltc) FSS_TRY((upward<float, D>(ctx, src)));
         if (ev) FSS_HIP(hipEventRecord(ev[4], s));
@@ -1253,7 +1253,7 @@ static fss_status run_degree(fss_ctx *ctx, const fss_particles *pp, fss_velocity
         {
             hipLaunchKernelGGL((k_proxy_list<float, D>), dim3((unsigned)div_up(T.n_proxy, 4)), dim3(256), 0, s,
                                T.proxy_items.as<ProxyItem>(), T.n_proxy, T.far_off.as<int64_t>(), T.far_src.as<int32_t>(), src,
-                               T.recnode.as<int32_t>(), (const float *)aoff, p0, T.tri_info.as<double>(),
+                               T.recnode.as<int32_t>(), (const float *)aoff, p0, T.d_info,
                                T.proxy_xyz.as<double4>(), ctx->phi.as<double>());
         }
         if (ev) FSS_HIP(hipEventRecord(ev[1], s));
@@ -1261,7 +1261,7 @@ static fss_status run_degree(fss_ctx *ctx, const fss_particles *pp, fss_velocity
             auto kn = ctx->near_r == 4 ? k_near<float, 4, false> : k_near<float, 2, false>; // default 2
             hipLaunchKernelGGL(kn, dim3((unsigned)T.n_near), dim3(64), 0, s, T.near_items.as<NearItem>(),
                                T.near_src.as<int32_t>(), src, T.recid.as<int32_t>(), T.recnode.as<int32_t>(), p0, p,
-                               T.tri_info.as<double>(), pp->x, pp->y, pp->z, ost, ctx->out3.as<double>());
+                               T.d_info, pp->x, pp->y, pp->z, ost, ctx->out3.as<double>());
         }
         if (ev) FSS_HIP(hipEventRecord(ev[2], s));
     }
@@ -1273,16 +1273,16 @@ static fss_status run_degree(fss_ctx *ctx, const fss_particles *pp, fss_velocity
         hipLaunchKernelGGL((k_combine<float, D>), dim3((unsigned)div_up(p0, 256)), dim3(256), 0, s,
                            T.recid.as<int32_t>(), T.recnode.as<int32_t>(), T.rinfo.as<uint8_t>(), T.nrange.as<int4>(),
                            T.oslot.as<int32_t>(), T.node_slot.as<int32_t>(), T.nodeof.as<int32_t>(),
-                           T.inv_active.as<int32_t>(), ctx->alpha.as<double>(), T.tinv.as<double>(),
-                           ctx->src32.as<float4>(), T.tri_info.as<double>(), T.inst.as<Instance>(), T.ninst, p0, ost,
+                           T.inv_active.as<int32_t>(), ctx->alpha.as<double>(), T.d_tinv,
+                           ctx->src32.as<float4>(), T.d_info, T.inst.as<Instance>(), T.ninst, p0, ost,
                            ctx->out3.as<double>(), bltc ? 1 : 0, scale, ctx->cfg.omega, out->u, out->v, out->w,
                            out->dvort);
     else
         hipLaunchKernelGGL((k_combine<double, D>), dim3((unsigned)div_up(p0, 256)), dim3(256), 0, s,
                            T.recid.as<int32_t>(), T.recnode.as<int32_t>(), T.rinfo.as<uint8_t>(), T.nrange.as<int4>(),
                            T.oslot.as<int32_t>(), T.node_slot.as<int32_t>(), T.nodeof.as<int32_t>(),
-                           T.inv_active.as<int32_t>(), ctx->alpha.as<double>(), T.tinv.as<double>(),
-                           ctx->src64.as<double4>(), T.tri_info.as<double>(), T.inst.as<Instance>(), T.ninst, p0, ost,
+                           T.inv_active.as<int32_t>(), ctx->alpha.as<double>(), T.d_tinv,
+                           ctx->src64.as<double4>(), T.d_info, T.inst.as<Instance>(), T.ninst, p0, ost,
                            ctx->out3.as<double>(), bltc ? 1 : 0, scale, ctx->cfg.omega, out->u, out->v, out->w,
                            out->dvort);
     if (ev) FSS_HIP(hipEventRecord(ev[3], s));

@@ -161,19 +161,19 @@ struct Tree {
     int64_t ntri_all = 0; // triangles on levels 0..L (geometry is built one level deeper)
     int64_t p0 = 0;       // particle records: n main + exception records
     int64_t nlist = 0;    // sum of the node list lengths (reference lists, export)
+    // triangles of levels 0..L and inverse vertex matrices: the context's Geo, or
+    // a batch's own arrays below
+    const double *d_xyz = nullptr, *d_info = nullptr, *d_tinv = nullptr;
     int64_t nslot_out = 0; // output slots of the near kernel (targets x levels with work)
     int64_t ninter = 0;
     int ngen = 0;
     std::vector<int64_t> level_base; // L+1 entries, host copy
     fss_tree_stats stats{};
 
-    DevBuf tri_xyz;  // 9 doubles per triangle (vertex coordinates, tree_tri_verts order)
-    DevBuf tri_info; // 4 doubles per triangle (centre, radius)
+    DevBuf tri_xyz, tri_info, tinv; // of a batch, all nodes of all instances (see Geo)
     DevBuf loc;      // int32 [L][n]
     DevBuf found;    // uint8 [L][n]
     DevBuf counts;   // int32 [nn]
-    DevBuf offsets;  // int32 [nn] global start in ids
-    DevBuf ids;      // int32 [nlist]: reference node lists (ascending ids per node)
     DevBuf inter;    // int32 [7][ninter] AoS
     DevBuf recid;    // int32 [p0]: particle of every record
     DevBuf recnode;  // int32 [p0]: node whose centre is the origin of the record (mixed precision)
@@ -181,6 +181,7 @@ struct Tree {
     DevBuf ipos;     // int32 [n]: main record of every particle
     DevBuf oslot;    // int32 [nn]: output slot of a node's first main target, or -1 (no near work)
     DevBuf nrange;   // int4 [nn]: {main start, main count, exception start, exception count}
+    // for memberships outside the main paths (only where there are any: p0 > n)
     DevBuf inv_active; // int32 [L][n]: output slot of a particle in a class-A node, or -1
     DevBuf nodeof;     // int32 [L][n]: global node of a particle per level, or -1 (dropped)
     DevBuf node_slot;  // int32 [nn]: interpolant slot of a node with class-B work, or -1
@@ -189,7 +190,7 @@ struct Tree {
     int64_t n_near = 0, n_proxy = 0, n_slot = 0, n_ra = 0, n_rb = 0, n_charge = 0;
     DevBuf near_items;  // NearItem[n_near]
     DevBuf near_src;    // int32 source record positions of every near item, item by item
-    int64_t n_near_src = 0;
+    int64_t n_near_src = 0, n_far_src = 0; // entries of near_src and far_src
     DevBuf proxy_items; // ProxyItem[n_proxy]
     DevBuf proxy_slots; // ProxySlot[n_slot]
     DevBuf far_off;     // int64 [n_proxy + 1]: source list of every proxy item in far_src
@@ -205,7 +206,6 @@ struct Tree {
     int64_t n_up = 0, n_up_multi = 0, n_up_partial = 0, n_up_small = 0; // items <= 32 records first
     DevBuf up_items;    // int4 [n_up] {node, first record, records, partial index or -1}
     DevBuf up_multi;    // int4 [n_up_multi] {node, first partial, end partial, 0}
-    DevBuf tinv;        // double [9 nn]: rows r_m with barycentric c_m = r_m . p
     DevBuf proxy_xyz;   // double4 [nn * p] static proxy positions (w unused)
     int64_t pairs_near = 0, pairs_far = 0;
 };
@@ -228,6 +228,27 @@ struct Sal {
     DevBuf mlpop; // the network in the form of its matrix-core evaluation (MlpOp, fss_sal_dev.h)
     bool has_mlp = false;
     int64_t adam_t = 0;
+};
+
+// Triangles of levels 0 .. levels-1 (levels concatenated): fixed by the depth, so
+// they are computed once per context for its deepest tree.
+struct Geo {
+    int levels = 0;
+    DevBuf xyz;  // 9 doubles per triangle (vertex coordinates, tree_tri_verts order)
+    DevBuf info; // 4 doubles per triangle (centre, radius)
+    DevBuf tinv; // 9 doubles: rows r_m with barycentric c_m = r_m . p
+    DevBuf aux;  // double2: norm of the centre, arc radius of the cap
+};
+
+// Scratch of tree_build, kept between builds while it is small (BUILD_SCRATCH_KEEP).
+struct BuildScratch {
+    DevBuf info, cub, ecnt, k0, k1, v0, v1, ek0, ek1, ev0, ev1, f0, f1, act, blk, types, begend, charge, per, pos, keys,
+        keys2, vals, vals2, rcnt, rpos, rkeys, prox_one, cnt, off;
+    std::vector<DevBuf *> all()
+    {
+        return {&info, &cub,    &ecnt, &k0,  &k1,  &v0,   &v1,    &ek0,  &ek1,   &ev0,  &ev1,  &f0,    &f1,       &act, &blk,
+                &types, &begend, &charge, &per, &pos, &keys, &keys2, &vals, &vals2, &rcnt, &rpos, &rkeys, &prox_one, &cnt, &off};
+    }
 };
 
 // Workspace of the remesh: missed targets, counters, and the triangle bins of
@@ -264,6 +285,8 @@ struct fss_ctx {
     fss::Timing timing;
     fss::Sal sal;
     fss::Remesh remesh;
+    fss::Geo geo;
+    fss::BuildScratch build;
 
     // device constants
     fss::DevBuf d_lu, d_perm, d_vinv, d_pts;
@@ -298,13 +321,13 @@ namespace fss {
 
 // ---- kernels / launchers (fss_tree.hip) ----
 fss_status tree_build(fss_ctx *ctx, const double *x, const double *y, const double *z, int64_t n);
-// derived per-node data shared by single and batched plans (inverse triangle
-// matrices, upward-pass items); called last by both builders
+// source lists, item order and upward-pass items of single and batched plans;
+// called last by both builders, and waits for the stream
 fss_status plan_finish(fss_ctx *ctx);
+void build_scratch_trim(BuildScratch &b);
 fss_status tree_export(fss_ctx *ctx, int32_t *loc, uint8_t *found, int32_t *counts,
                        int32_t *offsets, int32_t *ids, int32_t *inter, double *tri_info,
                        double *tri_xyz);
-void tree_release(Tree &t);
 
 // ---- interpolation constants (fss_api.cpp) ----
 fss_status interp_setup(fss_ctx *ctx);

@@ -431,7 +431,7 @@ template <int KIND, int D> fss_status run(fss_ctx *ctx, const KernelArgs &ka, do
     hipLaunchKernelGGL((k_sal_combine<D>), dim3((unsigned)div_up(p0, 256)), dim3(256), 0, s, T.recid.as<int32_t>(),
                        T.recnode.as<int32_t>(), T.rinfo.as<uint8_t>(), T.nrange.as<int4>(), T.oslot.as<int32_t>(),
                        T.node_slot.as<int32_t>(), T.nodeof.as<int32_t>(), T.inv_active.as<int32_t>(),
-                       ctx->alpha.as<double>(), T.tinv.as<double>(), src, T.inst.as<Instance>(), T.ninst, p0,
+                       ctx->alpha.as<double>(), T.d_tinv, src, T.inst.as<Instance>(), T.ninst, p0,
                        ctx->out3.as<double>(), ctx->acc3.as<double>());
     hipLaunchKernelGGL(k_sal_scatter, dim3((unsigned)div_up(T.n, 256)), dim3(256), 0, s, T.ipos.as<int32_t>(), T.n,
                        ctx->acc3.as<double>(), result);
