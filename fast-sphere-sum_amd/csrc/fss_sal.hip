@@ -44,16 +44,21 @@ __global__ void k_series_table(const double *__restrict__ c, int N, int64_t M, d
 {
     int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
     if (i >= M) return;
-    const int64_t m1 = M / 2;
+    const int64_t m1 = M / 2, m2 = M - m1;
     double t;
     if (i < m1) {
         const double si = SAL_TAB_SPAN * (double)i / (double)(m1 - 1);
         t = 1.0 - 2.0 * si * si;
     } else {
-        const double ui = SAL_TAB_SPAN * (double)(i - m1) / (double)(M - m1 - 1);
+        const double ui = SAL_TAB_SPAN * (double)(i - m1) / (double)(m2 - 1);
         t = 2.0 * ui * ui - 1.0;
     }
-    tab[i] = legendre_sum(c, N, t);
+    // with the padding of SalTab
+    const double g = legendre_sum(c, N, t);
+    const int64_t at = i < m1 ? i + 1 : i + 3;
+    tab[at] = g;
+    if (i == 0 || i == m1) tab[at - 1] = g;
+    if (i == m1 - 1 || i == M - 1) tab[at + 1] = g;
 }
 
 // ------------------------------------------------------------------
@@ -379,8 +384,7 @@ __global__ void __launch_bounds__(STILE) k_sal_direct_table(const double *__rest
                                                              const double *__restrict__ z,
                                                              const double *__restrict__ w, int64_t n,
                                                              const int64_t *__restrict__ idx, int64_t m,
-                                                             const double *__restrict__ tab, int64_t M,
-                                                             double g0, double *out)
+                                                             SalTab tab, double g0, double *out)
 {
     __shared__ double4 tile[STILE];
     int64_t r = (int64_t)blockIdx.x * STILE + threadIdx.x;
@@ -396,9 +400,9 @@ __global__ void __launch_bounds__(STILE) k_sal_direct_table(const double *__rest
         for (int k = 0; k < cnt; k++) {
             double4 sj = tile[k];
             double dx = sj.x - xi, dy = sj.y - yi, dz = sj.z - zi;
-            double s = 0.5 * sqrt(dx * dx + dy * dy + dz * dz);
+            double q = dx * dx + dy * dy + dz * dz;
             // self term: the truncated series at theta = 0
-            double gk = base + k == i ? g0 : table_eval(tab, M, s);
+            double gk = base + k == i ? g0 : table_eval_dist2(tab, q);
             acc = fma(gk, sj.w, acc);
         }
     }
@@ -462,7 +466,7 @@ fss_status sal_set_series(fss_ctx *ctx, const double *c_host, int nmax, int64_t 
     S.M = table_points;
     FSS_TRY(S.c.ensure(sizeof(double) * (nmax + 1)));
     FSS_HIP(hipMemcpyAsync(S.c.p, c_host, sizeof(double) * (nmax + 1), hipMemcpyHostToDevice, s));
-    FSS_TRY(S.tab.ensure(sizeof(double) * table_points));
+    FSS_TRY(S.tab.ensure(sizeof(double) * (table_points + 4)));
     hipLaunchKernelGGL(k_series_table, dim3((unsigned)div_up(table_points, 256)), dim3(256), 0, s,
                        S.c.as<double>(), nmax, table_points, S.tab.as<double>());
     double g0 = 0;
@@ -623,11 +627,10 @@ fss_status sal_mlp_grad(fss_ctx *ctx, const float *x_host, const float *y_host, 
     return FSS_OK;
 }
 
-__global__ void k_table(const double *__restrict__ tab, int64_t M, const double *__restrict__ s, int64_t m,
-                        double *g)
+__global__ void k_table(SalTab tab, const double *__restrict__ s, int64_t m, double *g)
 {
     int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (i < m) g[i] = table_eval(tab, M, s[i]);
+    if (i < m) g[i] = table_eval(tab, s[i]);
 }
 
 fss_status sal_kernel_eval(fss_ctx *ctx, int kind, const double *s_dev, int64_t m, double *g_dev)
@@ -637,7 +640,7 @@ fss_status sal_kernel_eval(fss_ctx *ctx, int kind, const double *s_dev, int64_t 
     if (kind == 0) return sal_series_eval(ctx, s_dev, m, g_dev);
     if (kind == 2) {
         if (!S.c.p) return set_error("sal: series not set"), FSS_ERR_STATE;
-        hipLaunchKernelGGL(k_table, dim3((unsigned)div_up(m, 256)), dim3(256), 0, s, S.tab.as<double>(), S.M, s_dev,
+        hipLaunchKernelGGL(k_table, dim3((unsigned)div_up(m, 256)), dim3(256), 0, s, sal_tab(S.tab.as<double>(), S.M), s_dev,
                            m, g_dev);
         FSS_HIP(hipGetLastError());
         return FSS_OK;
@@ -671,7 +674,7 @@ fss_status sal_direct(fss_ctx *ctx, const double *x, const double *y, const doub
     float lmin = (float)std::log(S.s_min), ispan = (float)(1.0 / -std::log(S.s_min));
     if (kind == 0)
         hipLaunchKernelGGL(k_sal_direct_table, dim3(g), dim3(STILE), 0, s, x, y, z, S.w.as<double>(), n, idx, m,
-                           S.tab.as<double>(), S.M, S.g0, out);
+                           sal_tab(S.tab.as<double>(), S.M), S.g0, out);
     else
         hipLaunchKernelGGL(k_sal_direct_mlp, dim3(g), dim3(STILE), 0, s, x, y, z, S.w.as<double>(), n, idx, m,
                            S.mlpop.as<MlpOp>(), S.A, S.mu, S.sigma, S.g0, lmin, ispan, out);

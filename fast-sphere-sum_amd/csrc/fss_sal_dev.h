@@ -43,28 +43,67 @@ __device__ inline double legendre_sum(const double *__restrict__ c, int N, doubl
 constexpr double SAL_TAB_SPAN = 0.75;
 constexpr double SAL_TAB_SWITCH = 0.70710678118654752; // sqrt(1/2)
 
-// cubic (Catmull-Rom) interpolation of n samples of [0, SAL_TAB_SPAN] at x
-__device__ inline double catmull_rom(const double *__restrict__ tab, int64_t n, double x)
+// In memory each half is padded by a copy of its first and last sample, so that
+// the four samples around any cell are consecutive.
+struct SalTab {
+    const double *tab; // half 1 padded (n1 + 2 entries), then half 2 padded (n2 + 2)
+    int64_t n1, n2;
+    double inv1, inv2; // cells per unit of s, of u
+    bool wide;         // a half has more than 2^32 cells
+};
+inline SalTab sal_tab(const double *tab, int64_t M)
 {
-    double v = x * ((double)(n - 1) / SAL_TAB_SPAN);
-    int64_t k = (int64_t)v;
-    if (k > n - 2) k = n - 2;
-    if (k < 0) k = 0;
-    double f = v - (double)k;
-    double p0 = tab[k > 0 ? k - 1 : 0], p1 = tab[k], p2 = tab[k + 1], p3 = tab[k + 2 < n ? k + 2 : n - 1];
-    double a = -0.5 * p0 + 1.5 * p1 - 1.5 * p2 + 0.5 * p3;
-    double b = p0 - 2.5 * p1 + 2.0 * p2 - 0.5 * p3;
-    double cc = -0.5 * p0 + 0.5 * p2;
-    return ((a * f + b) * f + cc) * f + p1;
+    SalTab t{tab, M / 2, M - M / 2, 0, 0, M > ((int64_t)1 << 33)};
+    t.inv1 = (double)(t.n1 - 1) / SAL_TAB_SPAN;
+    t.inv2 = (double)(t.n2 - 1) / SAL_TAB_SPAN;
+    return t;
 }
 
-// G at s in [0, 1] from the two-part table of M entries
-__device__ inline double table_eval(const double *__restrict__ tab, int64_t M, double s)
+// G at s (u = 0) or u = cos(theta/2): cubic (Catmull-Rom) interpolation at x.
+// A lane reads its four samples as two 16-byte loads: the lanes of a wave read
+// unrelated cells, and each of their loads is a lookup of its own in the L1
+// (as four 8-byte loads the near pairs of a level-8 grid took 3.31 ms, now 2.76,
+// the proxy values 2.00, now 1.49).
+__device__ inline double table_at(const SalTab &t, double x, bool u)
 {
-    const int64_t m1 = M / 2;
-    if (s <= SAL_TAB_SWITCH) return catmull_rom(tab, m1, s);
-    const double u = sqrt(fmax(0.0, (1.0 - s) * (1.0 + s)));
-    return catmull_rom(tab + m1, M - m1, u);
+    typedef double pair8 __attribute__((ext_vector_type(2), aligned(8)));
+    const double v = x * (u ? t.inv2 : t.inv1);
+    const double k = fmin(floor(v), (double)((u ? t.n2 : t.n1) - 2)), f = v - k;
+    const pair8 *q = reinterpret_cast<const pair8 *>(t.tab + (u ? t.n1 + 2 : 0) + (t.wide ? (int64_t)k : (int64_t)(uint32_t)k));
+    const pair8 a = q[0], b = q[1];
+    // the cubic with slopes (p2 - p0) / 2 and (p3 - p1) / 2
+    const double e1 = b.x - a.x, e2 = b.y - a.y, d = a.y - b.x;
+    const double c3 = fma(0.5, e1 + e2, d + d), c2 = fma(-3.0, d, fma(-0.5, e2, -e1));
+    return fma(fma(fma(c3, f, c2), f, 0.5 * e1), f, a.y);
+}
+
+// square root of q >= 0 from v_rsq_f64 (relative error below 1e-7) and two
+// Newton steps: within an ulp or two, without the scaling that the library's needs
+// for the smallest and largest numbers (q in [0, 4] here; 0 gives 1e-100)
+__device__ inline double sqrt_plain(double q)
+{
+    q = fmax(q, 1e-200);
+    const double r = __builtin_amdgcn_rsq(q);
+    double g = q * r, h = 0.5 * r;
+    const double e = fma(-h, g, 0.5);
+    g = fma(g, e, g);
+    h = fma(h, e, h);
+    return fma(fma(-g, g, q), h, g);
+}
+
+// G at s in [0, 1]
+__device__ inline double table_eval(const SalTab &t, double s)
+{
+    const bool u = s > SAL_TAB_SWITCH;
+    return table_at(t, u ? sqrt(fmax(0.0, (1.0 - s) * (1.0 + s))) : s, u);
+}
+
+// G at s = sqrt(q) / 2 from the squared distance: s^2 = q / 4, u^2 = 1 - q / 4, one
+// square root for either half of the table
+__device__ inline double table_eval_dist2(const SalTab &t, double q)
+{
+    const bool u = q > 2.0;
+    return table_at(t, sqrt_plain(u ? fma(-0.25, q, 1.0) : 0.25 * q), u);
 }
 
 // ------------------------------------------------------------------

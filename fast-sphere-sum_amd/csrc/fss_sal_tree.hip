@@ -20,13 +20,12 @@ namespace fss {
 
 namespace {
 
-constexpr int NCH_S = 256;
+constexpr int NCH_S = 128; // 4.6 KiB a one-wave block: eight waves per SIMD
 
 template <int D> constexpr int npts_s() { return (D + 1) * (D + 2) / 2; }
 
 struct KernelArgs {
-    const double *tab;
-    int64_t M;
+    SalTab tab;
     const float *P;
     const MlpOp *mlp;   // the network's parameters in the form of the matrix-core evaluation
     double A, mu, sigma, g0;
@@ -35,19 +34,23 @@ struct KernelArgs {
     int N;
 };
 
-// the series kernels (KIND 0: table, 2: Clenshaw); the learned kernel has
-// its own matrix-core kernels below
-template <int KIND> __device__ inline double gfun(const KernelArgs &k, double s)
-{
-    static_assert(KIND == 0 || KIND == 2, "series kernels only");
-    if (KIND == 0) return table_eval(k.tab, k.M, s);
-    return legendre_sum(k.c, k.N, 1.0 - 2.0 * s * s);
-}
-
-__device__ inline double half_dist(const double4 &a, const double4 &b)
+__device__ inline double dist2(const double4 &a, const double4 &b)
 {
     double dx = a.x - b.x, dy = a.y - b.y, dz = a.z - b.z;
-    return 0.5 * sqrt(dx * dx + dy * dy + dz * dz);
+    return dx * dx + dy * dy + dz * dz;
+}
+
+__device__ inline double half_dist(const double4 &a, const double4 &b) { return 0.5 * sqrt(dist2(a, b)); }
+
+// the series kernels (KIND 0: table, 2: Clenshaw); the learned kernel has
+// its own matrix-core kernels below
+template <int KIND> __device__ inline double gfun(const KernelArgs &k, const double4 &a, const double4 &b)
+{
+    static_assert(KIND == 0 || KIND == 2, "series kernels only");
+    const double q = dist2(a, b);
+    if (KIND == 0) return table_eval_dist2(k.tab, q);
+    const double s = 0.5 * sqrt(q);
+    return legendre_sum(k.c, k.N, 1.0 - 2.0 * s * s);
 }
 
 // near field: one wave per near item, one lane per (target, phase); the
@@ -79,7 +82,7 @@ __global__ void __launch_bounds__(64) k_sal_near(const NearItem *__restrict__ it
         if (act)
             for (int k = ph; k < m; k += P) {
                 const double4 s = lds[k];
-                acc = fma(gfun<KIND>(ka, half_dist(xt, s)), s.w, acc);
+                acc = fma(gfun<KIND>(ka, xt, s), s.w, acc);
             }
         __syncthreads();
     }
@@ -124,7 +127,7 @@ __global__ void __launch_bounds__(64) k_sal_proxy(const ProxyItem *__restrict__ 
         if (act)
             for (int kk = ph; kk < m; kk += P) {
                 const double4 s = lds[kk];
-                acc = fma(gfun<KIND>(ka, half_dist(yk, s)), s.w, acc);
+                acc = fma(gfun<KIND>(ka, yk, s), s.w, acc);
             }
         __syncthreads();
     }
@@ -465,8 +468,7 @@ fss_status sal_tree(fss_ctx *ctx, const fss_particles *pp, int kind, double *out
     if (kind < 0 || kind > 2) return set_error("sal: kind 0 (table), 1 (learned) or 2 (series)"), FSS_ERR_INVALID;
     if (kind == 1) FSS_TRY(sal_mlp_prepare(ctx));
     KernelArgs ka;
-    ka.tab = S.tab.as<double>();
-    ka.M = S.M;
+    ka.tab = sal_tab(S.tab.as<double>(), S.M);
     ka.P = S.P.as<float>();
     ka.mlp = S.mlpop.as<MlpOp>();
     ka.A = S.A;
