@@ -2,6 +2,7 @@
 // interpolation constants and argument checking.  No exception crosses the ABI.
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
 #include <atomic>
 #include <cfloat>
 #include <cmath>
@@ -9,6 +10,7 @@
 #include <exception>
 #include <new>
 #include <string>
+#include <vector>
 
 #include "fss_internal.h"
 
@@ -256,6 +258,48 @@ fss_status interp_setup(fss_ctx *ctx)
     return FSS_OK;
 }
 
+static fss_status timing_setup(fss_ctx *ctx)
+{
+    Timing &t = ctx->timing;
+    int khz = 0;
+    FSS_HIP(hipDeviceGetAttribute(&khz, hipDeviceAttributeWallClockRate, ctx->cfg.device));
+    if (khz <= 0) return set_error("no device clock rate"), FSS_ERR_HIP;
+    t.ms_per_tick = 1.0 / khz;
+    const size_t bytes = sizeof(uint64_t) * Timing::RING * Timing::SLOT;
+    FSS_TRY(t.stamps.ensure(bytes));
+    FSS_HIP(hipMemsetAsync(t.stamps.p, 0, bytes, ctx->stream));
+    return FSS_OK;
+}
+
+fss_status timing_read(fss_ctx *ctx, int64_t first, int64_t count, double *stage, double *main, double *far)
+{
+    Timing &t = ctx->timing;
+    std::vector<uint64_t> h((size_t)count * Timing::SLOT);
+    if (t.stream != ctx->stream) FSS_HIP(hipDeviceSynchronize()); // the calls ran on another stream
+    FSS_HIP(hipMemcpyAsync(h.data(), t.stamps.as<uint64_t>() + first * Timing::SLOT, sizeof(uint64_t) * h.size(),
+                           hipMemcpyDeviceToHost, ctx->stream));
+    FSS_HIP(hipStreamSynchronize(ctx->stream));
+    double sum[3] = {0, 0, 0};
+    for (int64_t i = 0; i < count; i++) {
+        const uint64_t *v = h.data() + i * Timing::SLOT;
+        const int have = t.have[first + i];
+        const uint64_t end = *std::max_element(v + Timing::END, v + Timing::SLOT);
+        auto ticks = [](uint64_t a, uint64_t b) { return b > a ? (double)(b - a) : 0.0; };
+        sum[0] += ticks(v[Timing::START], end);
+        if (have & (1 << Timing::MAIN)) {
+            sum[1] += ticks(v[Timing::MAIN], have & (1 << Timing::MAIN_END) ? v[Timing::MAIN_END] : end);
+            if (have & (1 << Timing::FAR)) sum[2] += ticks(v[Timing::FAR], v[Timing::MAIN]);
+        } else if (have & (1 << Timing::FAR)) {
+            sum[2] += ticks(v[Timing::FAR], have & (1 << Timing::MAIN_END) ? v[Timing::MAIN_END] : end);
+        }
+    }
+    const double f = t.ms_per_tick / (double)count;
+    if (stage) *stage = sum[0] * f;
+    if (main) *main = sum[1] * f;
+    if (far) *far = sum[2] * f;
+    return FSS_OK;
+}
+
 static fss_status validate(const fss_config *c)
 {
     if (!(c->theta > 0) || !std::isfinite(c->theta)) return set_error("theta must be > 0"), FSS_ERR_INVALID;
@@ -358,13 +402,8 @@ fss_status fss_create(fss_ctx **out, const fss_config *cfg)
             return set_error("hipStreamCreate failed"), FSS_ERR_HIP;
         }
         c->own_stream = true;
-        for (auto &row : c->timing.ev)
-            for (auto &e : row)
-                if (hipEventCreate(&e) != hipSuccess) {
-                    fss_destroy(c);
-                    return set_error("hipEventCreate failed"), FSS_ERR_HIP;
-                }
-        fss_status s = interp_setup(c);
+        fss_status s = timing_setup(c);
+        if (s == FSS_OK) s = interp_setup(c);
         if (s != FSS_OK) {
             fss_destroy(c);
             return s;
@@ -381,9 +420,6 @@ fss_status fss_destroy(fss_ctx *ctx)
     if (ctx->stream) (void)hipStreamSynchronize(ctx->stream);
     if (ctx->graph_exec) (void)hipGraphExecDestroy(ctx->graph_exec);
     if (ctx->graph) (void)hipGraphDestroy(ctx->graph);
-    for (auto &row : ctx->timing.ev)
-        for (auto &e : row)
-            if (e) (void)hipEventDestroy(e);
     if (ctx->own_stream && ctx->stream) (void)hipStreamDestroy(ctx->stream);
     delete ctx; // DevBuf members free their device memory
     return FSS_OK;
@@ -591,14 +627,7 @@ fss_status fss_last_timing(fss_ctx *ctx, double *stage_ms, double *main_ms)
 {
     if (!ctx) return set_error("null context"), FSS_ERR_INVALID;
     if (!ctx->timing.valid || ctx->timing.cur < 0) return set_error("no timed call yet"), FSS_ERR_STATE;
-    hipEvent_t *ev = ctx->timing.slot();
-    FSS_HIP(hipEventSynchronize(ev[3]));
-    float a = 0, b = 0;
-    FSS_HIP(hipEventElapsedTime(&a, ev[0], ev[3]));
-    FSS_HIP(hipEventElapsedTime(&b, ev[1], ev[2]));
-    if (stage_ms) *stage_ms = a;
-    if (main_ms) *main_ms = b;
-    return FSS_OK;
+    return timing_read(ctx, ctx->timing.cur, 1, stage_ms, main_ms, nullptr);
 }
 
 fss_status fss_sal_set_series(fss_ctx *ctx, const double *c, int nmax, int64_t table_points, double A)
@@ -701,20 +730,8 @@ fss_status fss_timing_mean(fss_ctx *ctx, int64_t *calls, double *stage_ms, doubl
     if (!t.valid || t.calls < 1) return set_error("no timed call yet"), FSS_ERR_STATE;
     if (t.calls > Timing::RING)
         return set_error("more timed calls than event slots; reset more often"), FSS_ERR_STATE;
-    double sa = 0, sb = 0;
-    for (int64_t i = 0; i < t.calls; i++) {
-        hipEvent_t *ev = t.ev[i];
-        FSS_HIP(hipEventSynchronize(ev[3]));
-        float a = 0, b = 0;
-        FSS_HIP(hipEventElapsedTime(&a, ev[0], ev[3]));
-        FSS_HIP(hipEventElapsedTime(&b, ev[1], ev[2]));
-        sa += a;
-        sb += b;
-    }
     if (calls) *calls = t.calls;
-    if (stage_ms) *stage_ms = sa / t.calls;
-    if (main_ms) *main_ms = sb / t.calls;
-    return FSS_OK;
+    return timing_read(ctx, 0, t.calls, stage_ms, main_ms, nullptr);
 }
 
 fss_status fss_timing_far_mean(fss_ctx *ctx, double *far_ms)
@@ -724,16 +741,7 @@ fss_status fss_timing_far_mean(fss_ctx *ctx, double *far_ms)
     if (!t.valid || t.calls < 1) return set_error("no timed call yet"), FSS_ERR_STATE;
     if (t.calls > Timing::RING)
         return set_error("more timed calls than event slots; reset more often"), FSS_ERR_STATE;
-    double sf = 0;
-    for (int64_t i = 0; i < t.calls; i++) {
-        hipEvent_t *ev = t.ev[i];
-        FSS_HIP(hipEventSynchronize(ev[3]));
-        float f = 0;
-        FSS_HIP(hipEventElapsedTime(&f, ev[4], ev[1]));
-        sf += f;
-    }
-    *far_ms = sf / t.calls;
-    return FSS_OK;
+    return timing_read(ctx, 0, t.calls, nullptr, nullptr, far_ms);
 }
 
 } // extern "C"

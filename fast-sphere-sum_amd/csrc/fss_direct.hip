@@ -48,16 +48,18 @@ __device__ inline double rcp64d(double d)
 
 __global__ void k_pack64(const double *__restrict__ x, const double *__restrict__ y,
                          const double *__restrict__ z, const double *__restrict__ vort,
-                         const double *__restrict__ area, int64_t n, double4 *src)
+                         const double *__restrict__ area, int64_t n, double4 *src, uint64_t *ts)
 {
+    stamp_start(ts, Timing::START);
     int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
     if (i < n) src[i] = make_double4(x[i], y[i], z[i], vort[i] * area[i]);
 }
 
 __global__ void k_pack32(const double *__restrict__ x, const double *__restrict__ y,
                          const double *__restrict__ z, const double *__restrict__ vort,
-                         const double *__restrict__ area, int64_t n, float4 *src)
+                         const double *__restrict__ area, int64_t n, float4 *src, uint64_t *ts)
 {
+    stamp_start(ts, Timing::START);
     int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
     if (i < n) src[i] = make_float4((float)x[i], (float)y[i], (float)z[i], 2.0f * (float)(vort[i] * area[i]));
 }
@@ -85,6 +87,7 @@ struct DirectArgs {
     double scale, omega;
     double *part;
     double *u, *v, *w, *dvort;
+    uint64_t *ts; // time stamps, or null
 };
 
 __device__ inline void direct_source(const DirectArgs &a, int64_t j, double4 &s)
@@ -206,6 +209,8 @@ __global__ void __launch_bounds__(256, 4) k_direct(DirectArgs a)
     T4 *tile = reinterpret_cast<T4 *>(smem) + wave * WT;
     double *red = reinterpret_cast<double *>(smem); // [4][NT], after a segment's last tile
     const T4 *rec = static_cast<const T4 *>(a.rec);
+    if (SPLIT) stamp_start(a.ts, Timing::START);
+    stamp_start(a.ts, Timing::MAIN);
     const int64_t b = blockIdx.x;
     int64_t u = direct_first(b, a.B1, a.q1, a.q);
     const int64_t u1 = min(u + (b < a.B1 ? a.q1 : a.q), a.U);
@@ -299,6 +304,7 @@ __global__ void __launch_bounds__(256, 4) k_direct(DirectArgs a)
         }
         u += t1 - t0;
     }
+    if (!SPLIT) stamp_end(a.ts);
 }
 
 // sums the partials of every target over the blocks of its group: 16 targets x
@@ -306,7 +312,7 @@ __global__ void __launch_bounds__(256, 4) k_direct(DirectArgs a)
 // one thread per target would walk them alone), ways added in order
 __global__ void __launch_bounds__(256) k_direct_sum(const double *__restrict__ part, int64_t m, int nt, int64_t K,
                                                     int64_t B1, int64_t q1, int64_t q, double omega, double *u, double *v, double *w,
-                                                    double *dvort)
+                                                    double *dvort, uint64_t *ts)
 {
     __shared__ double red[3][16][17];
     const int tl = threadIdx.x & 15, way = threadIdx.x >> 4;
@@ -334,6 +340,7 @@ __global__ void __launch_bounds__(256) k_direct_sum(const double *__restrict__ p
         w[r] = red[2][0][tl];
         dvort[r] = -2 * omega * red[2][0][tl];
     }
+    stamp_end(ts);
 }
 
 struct DirectPlan {
@@ -406,27 +413,23 @@ static DirectPlan direct_plan(int64_t n, int64_t m, bool mixed)
     return p;
 }
 
-// buf: at least direct_plan().bytes; ev: the call's timing events or null
+// buf: at least direct_plan().bytes; ts: the call's time stamps or null
 static fss_status launch_direct(fss_ctx *ctx, const fss_particles *p, const int64_t *idx, int64_t m,
-                                fss_velocity *out, bool mixed, void *buf, hipEvent_t *ev)
+                                fss_velocity *out, bool mixed, void *buf, uint64_t *ts)
 {
     hipStream_t s = ctx->stream;
     const DirectPlan P = direct_plan(p->n, m, mixed);
     DirectArgs a{p->x, p->y, p->z, p->vort, p->area, nullptr, idx, p->n, m, P.K, P.U, P.B1, P.q1, P.q, -1.0 / (4.0 * M_PI),
-                 ctx->cfg.omega, static_cast<double *>(buf), out->u, out->v, out->w, out->dvort};
+                 ctx->cfg.omega, static_cast<double *>(buf), out->u, out->v, out->w, out->dvort, ts};
     if (!P.split) {
         const dim3 gp((unsigned)div_up(p->n, 256));
         a.rec = buf;
         if (mixed)
             hipLaunchKernelGGL(k_pack32, gp, dim3(256), 0, s, p->x, p->y, p->z, p->vort, p->area, p->n,
-                               static_cast<float4 *>(buf));
+                               static_cast<float4 *>(buf), ts);
         else
             hipLaunchKernelGGL(k_pack64, gp, dim3(256), 0, s, p->x, p->y, p->z, p->vort, p->area, p->n,
-                               static_cast<double4 *>(buf));
-    }
-    if (ev) {
-        FSS_HIP(hipEventRecord(ev[4], s));
-        FSS_HIP(hipEventRecord(ev[1], s));
+                               static_cast<double4 *>(buf), ts);
     }
     void (*k)(DirectArgs);
     if (mixed)
@@ -440,7 +443,7 @@ static fss_status launch_direct(fss_ctx *ctx, const fss_particles *p, const int6
     hipLaunchKernelGGL(k, dim3((unsigned)P.B), dim3(256), 0, s, a);
     if (P.split)
         hipLaunchKernelGGL(k_direct_sum, dim3((unsigned)div_up(m, 16)), dim3(256), 0, s, a.part, m, 64 * P.R, P.K, P.B1, P.q1,
-                           P.q, a.omega, out->u, out->v, out->w, out->dvort);
+                           P.q, a.omega, out->u, out->v, out->w, out->dvort, ts);
     FSS_HIP(hipGetLastError());
     return FSS_OK;
 }
@@ -448,7 +451,6 @@ static fss_status launch_direct(fss_ctx *ctx, const fss_particles *p, const int6
 fss_status velocity_direct(fss_ctx *ctx, const fss_particles *p, const int64_t *idx, int64_t m,
                            fss_velocity *out, bool force_fp64)
 {
-    hipStream_t s = ctx->stream;
     const int64_t n = p->n;
     if (n < 1) {
         set_error("velocity_direct: n < 1");
@@ -457,16 +459,13 @@ fss_status velocity_direct(fss_ctx *ctx, const fss_particles *p, const int64_t *
     if (!idx) m = n;
     const bool mixed = !force_fp64 && ctx->cfg.precision == FSS_MIXED;
     DevBuf &buf = mixed ? ctx->src32 : ctx->src64;
-    if (!ctx->capturing) timing_begin(ctx->timing);
-    hipEvent_t *ev = ctx->capturing ? nullptr : ctx->timing.slot();
-    if (ev) FSS_HIP(hipEventRecord(ev[0], s));
     FSS_TRY(buf.ensure(direct_plan(n, m, mixed).bytes));
-    FSS_TRY(launch_direct(ctx, p, idx, m, out, mixed, buf.p, ev));
-    if (ev) {
-        FSS_HIP(hipEventRecord(ev[2], s));
-        FSS_HIP(hipEventRecord(ev[3], s));
-        ctx->timing.valid = true;
-    }
+    if (ctx->capturing) return launch_direct(ctx, p, idx, m, out, mixed, buf.p, nullptr);
+    Timing &t = ctx->timing;
+    timing_begin(t, ctx->stream);
+    t.have[t.cur] = 1 << Timing::MAIN;
+    FSS_TRY(launch_direct(ctx, p, idx, m, out, mixed, buf.p, t.slot()));
+    t.valid = true;
     return FSS_OK;
 }
 

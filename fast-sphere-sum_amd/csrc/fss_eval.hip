@@ -151,8 +151,9 @@ __global__ void k_gather64(const double *__restrict__ x, const double *__restric
                            const double *__restrict__ z, const double *__restrict__ vort,
                            const double *__restrict__ area, const int32_t *__restrict__ recid,
                            int64_t p0, const double4 *__restrict__ proxy, int64_t nprox,
-                           double4 *src)
+                           double4 *src, uint64_t *ts)
 {
+    stamp_start(ts, Timing::START);
     int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
     if (i < p0) {
         int32_t id = recid[i];
@@ -168,8 +169,9 @@ __global__ void k_gather32(const double *__restrict__ x, const double *__restric
                            const double *__restrict__ area, const int32_t *__restrict__ recid,
                            int64_t p0, const double4 *__restrict__ proxy, int64_t nprox, int p,
                            const int32_t *__restrict__ recnode, const double *__restrict__ centres,
-                           int planar, float4 *src, float *aoff)
+                           int planar, float4 *src, float *aoff, uint64_t *ts)
 {
+    stamp_start(ts, Timing::START);
     // FP32 records hold the offset from the centre of the record's node
     // (FP64 subtraction, then rounding): differences of nearby points keep
     // ~1e-9 absolute accuracy instead of the 6e-8 of rounded coordinates.
@@ -632,8 +634,10 @@ __global__ void __launch_bounds__(64, sizeof(Real) == 4 && R == 2 ? 8 : 4) k_nea
                                              const double *__restrict__ centres,
                                              const double *__restrict__ x,
                                              const double *__restrict__ y,
-                                             const double *__restrict__ z, int64_t ostride, double *out)
+                                             const double *__restrict__ z, int64_t ostride, double *out,
+                                             uint64_t *ts)
 {
+    stamp_start(ts, Timing::MAIN);
     using T4 = typename Rec<Real>::T4;
     // staged records and their particle ids, or after the last chunk the
     // phase partials [64][3R] and sums [T][3R] (T <= 64 / R + 1); one buffer
@@ -862,8 +866,10 @@ __global__ void __launch_bounds__(256) k_proxy_list(const ProxyItem *__restrict_
                                                    const int32_t *__restrict__ recnode,
                                                    const float *__restrict__ aoff, int64_t p0,
                                                    const double *__restrict__ centres,
-                                                   const double4 *__restrict__ proxy_xyz, double *phi)
+                                                   const double4 *__restrict__ proxy_xyz, double *phi,
+                                                   uint64_t *ts)
 {
+    stamp_start(ts, Timing::FAR);
     using T4 = typename Rec<Real>::T4;
     constexpr int PP = npts<D>();
     // proxies per lane: FP64 3 up to degree 2, 2 beyond (registers); FP32 the
@@ -977,8 +983,9 @@ __global__ void __launch_bounds__(256) k_proxy_list(const ProxyItem *__restrict_
 template <int D>
 __global__ void __launch_bounds__(128) k_solve(const ProxySlot *__restrict__ slots, int64_t nslot,
                         const double *__restrict__ phi, const double *__restrict__ lu,
-                        const int32_t *__restrict__ perm, double *alpha)
+                        const int32_t *__restrict__ perm, double *alpha, uint64_t *ts)
 {
+    stamp_start(ts, Timing::MAIN_END);
     constexpr int P = npts<D>();
     int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
     if (i >= 3 * nslot) return;
@@ -1081,8 +1088,9 @@ __global__ void k_combine(const int32_t *__restrict__ recid, const int32_t *__re
                           const typename Rec<Real>::T4 *__restrict__ src, const double *__restrict__ centres,
                           const Instance *__restrict__ inst, int ninst, int64_t nrec, int64_t ostride,
                           const double *__restrict__ out, int normalise, double scale, double omega,
-                          double *u, double *v, double *w, double *dvort)
+                          double *u, double *v, double *w, double *dvort, uint64_t *ts_first, uint64_t *ts)
 {
+    stamp_start(ts_first, Timing::MAIN_END);
     int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
     if (i >= nrec) return;
     // instance of record i: last k with rbase <= i
@@ -1166,6 +1174,7 @@ __global__ void k_combine(const int32_t *__restrict__ recid, const int32_t *__re
     v[id] = a1 * scale;
     w[id] = s2;
     dvort[id] = -2 * omega * s2;
+    stamp_end(ts);
 }
 
 // ------------------------------------------------------------------
@@ -1200,7 +1209,7 @@ static fss_status upward(fss_ctx *ctx, typename Rec<Real>::T4 *src)
 }
 
 template <int D>
-static fss_status run_degree(fss_ctx *ctx, const fss_particles *pp, fss_velocity *out, hipEvent_t *ev)
+static fss_status run_degree(fss_ctx *ctx, const fss_particles *pp, fss_velocity *out, uint64_t *ts)
 {
     Tree &T = ctx->tree;
     hipStream_t s = ctx->stream;
@@ -1213,62 +1222,56 @@ static fss_status run_degree(fss_ctx *ctx, const fss_particles *pp, fss_velocity
     FSS_TRY(ctx->out3.ensure(sizeof(double) * 3 * ost));
     FSS_TRY(ctx->phi.ensure(sizeof(double) * 3 * p * std::max<int64_t>(1, T.n_proxy)));
     FSS_TRY(ctx->alpha.ensure(sizeof(double) * 3 * p * std::max<int64_t>(1, T.n_slot)));
-    if (ev) FSS_HIP(hipEventRecord(ev[0], s));
     unsigned gs = (unsigned)div_up(nsrc, 256);
     if (!mixed) {
         FSS_TRY(ctx->src64.ensure(sizeof(double4) * nsrc));
         double4 *src = ctx->src64.as<double4>();
         hipLaunchKernelGGL(k_gather64, dim3(gs), dim3(256), 0, s, pp->x, pp->y, pp->z, pp->vort,
-                           pp->area, T.recid.as<int32_t>(), p0, T.proxy_xyz.as<double4>(), nprox, src);
+                           pp->area, T.recid.as<int32_t>(), p0, T.proxy_xyz.as<double4>(), nprox, src, ts);
         if (bltc) FSS_TRY((upward<double, D>(ctx, src)));
-        if (ev) FSS_HIP(hipEventRecord(ev[4], s));
-        if (T.n_proxy > 0)
+            if (T.n_proxy > 0)
         {
             hipLaunchKernelGGL((k_proxy_list<double, D>), dim3((unsigned)div_up(T.n_proxy, 4)), dim3(256), 0, s,
                                T.proxy_items.as<ProxyItem>(), T.n_proxy, T.far_off.as<int64_t>(), T.far_src.as<int32_t>(), src,
                                T.recnode.as<int32_t>(), (const float *)nullptr, p0, T.d_info,
-                               T.proxy_xyz.as<double4>(), ctx->phi.as<double>());
+                               T.proxy_xyz.as<double4>(), ctx->phi.as<double>(), ts);
         }
-        if (ev) FSS_HIP(hipEventRecord(ev[1], s));
-        if (T.n_near > 0) {
+            if (T.n_near > 0) {
             // default 4 targets per lane; the treecode's near pairs use the sphere form
             auto kn = bltc ? (ctx->near_r == 2 ? k_near<double, 2, true> : k_near<double, 4, true>)
                            : (ctx->near_r == 2 ? k_near<double, 2, false> : k_near<double, 4, false>);
             hipLaunchKernelGGL(kn, dim3((unsigned)T.n_near), dim3(64), 0, s, T.near_items.as<NearItem>(),
                                T.near_src.as<int32_t>(), src, T.recid.as<int32_t>(), T.recnode.as<int32_t>(), p0, p,
-                               T.d_info, pp->x, pp->y, pp->z, ost, ctx->out3.as<double>());
+                               T.d_info, pp->x, pp->y, pp->z, ost, ctx->out3.as<double>(), ts);
         }
-        if (ev) FSS_HIP(hipEventRecord(ev[2], s));
-    } else {
+        } else {
         FSS_TRY(ctx->src32.ensure(sizeof(float4) * nsrc + sizeof(float) * nprox));
         float4 *src = ctx->src32.as<float4>();
         float *aoff = reinterpret_cast<float *>(src + nsrc);
         hipLaunchKernelGGL(k_gather32, dim3(gs), dim3(256), 0, s, pp->x, pp->y, pp->z, pp->vort,
                            pp->area, T.recid.as<int32_t>(), p0, T.proxy_xyz.as<double4>(), nprox, p,
                            T.recnode.as<int32_t>(), T.d_info, bltc ? 0 : 1, src,
-                           aoff);
+                           aoff, ts);
         if (bltc) FSS_TRY((upward<float, D>(ctx, src)));
-        if (ev) FSS_HIP(hipEventRecord(ev[4], s));
-        if (T.n_proxy > 0)
+            if (T.n_proxy > 0)
         {
             hipLaunchKernelGGL((k_proxy_list<float, D>), dim3((unsigned)div_up(T.n_proxy, 4)), dim3(256), 0, s,
                                T.proxy_items.as<ProxyItem>(), T.n_proxy, T.far_off.as<int64_t>(), T.far_src.as<int32_t>(), src,
                                T.recnode.as<int32_t>(), (const float *)aoff, p0, T.d_info,
-                               T.proxy_xyz.as<double4>(), ctx->phi.as<double>());
+                               T.proxy_xyz.as<double4>(), ctx->phi.as<double>(), ts);
         }
-        if (ev) FSS_HIP(hipEventRecord(ev[1], s));
-        if (T.n_near > 0) {
+            if (T.n_near > 0) {
             auto kn = ctx->near_r == 4 ? k_near<float, 4, false> : k_near<float, 2, false>; // default 2
             hipLaunchKernelGGL(kn, dim3((unsigned)T.n_near), dim3(64), 0, s, T.near_items.as<NearItem>(),
                                T.near_src.as<int32_t>(), src, T.recid.as<int32_t>(), T.recnode.as<int32_t>(), p0, p,
-                               T.d_info, pp->x, pp->y, pp->z, ost, ctx->out3.as<double>());
+                               T.d_info, pp->x, pp->y, pp->z, ost, ctx->out3.as<double>(), ts);
         }
-        if (ev) FSS_HIP(hipEventRecord(ev[2], s));
-    }
+        }
     if (T.n_slot > 0)
         hipLaunchKernelGGL((k_solve<D>), dim3((unsigned)div_up(3 * T.n_slot, 128)), dim3(128), 0, s,
                            T.proxy_slots.as<ProxySlot>(), T.n_slot, ctx->phi.as<double>(),
-                           ctx->d_lu.as<double>(), ctx->d_perm.as<int32_t>(), ctx->alpha.as<double>());
+                           ctx->d_lu.as<double>(), ctx->d_perm.as<int32_t>(), ctx->alpha.as<double>(), ts);
+    uint64_t *first = T.n_slot > 0 ? nullptr : ts;
     if (mixed)
         hipLaunchKernelGGL((k_combine<float, D>), dim3((unsigned)div_up(p0, 256)), dim3(256), 0, s,
                            T.recid.as<int32_t>(), T.recnode.as<int32_t>(), T.rinfo.as<uint8_t>(), T.nrange.as<int4>(),
@@ -1276,7 +1279,7 @@ static fss_status run_degree(fss_ctx *ctx, const fss_particles *pp, fss_velocity
                            T.inv_active.as<int32_t>(), ctx->alpha.as<double>(), T.d_tinv,
                            ctx->src32.as<float4>(), T.d_info, T.inst.as<Instance>(), T.ninst, p0, ost,
                            ctx->out3.as<double>(), bltc ? 1 : 0, scale, ctx->cfg.omega, out->u, out->v, out->w,
-                           out->dvort);
+                           out->dvort, first, ts);
     else
         hipLaunchKernelGGL((k_combine<double, D>), dim3((unsigned)div_up(p0, 256)), dim3(256), 0, s,
                            T.recid.as<int32_t>(), T.recnode.as<int32_t>(), T.rinfo.as<uint8_t>(), T.nrange.as<int4>(),
@@ -1284,15 +1287,14 @@ static fss_status run_degree(fss_ctx *ctx, const fss_particles *pp, fss_velocity
                            T.inv_active.as<int32_t>(), ctx->alpha.as<double>(), T.d_tinv,
                            ctx->src64.as<double4>(), T.d_info, T.inst.as<Instance>(), T.ninst, p0, ost,
                            ctx->out3.as<double>(), bltc ? 1 : 0, scale, ctx->cfg.omega, out->u, out->v, out->w,
-                           out->dvort);
-    if (ev) FSS_HIP(hipEventRecord(ev[3], s));
+                           out->dvort, first, ts);
     FSS_HIP(hipGetLastError());
     return FSS_OK;
 }
 
 // FP64 source records of a stage (tree order + proxies) with the BLTC
 // modified charges, for other kernels on the same plan (the SAL treecode)
-template <int D> static fss_status sources64_degree(fss_ctx *ctx, const fss_particles *pp)
+template <int D> static fss_status sources64_degree(fss_ctx *ctx, const fss_particles *pp, uint64_t *ts)
 {
     Tree &T = ctx->tree;
     hipStream_t s = ctx->stream;
@@ -1301,23 +1303,23 @@ template <int D> static fss_status sources64_degree(fss_ctx *ctx, const fss_part
     FSS_TRY(ctx->src64.ensure(sizeof(double4) * nsrc));
     double4 *src = ctx->src64.as<double4>();
     hipLaunchKernelGGL(k_gather64, dim3((unsigned)div_up(nsrc, 256)), dim3(256), 0, s, pp->x, pp->y, pp->z, pp->vort,
-                       pp->area, T.recid.as<int32_t>(), p0, T.proxy_xyz.as<double4>(), nprox, src);
+                       pp->area, T.recid.as<int32_t>(), p0, T.proxy_xyz.as<double4>(), nprox, src, ts);
     FSS_TRY((upward<double, D>(ctx, src)));
     FSS_HIP(hipGetLastError());
     return FSS_OK;
 }
 
-fss_status tree_sources64(fss_ctx *ctx, const fss_particles *pp)
+fss_status tree_sources64(fss_ctx *ctx, const fss_particles *pp, uint64_t *ts)
 {
     switch (ctx->interp.degree) {
-    case 1: return sources64_degree<1>(ctx, pp);
-    case 2: return sources64_degree<2>(ctx, pp);
-    case 3: return sources64_degree<3>(ctx, pp);
-    case 4: return sources64_degree<4>(ctx, pp);
-    case 5: return sources64_degree<5>(ctx, pp);
-    case 6: return sources64_degree<6>(ctx, pp);
-    case 7: return sources64_degree<7>(ctx, pp);
-    case 8: return sources64_degree<8>(ctx, pp);
+    case 1: return sources64_degree<1>(ctx, pp, ts);
+    case 2: return sources64_degree<2>(ctx, pp, ts);
+    case 3: return sources64_degree<3>(ctx, pp, ts);
+    case 4: return sources64_degree<4>(ctx, pp, ts);
+    case 5: return sources64_degree<5>(ctx, pp, ts);
+    case 6: return sources64_degree<6>(ctx, pp, ts);
+    case 7: return sources64_degree<7>(ctx, pp, ts);
+    case 8: return sources64_degree<8>(ctx, pp, ts);
     default: set_error("unsupported degree"); return FSS_ERR_INVALID;
     }
 }
@@ -1333,21 +1335,24 @@ fss_status velocity_tree(fss_ctx *ctx, const fss_particles *pp, fss_velocity *ou
         set_error("particle count differs from the tree's");
         return FSS_ERR_INVALID;
     }
-    hipEvent_t *ev = nullptr;
+    uint64_t *ts = nullptr;
     if (!ctx->capturing) {
-        timing_begin(ctx->timing);
-        ev = ctx->timing.slot();
+        Timing &t = ctx->timing;
+        timing_begin(t, ctx->stream);
+        t.have[t.cur] = (T.n_proxy > 0 ? 1 << Timing::FAR : 0) | (T.n_near > 0 ? 1 << Timing::MAIN : 0) |
+                        1 << Timing::MAIN_END;
+        ts = t.slot();
     }
     fss_status st;
     switch (ctx->interp.degree) {
-    case 1: st = run_degree<1>(ctx, pp, out, ev); break;
-    case 2: st = run_degree<2>(ctx, pp, out, ev); break;
-    case 3: st = run_degree<3>(ctx, pp, out, ev); break;
-    case 4: st = run_degree<4>(ctx, pp, out, ev); break;
-    case 5: st = run_degree<5>(ctx, pp, out, ev); break;
-    case 6: st = run_degree<6>(ctx, pp, out, ev); break;
-    case 7: st = run_degree<7>(ctx, pp, out, ev); break;
-    case 8: st = run_degree<8>(ctx, pp, out, ev); break;
+    case 1: st = run_degree<1>(ctx, pp, out, ts); break;
+    case 2: st = run_degree<2>(ctx, pp, out, ts); break;
+    case 3: st = run_degree<3>(ctx, pp, out, ts); break;
+    case 4: st = run_degree<4>(ctx, pp, out, ts); break;
+    case 5: st = run_degree<5>(ctx, pp, out, ts); break;
+    case 6: st = run_degree<6>(ctx, pp, out, ts); break;
+    case 7: st = run_degree<7>(ctx, pp, out, ts); break;
+    case 8: st = run_degree<8>(ctx, pp, out, ts); break;
     default: set_error("unsupported degree"); return FSS_ERR_INVALID;
     }
     if (st == FSS_OK && !ctx->capturing) ctx->timing.valid = true;

@@ -384,8 +384,10 @@ __global__ void __launch_bounds__(STILE) k_sal_direct_table(const double *__rest
                                                              const double *__restrict__ z,
                                                              const double *__restrict__ w, int64_t n,
                                                              const int64_t *__restrict__ idx, int64_t m,
-                                                             SalTab tab, double g0, double *out)
+                                                             SalTab tab, double g0, double *out, uint64_t *ts)
 {
+    stamp_start(ts, Timing::START);
+    stamp_start(ts, Timing::MAIN);
     __shared__ double4 tile[STILE];
     int64_t r = (int64_t)blockIdx.x * STILE + threadIdx.x;
     int64_t i = r < m ? (idx ? idx[r] : r) : 0;
@@ -407,6 +409,7 @@ __global__ void __launch_bounds__(STILE) k_sal_direct_table(const double *__rest
         }
     }
     if (r < m) out[r] = acc;
+    stamp_end(ts);
 }
 
 // the same with the learned kernel: every source of a tile is evaluated for
@@ -419,8 +422,10 @@ __global__ void __launch_bounds__(STILE) k_sal_direct_mlp(const double *__restri
                                                           const int64_t *__restrict__ idx, int64_t m,
                                                           const MlpOp *__restrict__ op, double A,
                                                           double mu, double sigma, double g0,
-                                                          float log_smin, float inv_span, double *out)
+                                                          float log_smin, float inv_span, double *out, uint64_t *ts)
 {
+    stamp_start(ts, Timing::START);
+    stamp_start(ts, Timing::MAIN);
     __shared__ double4 tile[STILE];
     __shared__ MlpOp Ml;
     mlp_stage(Ml, op);
@@ -445,6 +450,7 @@ __global__ void __launch_bounds__(STILE) k_sal_direct_mlp(const double *__restri
         }
     }
     if (r < m) out[r] = acc;
+    stamp_end(ts);
 }
 
 __global__ void k_mul(const double *__restrict__ a, const double *__restrict__ b, int64_t n, double *o)
@@ -664,25 +670,22 @@ fss_status sal_direct(fss_ctx *ctx, const double *x, const double *y, const doub
     if (!idx) m = n;
     FSS_TRY(S.w.ensure(sizeof(double) * n));
     hipLaunchKernelGGL(k_mul, dim3((unsigned)div_up(n, 256)), dim3(256), 0, s, eta, area, n, S.w.as<double>());
+    uint64_t *ts = nullptr;
     if (!ctx->capturing) {
-        timing_begin(ctx->timing);
-        FSS_HIP(hipEventRecord(ctx->timing.slot()[0], s));
-        FSS_HIP(hipEventRecord(ctx->timing.slot()[4], s));
-        FSS_HIP(hipEventRecord(ctx->timing.slot()[1], s));
+        Timing &t = ctx->timing;
+        timing_begin(t, ctx->stream);
+        t.have[t.cur] = 1 << Timing::MAIN;
+        ts = t.slot();
     }
     unsigned g = (unsigned)div_up(m, STILE);
     float lmin = (float)std::log(S.s_min), ispan = (float)(1.0 / -std::log(S.s_min));
     if (kind == 0)
         hipLaunchKernelGGL(k_sal_direct_table, dim3(g), dim3(STILE), 0, s, x, y, z, S.w.as<double>(), n, idx, m,
-                           sal_tab(S.tab.as<double>(), S.M), S.g0, out);
+                           sal_tab(S.tab.as<double>(), S.M), S.g0, out, ts);
     else
         hipLaunchKernelGGL(k_sal_direct_mlp, dim3(g), dim3(STILE), 0, s, x, y, z, S.w.as<double>(), n, idx, m,
-                           S.mlpop.as<MlpOp>(), S.A, S.mu, S.sigma, S.g0, lmin, ispan, out);
-    if (!ctx->capturing) {
-        FSS_HIP(hipEventRecord(ctx->timing.slot()[2], s));
-        FSS_HIP(hipEventRecord(ctx->timing.slot()[3], s));
-        ctx->timing.valid = true;
-    }
+                           S.mlpop.as<MlpOp>(), S.A, S.mu, S.sigma, S.g0, lmin, ispan, out, ts);
+    if (ts) ctx->timing.valid = true;
     FSS_HIP(hipGetLastError());
     return FSS_OK;
 }

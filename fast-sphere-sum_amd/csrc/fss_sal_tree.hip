@@ -32,6 +32,7 @@ struct KernelArgs {
     float log_smin, inv_span;
     const double *c;
     int N;
+    uint64_t *ts_near, *ts_proxy, *ts; // time stamps, or null
 };
 
 __device__ inline double dist2(const double4 &a, const double4 &b)
@@ -61,6 +62,7 @@ __global__ void __launch_bounds__(64) k_sal_near(const NearItem *__restrict__ it
                                                  const int32_t *__restrict__ near_src,
                                                  const double4 *__restrict__ src, KernelArgs ka, double *out)
 {
+    stamp_start(ka.ts_near, Timing::MAIN);
     __shared__ double4 lds[NCH_S];
     __shared__ double red[64];
     const NearItem it = items[blockIdx.x];
@@ -104,6 +106,7 @@ __global__ void __launch_bounds__(64) k_sal_proxy(const ProxyItem *__restrict__ 
                                                   const double4 *__restrict__ src, int64_t p0, KernelArgs ka,
                                                   double *phi)
 {
+    stamp_start(ka.ts_proxy, Timing::MAIN);
     constexpr int PP = npts_s<D>();
     constexpr int P = 64 / PP;
     __shared__ double4 lds[NCH_S];
@@ -168,6 +171,7 @@ __global__ void __launch_bounds__(256) k_sal_near_mlp(const NearItem *__restrict
                                                       const int32_t *__restrict__ near_src,
                                                       const double4 *__restrict__ src, KernelArgs ka, double *out)
 {
+    stamp_start(ka.ts_near, Timing::MAIN);
     __shared__ MlpOp Ml;
     __shared__ double4 stage[4][NCH_M];
     __shared__ double red[4][64];
@@ -220,6 +224,7 @@ __global__ void __launch_bounds__(256) k_sal_proxy_mlp(const ProxyItem *__restri
                                                        const double4 *__restrict__ src, int64_t p0, KernelArgs ka,
                                                        double *phi)
 {
+    stamp_start(ka.ts_proxy, Timing::MAIN);
     constexpr int PP = npts_s<D>();
     constexpr int P = 64 / PP;
     __shared__ MlpOp Ml;
@@ -390,10 +395,11 @@ __global__ void k_sal_combine(const int32_t *__restrict__ recid, const int32_t *
 }
 
 __global__ void k_sal_scatter(const int32_t *__restrict__ ipos, int64_t n, const double *__restrict__ acc,
-                              double *out)
+                              double *out, uint64_t *ts)
 {
     int64_t id = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
     if (id < n) out[id] = acc[ipos[id]];
+    stamp_end(ts);
 }
 
 template <int KIND, int D> fss_status run(fss_ctx *ctx, const KernelArgs &ka, double *result)
@@ -437,7 +443,7 @@ template <int KIND, int D> fss_status run(fss_ctx *ctx, const KernelArgs &ka, do
                        ctx->alpha.as<double>(), T.d_tinv, src, T.inst.as<Instance>(), T.ninst, p0,
                        ctx->out3.as<double>(), ctx->acc3.as<double>());
     hipLaunchKernelGGL(k_sal_scatter, dim3((unsigned)div_up(T.n, 256)), dim3(256), 0, s, T.ipos.as<int32_t>(), T.n,
-                       ctx->acc3.as<double>(), result);
+                       ctx->acc3.as<double>(), result, ka.ts);
     FSS_HIP(hipGetLastError());
     return FSS_OK;
 }
@@ -479,24 +485,18 @@ fss_status sal_tree(fss_ctx *ctx, const fss_particles *pp, int kind, double *out
     ka.inv_span = (float)(1.0 / -std::log(S.s_min));
     ka.c = S.c.as<double>();
     ka.N = S.nmax;
-    hipEvent_t *ev = nullptr;
+    ka.ts = ka.ts_near = ka.ts_proxy = nullptr;
     if (!ctx->capturing) {
-        timing_begin(ctx->timing);
-        ev = ctx->timing.slot();
-        FSS_HIP(hipEventRecord(ev[0], ctx->stream));
+        Timing &t = ctx->timing;
+        timing_begin(t, ctx->stream);
+        t.have[t.cur] = T.n_near > 0 || T.n_proxy > 0 ? 1 << Timing::MAIN : 0;
+        ka.ts = t.slot();
+        (T.n_near > 0 ? ka.ts_near : ka.ts_proxy) = ka.ts;
     }
-    FSS_TRY(tree_sources64(ctx, pp)); // records w = eta A and the modified charges
-    if (ev) {
-        FSS_HIP(hipEventRecord(ev[4], ctx->stream));
-        FSS_HIP(hipEventRecord(ev[1], ctx->stream));
-    }
+    FSS_TRY(tree_sources64(ctx, pp, ka.ts)); // records w = eta A and the modified charges
     fss_status st = kind == 0 ? run_kind<0>(ctx, ka, out) : kind == 1 ? run_kind<1>(ctx, ka, out)
                                                                     : run_kind<2>(ctx, ka, out);
-    if (ev) {
-        FSS_HIP(hipEventRecord(ev[2], ctx->stream));
-        FSS_HIP(hipEventRecord(ev[3], ctx->stream));
-        ctx->timing.valid = true;
-    }
+    if (ka.ts) ctx->timing.valid = true;
     return st;
 }
 

@@ -330,13 +330,12 @@ class Context:
 
     def _particles(self, x, y, z, vort, area):
         _check_state(self.device, x, y, z, vort, area)
-        return Particles(_dev_ptr(x).value, _dev_ptr(y).value, _dev_ptr(z).value,
-                         _dev_ptr(vort).value, _dev_ptr(area).value, x.numel())
+        return Particles(x.data_ptr(), y.data_ptr(), z.data_ptr(), vort.data_ptr(), area.data_ptr(), x.numel())
 
     def _out(self, m, out=None):
         import torch
         if out is None:
-            out = [torch.empty(m, dtype=torch.float64, device=self.device) for _ in range(4)]
+            out = torch.empty((4, m), dtype=torch.float64, device=self.device).unbind(0)
         for t in out:
             assert t.numel() == m and t.dtype == torch.float64 and t.is_contiguous()
         return out, Velocity(*(t.data_ptr() for t in out))

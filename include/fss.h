@@ -274,10 +274,11 @@ fss_status fss_amr(int64_t *n, int64_t *ntri, int64_t max_count, int64_t tri_cap
 fss_status fss_project_points(fss_ctx *ctx, double *x, double *y, double *z, double *vort,
                               int64_t n);
 
-/* ---- timing of the last velocity call's kernels (HIP events on the
- * context stream): total stage ms and the dominant kernel's ms. ---- */
+/* ---- timing of the last velocity call's kernels (device clock, read by the
+ * kernels themselves): total stage ms and the dominant kernel's ms.  The
+ * reading calls wait for the context's stream. ---- */
 fss_status fss_last_timing(fss_ctx *ctx, double *stage_ms, double *main_kernel_ms);
-/* Events are recorded into a ring of 256 slots without synchronizing;
+/* Calls are recorded in a ring of 256 slots without synchronizing;
  * fss_timing_reset() starts a new window and fss_timing_mean() returns the
  * mean over the calls since (at most 256). */
 fss_status fss_timing_reset(fss_ctx *ctx);
