@@ -458,7 +458,7 @@ fss_status velocity_direct(fss_ctx *ctx, const fss_particles *p, const int64_t *
     }
     if (!idx) m = n;
     const bool mixed = !force_fp64 && ctx->cfg.precision == FSS_MIXED;
-    DevBuf &buf = mixed ? ctx->src32 : ctx->src64;
+    DevBuf &buf = ctx->direct;
     FSS_TRY(buf.ensure(direct_plan(n, m, mixed).bytes));
     if (ctx->capturing) return launch_direct(ctx, p, idx, m, out, mixed, buf.p, nullptr);
     Timing &t = ctx->timing;

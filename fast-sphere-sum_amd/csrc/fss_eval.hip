@@ -147,49 +147,91 @@ template <int D> constexpr int npts() { return (D + 1) * (D + 2) / 2; }
 // ------------------------------------------------------------------
 // gather: source records in tree order, then the proxies
 // ------------------------------------------------------------------
+// particle of record j; recid null: the caller's arrays are in tree order
+__device__ inline int32_t rec_id(const int32_t *__restrict__ recid, int64_t j) { return recid ? recid[j] : (int32_t)j; }
+
 __global__ void k_gather64(const double *__restrict__ x, const double *__restrict__ y,
                            const double *__restrict__ z, const double *__restrict__ vort,
                            const double *__restrict__ area, const int32_t *__restrict__ recid,
-                           int64_t p0, const double4 *__restrict__ proxy, int64_t nprox,
-                           double4 *src, uint64_t *ts)
+                           int64_t p0, double4 *src, uint64_t *ts)
 {
     stamp_start(ts, Timing::START);
     int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (i < p0) {
-        int32_t id = recid[i];
-        src[i] = make_double4(x[id], y[id], z[id], vort[id] * area[id]);
-    } else if (i < p0 + nprox) {
-        double4 q = proxy[i - p0];
-        src[i] = make_double4(q.x, q.y, q.z, 0.0);
-    }
+    if (i >= p0) return;
+    int32_t id = rec_id(recid, i);
+    src[i] = make_double4(x[id], y[id], z[id], vort[id] * area[id]);
 }
 
 __global__ void k_gather32(const double *__restrict__ x, const double *__restrict__ y,
                            const double *__restrict__ z, const double *__restrict__ vort,
                            const double *__restrict__ area, const int32_t *__restrict__ recid,
-                           int64_t p0, const double4 *__restrict__ proxy, int64_t nprox, int p,
-                           const int32_t *__restrict__ recnode, const double *__restrict__ centres,
-                           int planar, float4 *src, float *aoff, uint64_t *ts)
+                           int64_t p0, const int32_t *__restrict__ recnode, const double *__restrict__ centres,
+                           float4 *src, uint64_t *ts)
 {
     stamp_start(ts, Timing::START);
     // FP32 records hold the offset from the centre of the record's node
     // (FP64 subtraction, then rounding): differences of nearby points keep
     // ~1e-9 absolute accuracy instead of the 6e-8 of rounded coordinates.
     int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (i < p0) {
-        int32_t id = recid[i];
-        const double *c = centres + 4 * (int64_t)recnode[i];
-        src[i] = make_float4((float)(x[id] - c[0]), (float)(y[id] - c[1]), (float)(z[id] - c[2]),
-                             (float)(2.0 * vort[id] * area[id]));
-    } else if (i < p0 + nprox) {
-        double4 q = proxy[i - p0];
-        const double *c = centres + 4 * ((i - p0) / p);
-        src[i] = make_float4((float)(q.x - c[0]), (float)(q.y - c[1]), (float)(q.z - c[2]), 0.0f);
-        // For a particle x on the sphere, 2 (1 - y.x) = |x - y|^2 + (1 - |y|^2).
-        // Planar proxies (PARITY) are off the sphere and carry that offset.
-        double nq = q.x * q.x + q.y * q.y + q.z * q.z;
-        aoff[i - p0] = planar ? (float)(1.0 - nq) : 0.0f;
-    }
+    if (i >= p0) return;
+    int32_t id = rec_id(recid, i);
+    const double *c = centres + 4 * (int64_t)recnode[i];
+    src[i] = make_float4((float)(x[id] - c[0]), (float)(y[id] - c[1]), (float)(z[id] - c[2]),
+                         (float)(2.0 * vort[id] * area[id]));
+}
+
+// The proxies' records: static but for the weight, which the upward pass writes
+// for the charge nodes, so they are laid down with the plan.  Copied with every
+// gather they were half of it at degree 7 on the level-10 grid (436,900 nodes of 36
+// proxies: 288 us, 143 without).
+__global__ void k_proxy_records64(const double4 *__restrict__ proxy, int64_t nprox, double4 *src)
+{
+    int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    if (i >= nprox) return;
+    double4 q = proxy[i];
+    src[i] = make_double4(q.x, q.y, q.z, 0.0);
+}
+
+__global__ void k_proxy_records32(const double4 *__restrict__ proxy, int64_t nprox, int p,
+                                  const double *__restrict__ centres, int planar, float4 *src, float *aoff)
+{
+    int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    if (i >= nprox) return;
+    double4 q = proxy[i];
+    const double *c = centres + 4 * (i / p);
+    src[i] = make_float4((float)(q.x - c[0]), (float)(q.y - c[1]), (float)(q.z - c[2]), 0.0f);
+    // For a particle x on the sphere, 2 (1 - y.x) = |x - y|^2 + (1 - |y|^2).
+    // Planar proxies (PARITY) are off the sphere and carry that offset.
+    double nq = q.x * q.x + q.y * q.y + q.z * q.z;
+    aoff[i] = planar ? (float)(1.0 - nq) : 0.0f;
+}
+
+// source records of the plan: room for the particles', the proxies' laid down.
+// In mixed precision the FP64 records serve only the SAL treecode and are laid
+// down by its calls.
+static fss_status proxy_records64(fss_ctx *ctx)
+{
+    Tree &T = ctx->tree;
+    const int64_t nprox = T.nn * ctx->interp.p;
+    FSS_TRY(T.src64.ensure(sizeof(double4) * (T.p0 + nprox)));
+    hipLaunchKernelGGL(k_proxy_records64, dim3((unsigned)div_up(nprox, 256)), dim3(256), 0, ctx->stream,
+                       T.proxy_xyz.as<double4>(), nprox, T.src64.as<double4>() + T.p0);
+    FSS_HIP(hipGetLastError());
+    return FSS_OK;
+}
+
+fss_status proxy_records(fss_ctx *ctx)
+{
+    Tree &T = ctx->tree;
+    if (ctx->cfg.precision != FSS_MIXED) return proxy_records64(ctx);
+    const int64_t nprox = T.nn * ctx->interp.p, nsrc = T.p0 + nprox;
+    FSS_TRY(T.src32.ensure(sizeof(float4) * nsrc + sizeof(float) * nprox));
+    float4 *src = T.src32.as<float4>();
+    hipLaunchKernelGGL(k_proxy_records32, dim3((unsigned)div_up(nprox, 256)), dim3(256), 0, ctx->stream,
+                       T.proxy_xyz.as<double4>(), nprox, ctx->interp.p, T.d_info,
+                       ctx->cfg.eval_mode == FSS_EVAL_BLTC ? 0 : 1, src + T.p0, reinterpret_cast<float *>(src + nsrc));
+    FSS_HIP(hipGetLastError());
+    return FSS_OK;
 }
 
 // ------------------------------------------------------------------
@@ -461,7 +503,7 @@ __device__ inline void target_pos(const float4 *, const int32_t *__restrict__ re
                                   const double *__restrict__ x, const double *__restrict__ y,
                                   const double *__restrict__ z, double *o)
 {
-    const int32_t id = recid[j];
+    const int32_t id = rec_id(recid, j);
     o[0] = x[id];
     o[1] = y[id];
     o[2] = z[id];
@@ -669,7 +711,7 @@ __global__ void __launch_bounds__(64, sizeof(Real) == 4 && R == 2 ? 8 : 4) k_nea
         int tt = (act && t < cnt) ? t : 0;
         int64_t j = (int64_t)it.tgt_start + tt;
         xt[q] = to_frame(src[j], recnode[j], centres, ct);
-        tid[q] = recid[j];
+        tid[q] = rec_id(recid, j);
     }
     Acc<Real, R> A;
     A.zero();
@@ -707,7 +749,7 @@ __global__ void __launch_bounds__(64, sizeof(Real) == 4 && R == 2 ? 8 : 4) k_nea
                 rec[s] = src[j];
                 const int32_t rn = recnode[min((int64_t)j, p0 - 1)];
                 nd[s] = j < p0 ? rn : (int32_t)((uint32_t)(j - p0) / (uint32_t)p);
-                id[s] = self_part ? recid[min((int64_t)j, p0 - 1)] : 0;
+                id[s] = self_part ? rec_id(recid, min((int64_t)j, p0 - 1)) : 0;
             }
 #pragma unroll
             for (int s = 0; s < S / 2; s++) rec[s] = to_frame(rec[s], nd[s], centres, ct);
@@ -1102,7 +1144,7 @@ __global__ void k_combine(const int32_t *__restrict__ recid, const int32_t *__re
     }
     const Instance I = inst[lo];
     if (i - I.rbase >= I.n) return; // exception record
-    const int64_t id = recid[i];
+    const int64_t id = rec_id(recid, i);
     double pt[3], wdummy;
     rec_point(src[i], recnode[i], centres, pt, wdummy);
     const int info = rinfo[i];
@@ -1209,25 +1251,24 @@ static fss_status upward(fss_ctx *ctx, typename Rec<Real>::T4 *src)
 }
 
 template <int D>
-static fss_status run_degree(fss_ctx *ctx, const fss_particles *pp, fss_velocity *out, uint64_t *ts)
+static fss_status run_degree(fss_ctx *ctx, const fss_particles *pp, fss_velocity *out, const int32_t *recid, uint64_t *ts)
 {
     Tree &T = ctx->tree;
     hipStream_t s = ctx->stream;
     constexpr int p = npts<D>();
     const bool mixed = ctx->cfg.precision == FSS_MIXED;
     const bool bltc = ctx->cfg.eval_mode == FSS_EVAL_BLTC;
-    const int64_t p0 = T.p0, nprox = T.nn * p, nsrc = p0 + nprox;
+    const int64_t p0 = T.p0, nsrc = p0 + T.nn * p;
     const double scale = -1.0 / (4.0 * M_PI);
     const int64_t ost = std::max<int64_t>(1, T.nslot_out);
     FSS_TRY(ctx->out3.ensure(sizeof(double) * 3 * ost));
     FSS_TRY(ctx->phi.ensure(sizeof(double) * 3 * p * std::max<int64_t>(1, T.n_proxy)));
     FSS_TRY(ctx->alpha.ensure(sizeof(double) * 3 * p * std::max<int64_t>(1, T.n_slot)));
-    unsigned gs = (unsigned)div_up(nsrc, 256);
+    const dim3 gs((unsigned)div_up(p0, 256));
     if (!mixed) {
-        FSS_TRY(ctx->src64.ensure(sizeof(double4) * nsrc));
-        double4 *src = ctx->src64.as<double4>();
-        hipLaunchKernelGGL(k_gather64, dim3(gs), dim3(256), 0, s, pp->x, pp->y, pp->z, pp->vort,
-                           pp->area, T.recid.as<int32_t>(), p0, T.proxy_xyz.as<double4>(), nprox, src, ts);
+        double4 *src = T.src64.as<double4>();
+        hipLaunchKernelGGL(k_gather64, gs, dim3(256), 0, s, pp->x, pp->y, pp->z, pp->vort, pp->area, recid, p0, src,
+                           ts);
         if (bltc) FSS_TRY((upward<double, D>(ctx, src)));
             if (T.n_proxy > 0)
         {
@@ -1241,17 +1282,14 @@ static fss_status run_degree(fss_ctx *ctx, const fss_particles *pp, fss_velocity
             auto kn = bltc ? (ctx->near_r == 2 ? k_near<double, 2, true> : k_near<double, 4, true>)
                            : (ctx->near_r == 2 ? k_near<double, 2, false> : k_near<double, 4, false>);
             hipLaunchKernelGGL(kn, dim3((unsigned)T.n_near), dim3(64), 0, s, T.near_items.as<NearItem>(),
-                               T.near_src.as<int32_t>(), src, T.recid.as<int32_t>(), T.recnode.as<int32_t>(), p0, p,
+                               T.near_src.as<int32_t>(), src, recid, T.recnode.as<int32_t>(), p0, p,
                                T.d_info, pp->x, pp->y, pp->z, ost, ctx->out3.as<double>(), ts);
         }
         } else {
-        FSS_TRY(ctx->src32.ensure(sizeof(float4) * nsrc + sizeof(float) * nprox));
-        float4 *src = ctx->src32.as<float4>();
+        float4 *src = T.src32.as<float4>();
         float *aoff = reinterpret_cast<float *>(src + nsrc);
-        hipLaunchKernelGGL(k_gather32, dim3(gs), dim3(256), 0, s, pp->x, pp->y, pp->z, pp->vort,
-                           pp->area, T.recid.as<int32_t>(), p0, T.proxy_xyz.as<double4>(), nprox, p,
-                           T.recnode.as<int32_t>(), T.d_info, bltc ? 0 : 1, src,
-                           aoff, ts);
+        hipLaunchKernelGGL(k_gather32, gs, dim3(256), 0, s, pp->x, pp->y, pp->z, pp->vort, pp->area, recid, p0,
+                           T.recnode.as<int32_t>(), T.d_info, src, ts);
         if (bltc) FSS_TRY((upward<float, D>(ctx, src)));
             if (T.n_proxy > 0)
         {
@@ -1263,7 +1301,7 @@ static fss_status run_degree(fss_ctx *ctx, const fss_particles *pp, fss_velocity
             if (T.n_near > 0) {
             auto kn = ctx->near_r == 4 ? k_near<float, 4, false> : k_near<float, 2, false>; // default 2
             hipLaunchKernelGGL(kn, dim3((unsigned)T.n_near), dim3(64), 0, s, T.near_items.as<NearItem>(),
-                               T.near_src.as<int32_t>(), src, T.recid.as<int32_t>(), T.recnode.as<int32_t>(), p0, p,
+                               T.near_src.as<int32_t>(), src, recid, T.recnode.as<int32_t>(), p0, p,
                                T.d_info, pp->x, pp->y, pp->z, ost, ctx->out3.as<double>(), ts);
         }
         }
@@ -1274,18 +1312,18 @@ static fss_status run_degree(fss_ctx *ctx, const fss_particles *pp, fss_velocity
     uint64_t *first = T.n_slot > 0 ? nullptr : ts;
     if (mixed)
         hipLaunchKernelGGL((k_combine<float, D>), dim3((unsigned)div_up(p0, 256)), dim3(256), 0, s,
-                           T.recid.as<int32_t>(), T.recnode.as<int32_t>(), T.rinfo.as<uint8_t>(), T.nrange.as<int4>(),
+                           recid, T.recnode.as<int32_t>(), T.rinfo.as<uint8_t>(), T.nrange.as<int4>(),
                            T.oslot.as<int32_t>(), T.node_slot.as<int32_t>(), T.nodeof.as<int32_t>(),
                            T.inv_active.as<int32_t>(), ctx->alpha.as<double>(), T.d_tinv,
-                           ctx->src32.as<float4>(), T.d_info, T.inst.as<Instance>(), T.ninst, p0, ost,
+                           T.src32.as<float4>(), T.d_info, T.inst.as<Instance>(), T.ninst, p0, ost,
                            ctx->out3.as<double>(), bltc ? 1 : 0, scale, ctx->cfg.omega, out->u, out->v, out->w,
                            out->dvort, first, ts);
     else
         hipLaunchKernelGGL((k_combine<double, D>), dim3((unsigned)div_up(p0, 256)), dim3(256), 0, s,
-                           T.recid.as<int32_t>(), T.recnode.as<int32_t>(), T.rinfo.as<uint8_t>(), T.nrange.as<int4>(),
+                           recid, T.recnode.as<int32_t>(), T.rinfo.as<uint8_t>(), T.nrange.as<int4>(),
                            T.oslot.as<int32_t>(), T.node_slot.as<int32_t>(), T.nodeof.as<int32_t>(),
                            T.inv_active.as<int32_t>(), ctx->alpha.as<double>(), T.d_tinv,
-                           ctx->src64.as<double4>(), T.d_info, T.inst.as<Instance>(), T.ninst, p0, ost,
+                           T.src64.as<double4>(), T.d_info, T.inst.as<Instance>(), T.ninst, p0, ost,
                            ctx->out3.as<double>(), bltc ? 1 : 0, scale, ctx->cfg.omega, out->u, out->v, out->w,
                            out->dvort, first, ts);
     FSS_HIP(hipGetLastError());
@@ -1298,12 +1336,10 @@ template <int D> static fss_status sources64_degree(fss_ctx *ctx, const fss_part
 {
     Tree &T = ctx->tree;
     hipStream_t s = ctx->stream;
-    constexpr int p = npts<D>();
-    const int64_t p0 = T.p0, nprox = T.nn * p, nsrc = p0 + nprox;
-    FSS_TRY(ctx->src64.ensure(sizeof(double4) * nsrc));
-    double4 *src = ctx->src64.as<double4>();
-    hipLaunchKernelGGL(k_gather64, dim3((unsigned)div_up(nsrc, 256)), dim3(256), 0, s, pp->x, pp->y, pp->z, pp->vort,
-                       pp->area, T.recid.as<int32_t>(), p0, T.proxy_xyz.as<double4>(), nprox, src, ts);
+    if (ctx->cfg.precision == FSS_MIXED) FSS_TRY(proxy_records64(ctx));
+    double4 *src = T.src64.as<double4>();
+    hipLaunchKernelGGL(k_gather64, dim3((unsigned)div_up(T.p0, 256)), dim3(256), 0, s, pp->x, pp->y, pp->z, pp->vort,
+                       pp->area, T.recid.as<int32_t>(), T.p0, src, ts);
     FSS_TRY((upward<double, D>(ctx, src)));
     FSS_HIP(hipGetLastError());
     return FSS_OK;
@@ -1324,9 +1360,10 @@ fss_status tree_sources64(fss_ctx *ctx, const fss_particles *pp, uint64_t *ts)
     }
 }
 
-fss_status velocity_tree(fss_ctx *ctx, const fss_particles *pp, fss_velocity *out)
+fss_status velocity_tree(fss_ctx *ctx, const fss_particles *pp, fss_velocity *out, bool tree_order)
 {
     Tree &T = ctx->tree;
+    const int32_t *recid = tree_order ? nullptr : T.recid.as<int32_t>();
     if (!T.built) {
         set_error("fss_velocity_tree before fss_tree_build");
         return FSS_ERR_STATE;
@@ -1345,14 +1382,14 @@ fss_status velocity_tree(fss_ctx *ctx, const fss_particles *pp, fss_velocity *ou
     }
     fss_status st;
     switch (ctx->interp.degree) {
-    case 1: st = run_degree<1>(ctx, pp, out, ts); break;
-    case 2: st = run_degree<2>(ctx, pp, out, ts); break;
-    case 3: st = run_degree<3>(ctx, pp, out, ts); break;
-    case 4: st = run_degree<4>(ctx, pp, out, ts); break;
-    case 5: st = run_degree<5>(ctx, pp, out, ts); break;
-    case 6: st = run_degree<6>(ctx, pp, out, ts); break;
-    case 7: st = run_degree<7>(ctx, pp, out, ts); break;
-    case 8: st = run_degree<8>(ctx, pp, out, ts); break;
+    case 1: st = run_degree<1>(ctx, pp, out, recid, ts); break;
+    case 2: st = run_degree<2>(ctx, pp, out, recid, ts); break;
+    case 3: st = run_degree<3>(ctx, pp, out, recid, ts); break;
+    case 4: st = run_degree<4>(ctx, pp, out, recid, ts); break;
+    case 5: st = run_degree<5>(ctx, pp, out, recid, ts); break;
+    case 6: st = run_degree<6>(ctx, pp, out, recid, ts); break;
+    case 7: st = run_degree<7>(ctx, pp, out, recid, ts); break;
+    case 8: st = run_degree<8>(ctx, pp, out, recid, ts); break;
     default: set_error("unsupported degree"); return FSS_ERR_INVALID;
     }
     if (st == FSS_OK && !ctx->capturing) ctx->timing.valid = true;

@@ -209,6 +209,8 @@ struct Tree {
     DevBuf up_items;    // int4 [n_up] {node, first record, records, partial index or -1}
     DevBuf up_multi;    // int4 [n_up_multi] {node, first partial, end partial, 0}
     DevBuf proxy_xyz;   // double4 [nn * p] static proxy positions (w unused)
+    DevBuf src64;       // double4 [p0 + nn * p] source records (see above)
+    DevBuf src32;       // float4 [p0 + nn * p], then float [nn * p] planar offsets
     int64_t pairs_near = 0, pairs_far = 0;
 };
 
@@ -316,9 +318,7 @@ struct fss_ctx {
     fss::DevBuf d_lu, d_perm, d_vinv, d_pts;
 
     // per-stage workspace
-    fss::DevBuf src64;   // double4 [p0 + nn*p] or [n] for the direct sum
-    fss::DevBuf src32;   // float4
-    fss::DevBuf srcid;   // int32 ids for the direct sum (unused for tree: ids reused)
+    fss::DevBuf direct;  // partial sums or packed records of the direct sum
     fss::DevBuf out3;    // 3 doubles SoA [p0] per-position partial velocities
     fss::DevBuf phi;     // 3*p doubles per proxy work item (partial proxy values)
     fss::DevBuf alpha;   // 3*p doubles per interpolant slot
@@ -327,7 +327,7 @@ struct fss_ctx {
     int near_r = 0;      // targets per lane of the near kernel: 2, 4 or 0 (4 in FP64, 2 in FP32)
     fss::DevBuf rk_k;    // 4 stages x 4 fields x n
     fss::DevBuf rk_y;    // stage state 4 x n
-    int64_t rk_n = 0;
+    fss::DevBuf rk_t;    // state and areas in tree order, 5 x n
 
     // hipGraph of one RK4 step
     hipGraph_t graph = nullptr;
@@ -357,7 +357,11 @@ fss_status tree_export(fss_ctx *ctx, int32_t *loc, uint8_t *found, int32_t *coun
 fss_status interp_setup(fss_ctx *ctx);
 
 // ---- evaluation (fss_eval.hip) ----
-fss_status velocity_tree(fss_ctx *ctx, const fss_particles *p, fss_velocity *out);
+// tree_order: the arrays are in tree order (element i belongs to main record i;
+// only for a tree without exception records)
+fss_status velocity_tree(fss_ctx *ctx, const fss_particles *p, fss_velocity *out, bool tree_order = false);
+// source records of a new plan (room for the particles', the proxies' laid down)
+fss_status proxy_records(fss_ctx *ctx);
 
 // ---- direct sum (fss_direct.hip) ----
 fss_status velocity_direct(fss_ctx *ctx, const fss_particles *p, const int64_t *idx, int64_t m,

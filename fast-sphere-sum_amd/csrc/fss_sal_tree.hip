@@ -408,7 +408,7 @@ template <int KIND, int D> fss_status run(fss_ctx *ctx, const KernelArgs &ka, do
     hipStream_t s = ctx->stream;
     constexpr int p = npts_s<D>();
     const int64_t p0 = T.p0;
-    const double4 *src = ctx->src64.as<double4>();
+    const double4 *src = T.src64.as<double4>();
     FSS_TRY(ctx->out3.ensure(sizeof(double) * std::max<int64_t>(1, T.nslot_out)));
     FSS_TRY(ctx->phi.ensure(sizeof(double) * p * std::max<int64_t>(1, T.n_proxy)));
     FSS_TRY(ctx->alpha.ensure(sizeof(double) * p * std::max<int64_t>(1, T.n_slot)));

@@ -1463,6 +1463,7 @@ fss_status plan_finish(fss_ctx *ctx)
         FSS_HIP(hipMemcpyAsync(&info->up, B.pos.as<int4>() + T.n_charge, sizeof(int4), hipMemcpyDeviceToDevice, s));
         FSS_HIP(hipGetLastError());
     }
+    FSS_TRY(proxy_records(ctx));
     BuildInfo h;
     FSS_TRY(d2h(&h, info, sizeof(h), s));
     if (!T.batched) T.n_proxy = T.n_slot > 0 ? h.n_proxy : 0;
