@@ -213,6 +213,32 @@ def test_rk4_graph_recaptured_after_workspace_grows(fsslib, case4, case5):
         np.testing.assert_array_equal(g, r)
 
 
+def test_rk4_graph_recaptured_after_rebuild(fsslib, case4):
+    """A captured graph holds the launch shapes of the plan it was captured on: a
+    rebuild on as many other particles keeps the buffers, and the next replay must
+    capture again.  The first build is the largest, so the others allocate nothing."""
+    x, y, z, vort, area, _ = case4
+    n, dt = len(x), 0.01
+    kw = dict(tree_levels=4, assign_mode=1, eval_mode=1)
+    ctx = fsslib.Context(**kw)
+    sets = [(x, y, z)]
+    for seed, spread in ((3, 0.2), (4, 0.5)):  # gathered around a point: fewer nodes and items
+        rng = np.random.default_rng(seed)
+        p = rng.normal(0, spread, (3, n)) + np.array([[0.0], [0.0], [1.0]])
+        sets.append(tuple(p / np.linalg.norm(p, axis=0)))
+    for k in (0, 1, 2, 1, 0):
+        b = _dev(*sets[k], vort, area)
+        a = _dev(*sets[k], vort, area)
+        ctx.tree_build(*b[:3])
+        ctx.rk4_run_graph(*b, dt, 3, use_tree=True)
+        ref = fsslib.Context(**kw)
+        ref.tree_build(*a[:3])
+        for _ in range(3):
+            ref.rk4_step(*a, dt, use_tree=True)
+        for g, r in zip(_host(*b[:4]), _host(*a[:4])):
+            np.testing.assert_array_equal(g, r)
+
+
 @pytest.fixture(scope="module")
 def random_case(fsslib):
     n = 12000
