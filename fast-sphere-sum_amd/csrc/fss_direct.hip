@@ -11,6 +11,9 @@
 // fixed order.  Beyond that a block takes a whole group and writes the
 // velocities itself.
 //
+// FP64 sums of all particles are taken over unordered pairs from 3,300
+// particles on (k_direct_sym).
+//
 // Bound by FP64 issue (17 four-cycle slots a pair at four targets a lane: 822 us
 // at N = 40,009, 1.95e12 pairs/s at about 2 GHz).  One target a lane, one block
 // per 256 targets and a reciprocal with two Newton steps per pair took 2,036
@@ -30,6 +33,8 @@
 //       are FP64.
 #include <algorithm>
 #include <cmath>
+#include <functional>
+#include <initializer_list>
 #include <mutex>
 
 #include "fss_internal.h"
@@ -90,7 +95,7 @@ struct DirectArgs {
     uint64_t *ts; // time stamps, or null
 };
 
-__device__ inline void direct_source(const DirectArgs &a, int64_t j, double4 &s)
+template <typename Args> __device__ inline void direct_source(const Args &a, int64_t j, double4 &s)
 {
     s = make_double4(a.x[j], a.y[j], a.z[j], a.vort[j] * a.area[j]);
 }
@@ -343,6 +348,239 @@ __global__ void __launch_bounds__(256) k_direct_sum(const double *__restrict__ p
     stamp_end(ts);
 }
 
+// ------------------------------------------------------------------
+// FP64 sum over unordered pairs: 1 - x.y and its reciprocal serve both
+// directions of a pair
+// ------------------------------------------------------------------
+// k_direct runs at the FP64 issue rate, so only fewer instructions help: a pair
+// in both directions takes 21.5 four-cycle slots at four targets a lane against
+// 2 x 17.  A block holds a row of T = 256 R targets (R a lane, w_i with them) and
+// walks the tiles of 64 particles from the row's own on.  In a tile every lane
+// starts at its own source and takes the next lane's at each of 64 steps (read
+// from LDS), while the sums of the sources travel the ring of lanes the other
+// way by one DPP move a word (a tenth of a step); after 64 steps every source's
+// sum is back with its lane, the four waves' are added and stored as column sums
+// of the row.  The row's own tiles take their pairs in one direction, which
+// keeps the self test and the remainders out of the main loop.  k_sym_sum adds
+// each target's column and run sums in a fixed order; rows go in slabs so that
+// both fit a bounded workspace.  N = 100,003: 1.98e12 -> 2.56e12 ordered pairs/s
+// (102 cycles a step and target at about 2 GHz, 98 of them issue).
+struct SymArgs {
+    const double *x, *y, *z, *vort, *area;
+    int64_t n, K;      // particles, tiles of 64 of them
+    int64_t r0, r1;    // rows of targets of this launch
+    int64_t U, B1, q1, q; // its units, and their cut into runs
+    double scale, omega;
+    double *col, *part;
+    double *u, *v, *w, *dvort;
+    uint64_t *ts;
+};
+
+// Row r: targets [r T, (r + 1) T); its units are the tiles r RT .. K - 1 (RT = T /
+// 64), numbered row by row from row r0; its column sums are those of the
+// particles after the row.
+__host__ __device__ inline int64_t sym_first(int64_t r, int64_t r0, int64_t K, int64_t RT)
+{
+    return (r - r0) * K - RT * (r * (r - 1) - r0 * (r0 - 1)) / 2;
+}
+__host__ __device__ inline int64_t sym_cols(int64_t r, int64_t K, int64_t T)
+{
+    return 64 * K > (r + 1) * T ? 64 * K - (r + 1) * T : 0;
+}
+__host__ __device__ inline int64_t sym_col_first(int64_t r, int64_t r0, int64_t K, int64_t T)
+{
+    return (r - r0) * 64 * K - T * (r * (r + 1) - r0 * (r0 + 1)) / 2;
+}
+
+// the value of a neighbouring lane, the wave taken as a ring
+__device__ inline int ring(int v) { return __builtin_amdgcn_mov_dpp(v, 0x134, 0xf, 0xf, false); }
+__device__ inline double ring(double v)
+{
+    return __hiloint2double(ring(__double2hiint(v)), ring(__double2loint(v)));
+}
+
+// One FP64 source of the lane against its R targets, both directions: c_q = w_j
+// / den_q goes to the targets' sums S, w_q / den_q to the source's A (with the
+// sign of x_j - x_q; the caller turns it).
+template <int R>
+__device__ inline void sym_eval(const double4 *xt, const double4 &s, double (*S)[3], double *A)
+{
+    double d[R][3], den[R], pre[R], c[R];
+#pragma unroll
+    for (int q = 0; q < R; q++) {
+        double dot;
+        {
+#pragma clang fp contract(off)
+            dot = xt[q].x * s.x;
+            dot = dot + xt[q].y * s.y;
+            dot = dot + xt[q].z * s.z;
+        }
+        den[q] = 1.0 - dot;
+        pre[q] = q == 0 ? den[0] : pre[q - 1] * den[q];
+        d[q][0] = s.x - xt[q].x;
+        d[q][1] = s.y - xt[q].y;
+        d[q][2] = s.z - xt[q].z;
+    }
+    if (__builtin_expect(__builtin_amdgcn_ballot_w64(!__builtin_amdgcn_class(pre[R - 1], 0x108)) == 0, 1)) { // normal numbers
+        double r = rcp64d(pre[R - 1]);
+#pragma unroll
+        for (int q = R - 1; q > 0; q--) {
+            c[q] = pre[q - 1] * r;
+            r = den[q] * r;
+        }
+        c[0] = r;
+    } else {
+#pragma unroll
+        for (int q = 0; q < R; q++) c[q] = rcp64d(den[q]);
+    }
+#pragma unroll
+    for (int q = 0; q < R; q++) {
+        const double cs = c[q] * s.w, ct = c[q] * xt[q].w;
+#pragma unroll
+        for (int k = 0; k < 3; k++) {
+            S[q][k] = fma(cs, d[q][k], S[q][k]);
+            A[k] = fma(ct, d[q][k], A[k]);
+        }
+    }
+}
+
+template <int R>
+__global__ void __launch_bounds__(256, R == 4 ? 3 : 4) k_direct_sym(SymArgs a)
+{
+    constexpr int T = 256 * R, RT = 4 * R;
+    __shared__ __align__(16) double2 txy[2][64], tzw[2][64]; // tiles in turn: (x, y), (z, w)
+    __shared__ double red[2][4][3][64];                       // a tile's column sums of the four waves
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
+    stamp_start(a.ts, Timing::START);
+    stamp_start(a.ts, Timing::MAIN);
+    const int64_t b = blockIdx.x;
+    int64_t u = direct_first(b, a.B1, a.q1, a.q);
+    const int64_t u1 = min(u + (b < a.B1 ? a.q1 : a.q), a.U);
+    int64_t row = a.r0;
+    // thread (component, source) of the tile that is fetched
+    auto fetch = [&](int64_t t) {
+        const int64_t j = min(64 * t + lane, a.n - 1);
+        return wave == 0 ? a.x[j] : wave == 1 ? a.y[j] : wave == 2 ? a.z[j] : 64 * t + lane < a.n ? a.vort[j] * a.area[j] : 0.0;
+    };
+    while (u < u1) {
+        while (sym_first(row + 1, a.r0, a.K, RT) <= u) row++;
+        const int64_t t0 = row * RT + u - sym_first(row, a.r0, a.K, RT), t1 = min(a.K, t0 + (u1 - u));
+        double4 xt[R];
+        double S[R][3];
+#pragma unroll
+        for (int q = 0; q < R; q++) {
+            direct_source(a, min(row * T + 64 * (wave * R + q) + lane, a.n - 1), xt[q]);
+            S[q][0] = S[q][1] = S[q][2] = 0.0;
+        }
+        double *col = a.col + 3 * sym_col_first(row, a.r0, a.K, T) - (row + 1) * T;
+        const int64_t len = sym_cols(row, a.K, T);
+        // column sums of tile t, left in red[i] by the four waves
+        auto store = [&](int i, int64_t t) {
+            if (wave < 3) {
+                const double v = ((red[i][0][wave][lane] + red[i][1][wave][lane]) + red[i][2][wave][lane]) + red[i][3][wave][lane];
+                col[wave * len + 64 * t + lane] = -v;
+            }
+        };
+        double nx = fetch(t0);
+        int i = 0;
+        for (int64_t t = t0; t < t1; t++, i ^= 1) {
+            reinterpret_cast<double *>(wave < 2 ? &txy[i][lane] : &tzw[i][lane])[wave & 1] = nx;
+            // one barrier a tile: it ends the stores to this tile's buffer and
+            // the reads of the other one, both of two tiles ago and of the last
+            __syncthreads();
+            if (t > t0 && t - 1 >= (row + 1) * RT) store(i ^ 1, t - 1);
+            if (t + 1 < t1) nx = fetch(t + 1);
+            if (t >= (row + 1) * RT) {
+                double A[3] = {0, 0, 0};
+                int at = lane;
+                double2 p = txy[i][at], zw = tzw[i][at];
+#pragma unroll 2
+                for (int k = 0; k < 64; k++) {
+                    const double4 s = make_double4(p.x, p.y, zw.x, zw.y);
+                    at = ring(at);
+                    p = txy[i][at];
+                    zw = tzw[i][at];
+                    sym_eval<R>(xt, s, S, A);
+#pragma unroll
+                    for (int c = 0; c < 3; c++) A[c] = ring(A[c]);
+                }
+#pragma unroll
+                for (int c = 0; c < 3; c++) red[i][wave][c][lane] = A[c];
+            } else {
+                // a tile of the row itself: its pairs in one direction
+                const int cnt = (int)min((int64_t)64, a.n - 64 * t);
+                int self[R];
+#pragma unroll
+                for (int q = 0; q < R; q++) self[q] = t == row * RT + wave * R + q ? lane : -1;
+                for (int k = 0; k < cnt; k++)
+                    direct_eval<R, true>(xt, make_double4(txy[i][k].x, txy[i][k].y, tzw[i][k].x, tzw[i][k].y), k, self, S);
+            }
+        }
+        __syncthreads();
+        if (t1 - 1 >= (row + 1) * RT) store(i ^ 1, t1 - 1);
+        double *pt = a.part + (b + (row - a.r0)) * 3 * T + wave * 64 * R + lane;
+#pragma unroll
+        for (int q = 0; q < R; q++)
+#pragma unroll
+            for (int c = 0; c < 3; c++) pt[c * T + 64 * q] = S[q][c];
+        u += t1 - t0;
+    }
+}
+
+// adds a slab's column and run sums of every target from its first row on, 16
+// targets x 16 ways per block, ways added in order; the velocities of a
+// target are written by the first slab and raised by the others
+template <int R> __global__ void __launch_bounds__(256) k_sym_sum(SymArgs a)
+{
+    constexpr int T = 256 * R, RT = 4 * R;
+    __shared__ double red[3][16][17];
+    const int tl = threadIdx.x & 15, way = threadIdx.x >> 4;
+    const int64_t at = a.r0 * T + (int64_t)blockIdx.x * 16 + tl, j = min(at, a.n - 1), row = j / T;
+    double s[3] = {0, 0, 0};
+#pragma unroll 4
+    for (int64_t r = a.r0 + way; r < min(row, a.r1); r += 16) {
+        const int64_t len = sym_cols(r, a.K, T);
+        const double *c = a.col + 3 * sym_col_first(r, a.r0, a.K, T) + (j - (r + 1) * T);
+        s[0] += c[0];
+        s[1] += c[len];
+        s[2] += c[2 * len];
+    }
+    if (row < a.r1) {
+        const int64_t b0 = direct_block(sym_first(row, a.r0, a.K, RT), a.B1, a.q1, a.q);
+        const int64_t b1 = direct_block(sym_first(row + 1, a.r0, a.K, RT) - 1, a.B1, a.q1, a.q);
+#pragma unroll 4
+        for (int64_t b = b0 + way; b <= b1; b += 16) {
+            const double *pt = a.part + (b + (row - a.r0)) * 3 * T + (j - row * T);
+            s[0] += pt[0];
+            s[1] += pt[T];
+            s[2] += pt[2 * T];
+        }
+    }
+    for (int c = 0; c < 3; c++) red[c][way][tl] = s[c];
+    __syncthreads();
+    if (way < 3) {
+        double t = 0;
+        for (int h = 0; h < 16; h++) t += red[way][h][tl];
+        red[way][0][tl] = t;
+    }
+    __syncthreads();
+    if (way == 0 && at < a.n) {
+        const double x0 = a.x[j], x1 = a.y[j], x2 = a.z[j];
+        const double s0 = red[0][0][tl], s1 = red[1][0][tl], s2 = red[2][0][tl];
+        double v0 = (x1 * s2 - x2 * s1) * a.scale, v1 = (x2 * s0 - x0 * s2) * a.scale, v2 = (x0 * s1 - x1 * s0) * a.scale;
+        if (a.r0 > 0) {
+            v0 += a.u[j];
+            v1 += a.v[j];
+            v2 += a.w[j];
+        }
+        a.u[j] = v0;
+        a.v[j] = v1;
+        a.w[j] = v2;
+        a.dvort[j] = -2 * a.omega * v2;
+    }
+    stamp_end(a.ts);
+}
+
 struct DirectPlan {
     int R, wt; // targets per lane, sources per wave tile
     bool split;
@@ -413,11 +651,96 @@ static DirectPlan direct_plan(int64_t n, int64_t m, bool mixed)
     return p;
 }
 
-// buf: at least direct_plan().bytes; ts: the call's time stamps or null
+// Workspace of the sum over unordered pairs, within FSS_DIRECT_SCRATCH_BYTES.
+constexpr int64_t SYM_BYTES = (int64_t)30 << 20;
+
+// Targets per lane of the sum over unordered pairs, or 0 where k_direct does
+// the call: chosen targets and mixed precision (whose FP32 partial sums keep
+// their order), few particles, whose units are fewer than the resident blocks,
+// and more than one row's column sums have room for.  Us a call, k_direct
+// against two / four targets a lane: N = 2,562 14.3, 17.3 / 22.1; 3,500 21.7, 18.6 /
+// 23.6; 10,242 75.3, 59.8 / 60.5; 15,000 146.7, 105.9 / 116.7; 20,011 233.4, 197.1 /
+// 186.3; 40,009 824, 705 / 630; 100,003 5,045, 4,361 / 3,902.
+// Outputs that overlap the inputs stay with k_direct, whose last kernel alone
+// writes them.
+static int sym_targets(const fss_particles *p, const fss_velocity *o, const int64_t *idx, bool mixed)
+{
+    const int64_t n = p->n;
+    if (idx || mixed || n < 3300 || n > 500000) return 0;
+    for (const double *in : {p->x, p->y, p->z, p->vort, p->area})
+        for (const double *out : {o->u, o->v, o->w, o->dvort})
+            if (std::less<const double *>()(in, out + n) && std::less<const double *>()(out, in + n)) return 0;
+    return n < 18000 ? 2 : 4;
+}
+
+// The next slab from row a.r0: as many rows as leave room for their column sums
+// beside the run sums of one round of resident blocks.  Its runs: one unit each
+// up to two rounds; beyond that three quarters of the work in one round of long
+// runs and the rest in short ones, as far as there is room for their sums.
+// Returns the doubles that it needs of the workspace.
+static int64_t sym_slab(int64_t n, int R, SymArgs &a, int64_t *blocks)
+{
+    const int64_t T = 256 * R, RT = 4 * R, rows = div_up(n, T), slots = R == 4 ? 768 : 1024;
+    const int64_t room = SYM_BYTES / 24;
+    a.K = div_up(n, 64);
+    a.r1 = a.r0 + 1;
+    while (a.r1 < rows && sym_col_first(a.r1 + 1, a.r0, a.K, T) + (a.r1 + 1 - a.r0 + slots) * T <= room) a.r1++;
+    a.U = sym_first(a.r1, a.r0, a.K, RT);
+    const int64_t cols = sym_col_first(std::min(a.r1, rows - 1), a.r0, a.K, T); // the last row has none
+    const int64_t runs = (room - cols) / T - (a.r1 - a.r0);
+    a.B1 = a.q1 = 0;
+    if (a.U <= std::min(2 * slots, runs)) {
+        a.q = 1;
+    } else if (runs < 2 * slots) {
+        a.q = div_up(a.U, slots);
+    } else {
+        a.B1 = slots;
+        a.q1 = 3 * a.U / (4 * slots);
+        a.q = div_up(a.U - a.B1 * a.q1, std::min<int64_t>(2 * slots, runs - slots));
+    }
+    *blocks = a.B1 + div_up(std::max<int64_t>(0, a.U - a.B1 * a.q1), a.q);
+    a.part = a.col + 3 * cols;
+    return 3 * (cols + (*blocks + a.r1 - a.r0) * T);
+}
+
+static size_t sym_bytes(int64_t n, int R)
+{
+    SymArgs a{};
+    int64_t most = 0, blocks;
+    for (; a.r0 * 256 * R < n; a.r0 = a.r1) most = std::max(most, sym_slab(n, R, a, &blocks));
+    return sizeof(double) * (size_t)most;
+}
+
+template <int R>
+static fss_status launch_sym(fss_ctx *ctx, const fss_particles *p, fss_velocity *out, void *buf, uint64_t *ts)
+{
+    constexpr int64_t T = 256 * R;
+    SymArgs a{};
+    a.x = p->x, a.y = p->y, a.z = p->z, a.vort = p->vort, a.area = p->area;
+    a.n = p->n;
+    a.scale = -1.0 / (4.0 * M_PI);
+    a.omega = ctx->cfg.omega;
+    a.col = static_cast<double *>(buf);
+    a.u = out->u, a.v = out->v, a.w = out->w, a.dvort = out->dvort;
+    for (a.r0 = 0; a.r0 * T < a.n; a.r0 = a.r1) {
+        int64_t blocks;
+        sym_slab(a.n, R, a, &blocks);
+        a.ts = a.r0 == 0 ? ts : nullptr;
+        hipLaunchKernelGGL(k_direct_sym<R>, dim3((unsigned)blocks), dim3(256), 0, ctx->stream, a);
+        a.ts = ts;
+        hipLaunchKernelGGL(k_sym_sum<R>, dim3((unsigned)div_up(a.n - a.r0 * T, 16)), dim3(256), 0, ctx->stream, a);
+    }
+    FSS_HIP(hipGetLastError());
+    return FSS_OK;
+}
+
+// buf: at least sym_bytes() or direct_plan().bytes; ts: the call's time stamps or null
 static fss_status launch_direct(fss_ctx *ctx, const fss_particles *p, const int64_t *idx, int64_t m,
                                 fss_velocity *out, bool mixed, void *buf, uint64_t *ts)
 {
     hipStream_t s = ctx->stream;
+    if (const int R = sym_targets(p, out, idx, mixed))
+        return R == 2 ? launch_sym<2>(ctx, p, out, buf, ts) : launch_sym<4>(ctx, p, out, buf, ts);
     const DirectPlan P = direct_plan(p->n, m, mixed);
     DirectArgs a{p->x, p->y, p->z, p->vort, p->area, nullptr, idx, p->n, m, P.K, P.U, P.B1, P.q1, P.q, -1.0 / (4.0 * M_PI),
                  ctx->cfg.omega, static_cast<double *>(buf), out->u, out->v, out->w, out->dvort, ts};
@@ -459,7 +782,8 @@ fss_status velocity_direct(fss_ctx *ctx, const fss_particles *p, const int64_t *
     if (!idx) m = n;
     const bool mixed = !force_fp64 && ctx->cfg.precision == FSS_MIXED;
     DevBuf &buf = ctx->direct;
-    FSS_TRY(buf.ensure(direct_plan(n, m, mixed).bytes));
+    const int R = sym_targets(p, out, idx, mixed);
+    FSS_TRY(buf.ensure(R ? sym_bytes(n, R) : direct_plan(n, m, mixed).bytes));
     if (ctx->capturing) return launch_direct(ctx, p, idx, m, out, mixed, buf.p, nullptr);
     Timing &t = ctx->timing;
     timing_begin(t, ctx->stream);
