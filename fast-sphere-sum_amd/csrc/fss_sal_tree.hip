@@ -54,25 +54,56 @@ template <int KIND> __device__ inline double gfun(const KernelArgs &k, const dou
     return legendre_sum(k.c, k.N, 1.0 - 2.0 * s * s);
 }
 
-// near field: one wave per near item, one lane per (target, phase); the
+// the staged sources ph, ph + P, ... below m against the R targets of a lane
+template <int KIND, int R>
+__device__ inline void sal_chunk(const KernelArgs &ka, const double4 *xt, const double4 *lds, int ph, int P, int m,
+                                 double *acc)
+{
+    for (int k = ph; k < m; k += P) {
+        const double4 s = lds[k];
+#pragma unroll
+        for (int q = 0; q < R; q++) acc[q] = fma(gfun<KIND>(ka, xt[q], s), s.w, acc[q]);
+    }
+}
+
+// Targets (proxies) per lane.  The table lookups bound these kernels: every lane
+// reads its own two lines from L1, one lookup a cycle and CU (level-8 grid, degree
+// 3: 2.26 lookups a near pair, 1.02 a cycle), so several targets a lane help by
+// what they put in flight and by the lanes that one target a lane leaves idle (33 to
+// 64 targets: the lanes beyond them; level-8 grid, near field with 1 / 2 / 3 / 4 / 5 /
+// 6 targets a lane: call of 4.35 / 3.88 / 4.35 / 3.63 / 3.95 / 4.84 ms).  Proxies: all of a
+// node's up to degree 3, a third beyond (call at degree 3 with 1 / 2 / 5 / 10: 3.63 / 3.51 /
+// 3.38 / 3.27 ms; degree 4 with 1 / 3 / 5 / 8: 5.96 / 6.33 / 5.73 / 5.82; degree 5 with 1 / 3 / 6 /
+// 7: 9.97 / 10.63 / 12.61 / 9.63).  Contiguous runs of items per XCD are slower (6.1
+// against 4.3 ms), and so are two lanes sharing each window of the table (half the
+// loads' lines, but the exchange costs more: 4.0 ms).
+constexpr int SAL_NEAR_R = 4;
+constexpr int sal_proxy_r(int pp) { return pp <= 10 ? pp : pp / 3; }
+
+// near field: one wave per near item, R targets per lane and phase; the
 // item's source list (the self ranges too: j = i is part of the sum) staged in
 // LDS chunks, every chunk's loads independent
-template <int KIND>
+template <int KIND, int R>
 __global__ void __launch_bounds__(64) k_sal_near(const NearItem *__restrict__ items,
                                                  const int32_t *__restrict__ near_src,
                                                  const double4 *__restrict__ src, KernelArgs ka, double *out)
 {
     stamp_start(ka.ts_near, Timing::MAIN);
     __shared__ double4 lds[NCH_S];
-    __shared__ double red[64];
+    __shared__ double red[64 * R];
     const NearItem it = items[blockIdx.x];
     const int lane = threadIdx.x;
     const int cnt = it.tgt_cnt;
-    const int P = 64 / cnt;
-    const int ph = lane / cnt, tl = lane - ph * cnt;
+    const int T = (cnt + R - 1) / R, P = 64 / T;
+    const int ph = lane / T, tl = lane - ph * T;
     const bool act = ph < P;
-    const double4 xt = src[it.tgt_start + (act ? tl : 0)];
-    double acc = 0.0;
+    double4 xt[R];
+    double acc[R] = {};
+#pragma unroll
+    for (int q = 0; q < R; q++) {
+        // a missing target repeats the lane's first: the same table cells
+        xt[q] = src[it.tgt_start + (act ? (tl + q * T < cnt ? tl + q * T : tl) : 0)];
+    }
     const int32_t *list = near_src + it.src_off;
     const int total = it.n_other + it.n_self;
     for (int base = 0; base < total; base += NCH_S) {
@@ -81,25 +112,23 @@ __global__ void __launch_bounds__(64) k_sal_near(const NearItem *__restrict__ it
         for (int s = 0; s < NCH_S / 64; s++)
             if (lane + 64 * s < m) lds[lane + 64 * s] = src[list[base + lane + 64 * s]];
         __syncthreads();
-        if (act)
-            for (int k = ph; k < m; k += P) {
-                const double4 s = lds[k];
-                acc = fma(gfun<KIND>(ka, xt, s), s.w, acc);
-            }
+        if (act) sal_chunk<KIND, R>(ka, xt, lds, ph, P, m, acc);
         __syncthreads();
     }
-    red[lane] = acc;
+#pragma unroll
+    for (int q = 0; q < R; q++) red[64 * q + lane] = acc[q];
     __syncthreads();
-    if (ph == 0 && act) {
+    if (lane < cnt) {
+        const int q = lane / T, g = lane - q * T;
         double a = 0.0;
-        for (int h = 0; h < P; h++) a += red[h * cnt + tl];
-        out[it.out_base + tl] = a;
+        for (int h = 0; h < P; h++) a += red[64 * q + h * T + g];
+        out[it.out_base + lane] = a;
     }
 }
 
-// proxy values: one wave per proxy item, one lane per (proxy, phase); the
-// item's source list staged in LDS chunks as in k_sal_near
-template <int KIND, int D>
+// proxy values: one wave per proxy item, R proxies per lane, phases as in
+// k_sal_near; the item's source list staged in LDS chunks
+template <int KIND, int D, int R>
 __global__ void __launch_bounds__(64) k_sal_proxy(const ProxyItem *__restrict__ items,
                                                   const int64_t *__restrict__ far_off,
                                                   const int32_t *__restrict__ far_src,
@@ -108,16 +137,20 @@ __global__ void __launch_bounds__(64) k_sal_proxy(const ProxyItem *__restrict__ 
 {
     stamp_start(ka.ts_proxy, Timing::MAIN);
     constexpr int PP = npts_s<D>();
-    constexpr int P = 64 / PP;
+    constexpr int T = (PP + R - 1) / R, P = 64 / T;
     __shared__ double4 lds[NCH_S];
-    __shared__ double red[64];
+    __shared__ double red[64 * R];
     const int64_t item = blockIdx.x;
     const ProxyItem it = items[item];
     const int lane = threadIdx.x;
-    const int ph = lane / PP, k = lane - ph * PP;
+    const int ph = lane / T, tl = lane - ph * T;
     const bool act = ph < P;
-    const double4 yk = src[p0 + (int64_t)it.node * PP + (act ? k : 0)];
-    double acc = 0.0;
+    double4 yk[R];
+    double acc[R] = {};
+#pragma unroll
+    for (int q = 0; q < R; q++) {
+        yk[q] = src[p0 + (int64_t)it.node * PP + (act ? (tl + q * T < PP ? tl + q * T : tl) : 0)];
+    }
     const int64_t o0 = far_off[item];
     const int total = (int)(far_off[item + 1] - o0);
     const int32_t *list = far_src + o0;
@@ -127,19 +160,17 @@ __global__ void __launch_bounds__(64) k_sal_proxy(const ProxyItem *__restrict__ 
         for (int s = 0; s < NCH_S / 64; s++)
             if (lane + 64 * s < m) lds[lane + 64 * s] = src[list[base + lane + 64 * s]];
         __syncthreads();
-        if (act)
-            for (int kk = ph; kk < m; kk += P) {
-                const double4 s = lds[kk];
-                acc = fma(gfun<KIND>(ka, yk, s), s.w, acc);
-            }
+        if (act) sal_chunk<KIND, R>(ka, yk, lds, ph, P, m, acc);
         __syncthreads();
     }
-    red[lane] = acc;
+#pragma unroll
+    for (int q = 0; q < R; q++) red[64 * q + lane] = acc[q];
     __syncthreads();
-    if (ph == 0 && act) {
+    if (lane < PP) {
+        const int q = lane / T, g = lane - q * T;
         double a = 0.0;
-        for (int h = 0; h < P; h++) a += red[h * PP + k];
-        phi[item * PP + k] = a;
+        for (int h = 0; h < P; h++) a += red[64 * q + h * T + g];
+        phi[item * PP + lane] = a;
     }
 }
 
@@ -425,11 +456,12 @@ template <int KIND, int D> fss_status run(fss_ctx *ctx, const KernelArgs &ka, do
                                T.proxy_items.as<ProxyItem>(), T.n_proxy, T.far_off.as<int64_t>(),
                                T.far_src.as<int32_t>(), src, p0, ka, ctx->phi.as<double>());
     } else {
+        constexpr int RF = sal_proxy_r(npts_s<D>());
         if (T.n_near > 0)
-            hipLaunchKernelGGL((k_sal_near<KIND>), dim3((unsigned)T.n_near), dim3(64), 0, s,
+            hipLaunchKernelGGL((k_sal_near<KIND, SAL_NEAR_R>), dim3((unsigned)T.n_near), dim3(64), 0, s,
                                T.near_items.as<NearItem>(), T.near_src.as<int32_t>(), src, ka, ctx->out3.as<double>());
         if (T.n_proxy > 0)
-            hipLaunchKernelGGL((k_sal_proxy<KIND, D>), dim3((unsigned)T.n_proxy), dim3(64), 0, s,
+            hipLaunchKernelGGL((k_sal_proxy<KIND, D, RF>), dim3((unsigned)T.n_proxy), dim3(64), 0, s,
                                T.proxy_items.as<ProxyItem>(), T.far_off.as<int64_t>(), T.far_src.as<int32_t>(), src,
                                p0, ka, ctx->phi.as<double>());
     }

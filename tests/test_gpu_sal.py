@@ -327,3 +327,34 @@ def test_learned_treecode_converges_to_learned_direct(fsslib, sal):
         errs.append(np.linalg.norm(got - ref) / np.linalg.norm(ref))
     print("learned treecode rel-L2 vs learned direct, degree 2/4:", errs)
     assert errs[1] < 0.5 * errs[0] and errs[1] < 1e-3
+
+
+@pytest.mark.parametrize("n,levels", [(5, 1), (30, 2), (257, 2), (1280, 1), (3001, 3)])
+def test_sal_treecode_near_layouts(fsslib, sal, n, levels):
+    """Without far interactions (theta -> 0) the treecode is the direct sum in
+    another order, for every number of targets per item from 1 to 64.  The table is
+    read at distances that differ by an ulp or two: 1e4 radians per unit of s give
+    1e-12 of the largest value, about 50 times a target's sum."""
+    ctx, c, A, torch = sal
+    x, y, z = fsslib.grid_random(n, 3)
+    d = [torch.from_numpy(a).cuda() for a in (x, y, z, np.random.default_rng(n).normal(size=n), np.full(n, 4 * np.pi / n))]
+    t = fsslib.Context(tree_levels=levels, theta=1e-6, degree=2, eval_mode=1, assign_mode=1, node_rule=1, many_count=1)
+    t.sal_set_series(c, table_points=1 << 22, A=A)
+    t.tree_build(*d[:3])
+    print(f"sal near n={n} levels={levels}", flush=True)
+    got, ref = t.sal_tree(*d, kind=0).cpu().numpy(), ctx.sal_direct(*d, kind=0).cpu().numpy()
+    assert np.linalg.norm(got - ref) <= 1e-10 * np.linalg.norm(ref)
+
+
+@pytest.mark.parametrize("degree,bar", [(1, 0.1), (2, 1e-2), (3, 1e-2), (5, 1e-2)])
+def test_sal_treecode_proxy_layouts(fsslib, sal, degree, bar):
+    """Each degree's split of the proxies over the lanes: a proxy left out or taken
+    twice is an error of order one, the interpolation error of this kernel 3e-3 at
+    degree 2 and more at degree 1."""
+    _, _, A, torch = sal
+    ctx, d, _ = _sal_tree_case(fsslib, torch, _cesaro(fsslib), A, degree, 0.5)
+    print(f"sal proxies degree={degree}", flush=True)
+    ref = ctx.sal_direct(*d, kind=0).cpu().numpy()
+    for kind in (0, 2):
+        got = ctx.sal_tree(*d, kind=kind).cpu().numpy()
+        assert np.linalg.norm(got - ref) <= bar * np.linalg.norm(ref)
