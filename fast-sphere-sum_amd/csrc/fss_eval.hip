@@ -118,12 +118,9 @@ __device__ inline float4 to_frame(const float4 &s, int32_t rn, const double *__r
                        (float)((c[2] - ct[2]) + (double)s.z), s.w);
 }
 
-// record node of source position j: its own for particle records, the
-// owning node for proxies (p0 + node * p)
-__device__ inline int32_t src_node(int64_t j, int64_t p0, int p, const int32_t *__restrict__ recnode)
-{
-    return j < p0 ? recnode[j] : (int32_t)((j - p0) / p);
-}
+// node of source position j, whose centre its FP32 record is relative to
+__device__ inline int32_t node_of(const int32_t *__restrict__, int32_t, const double4 *) { return 0; }
+__device__ inline int32_t node_of(const int32_t *__restrict__ srcnode, int32_t j, const float4 *) { return srcnode[j]; }
 
 // monomials s^(i-j) t^j, index i(i+1)/2 + j (interp_utils.h:49-59)
 template <int D> __device__ inline void monomials(double s, double t, double *m)
@@ -192,13 +189,21 @@ __global__ void k_proxy_records64(const double4 *__restrict__ proxy, int64_t npr
     src[i] = make_double4(q.x, q.y, q.z, 0.0);
 }
 
+// srcnode: the node of every source position, records first: read with the
+// position's record by the kernels that move it to another node's frame.  (Worked
+// out there, p0 and a division told the two kinds apart: branches and a tenth
+// of the near kernel's instructions.)
 __global__ void k_proxy_records32(const double4 *__restrict__ proxy, int64_t nprox, int p,
-                                  const double *__restrict__ centres, int planar, float4 *src, float *aoff)
+                                  const double *__restrict__ centres, int planar, float4 *src, float *aoff,
+                                  const int32_t *__restrict__ recnode, int64_t p0, int32_t *srcnode)
 {
     int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    if (i < p0) srcnode[i] = recnode[i];
     if (i >= nprox) return;
     double4 q = proxy[i];
-    const double *c = centres + 4 * (i / p);
+    const int32_t g = (int32_t)((uint32_t)i / (uint32_t)p);
+    const double *c = centres + 4 * (int64_t)g;
+    srcnode[p0 + i] = g;
     src[i] = make_float4((float)(q.x - c[0]), (float)(q.y - c[1]), (float)(q.z - c[2]), 0.0f);
     // For a particle x on the sphere, 2 (1 - y.x) = |x - y|^2 + (1 - |y|^2).
     // Planar proxies (PARITY) are off the sphere and carry that offset.
@@ -226,10 +231,12 @@ fss_status proxy_records(fss_ctx *ctx)
     if (ctx->cfg.precision != FSS_MIXED) return proxy_records64(ctx);
     const int64_t nprox = T.nn * ctx->interp.p, nsrc = T.p0 + nprox;
     FSS_TRY(T.src32.ensure(sizeof(float4) * nsrc + sizeof(float) * nprox));
+    FSS_TRY(T.srcnode.ensure(sizeof(int32_t) * nsrc));
     float4 *src = T.src32.as<float4>();
-    hipLaunchKernelGGL(k_proxy_records32, dim3((unsigned)div_up(nprox, 256)), dim3(256), 0, ctx->stream,
+    hipLaunchKernelGGL(k_proxy_records32, dim3((unsigned)div_up(std::max(nprox, T.p0), 256)), dim3(256), 0, ctx->stream,
                        T.proxy_xyz.as<double4>(), nprox, ctx->interp.p, T.d_info,
-                       ctx->cfg.eval_mode == FSS_EVAL_BLTC ? 0 : 1, src + T.p0, reinterpret_cast<float *>(src + nsrc));
+                       ctx->cfg.eval_mode == FSS_EVAL_BLTC ? 0 : 1, src + T.p0, reinterpret_cast<float *>(src + nsrc),
+                       T.recnode.as<int32_t>(), T.p0, T.srcnode.as<int32_t>());
     FSS_HIP(hipGetLastError());
     return FSS_OK;
 }
@@ -672,7 +679,7 @@ __global__ void __launch_bounds__(64, sizeof(Real) == 4 && R == 2 ? 8 : 4) k_nea
                                              const int32_t *__restrict__ near_src,
                                              const typename Rec<Real>::T4 *__restrict__ src,
                                              const int32_t *__restrict__ recid,
-                                             const int32_t *__restrict__ recnode, int64_t p0, int p,
+                                             const int32_t *__restrict__ srcnode, int32_t p0,
                                              const double *__restrict__ centres,
                                              const double *__restrict__ x,
                                              const double *__restrict__ y,
@@ -710,7 +717,7 @@ __global__ void __launch_bounds__(64, sizeof(Real) == 4 && R == 2 ? 8 : 4) k_nea
         int t = tl + q * T;
         int tt = (act && t < cnt) ? t : 0;
         int64_t j = (int64_t)it.tgt_start + tt;
-        xt[q] = to_frame(src[j], recnode[j], centres, ct);
+        xt[q] = to_frame(src[j], node_of(srcnode, (int32_t)j, src), centres, ct);
         tid[q] = rec_id(recid, j);
     }
     Acc<Real, R> A;
@@ -747,9 +754,8 @@ __global__ void __launch_bounds__(64, sizeof(Real) == 4 && R == 2 ? 8 : 4) k_nea
             for (int s = 0; s < S / 2; s++) {
                 const int32_t j = jj[h + s];
                 rec[s] = src[j];
-                const int32_t rn = recnode[min((int64_t)j, p0 - 1)];
-                nd[s] = j < p0 ? rn : (int32_t)((uint32_t)(j - p0) / (uint32_t)p);
-                id[s] = self_part ? rec_id(recid, min((int64_t)j, p0 - 1)) : 0;
+                nd[s] = node_of(srcnode, j, src);
+                id[s] = self_part ? rec_id(recid, min(j, p0 - 1)) : 0;
             }
 #pragma unroll
             for (int s = 0; s < S / 2; s++) rec[s] = to_frame(rec[s], nd[s], centres, ct);
@@ -970,7 +976,7 @@ __global__ void __launch_bounds__(256) k_proxy_list(const ProxyItem *__restrict_
         for (int s = 0; s < S; s++)
             if (jn[s] >= 0) {
                 rn[s] = src[jn[s]];
-                nn[s] = src_node(jn[s], p0, PP, recnode);
+                nn[s] = jn[s] < (int32_t)p0 ? recnode[jn[s]] : (int32_t)((uint32_t)(jn[s] - (int32_t)p0) / (uint32_t)PP);
             }
     };
     load_list(0, jn);
@@ -1282,7 +1288,7 @@ static fss_status run_degree(fss_ctx *ctx, const fss_particles *pp, fss_velocity
             auto kn = bltc ? (ctx->near_r == 2 ? k_near<double, 2, true> : k_near<double, 4, true>)
                            : (ctx->near_r == 2 ? k_near<double, 2, false> : k_near<double, 4, false>);
             hipLaunchKernelGGL(kn, dim3((unsigned)T.n_near), dim3(64), 0, s, T.near_items.as<NearItem>(),
-                               T.near_src.as<int32_t>(), src, recid, T.recnode.as<int32_t>(), p0, p,
+                               T.near_src.as<int32_t>(), src, recid, T.srcnode.as<int32_t>(), (int32_t)p0,
                                T.d_info, pp->x, pp->y, pp->z, ost, ctx->out3.as<double>(), ts);
         }
         } else {
@@ -1301,7 +1307,7 @@ static fss_status run_degree(fss_ctx *ctx, const fss_particles *pp, fss_velocity
             if (T.n_near > 0) {
             auto kn = ctx->near_r == 4 ? k_near<float, 4, false> : k_near<float, 2, false>; // default 2
             hipLaunchKernelGGL(kn, dim3((unsigned)T.n_near), dim3(64), 0, s, T.near_items.as<NearItem>(),
-                               T.near_src.as<int32_t>(), src, recid, T.recnode.as<int32_t>(), p0, p,
+                               T.near_src.as<int32_t>(), src, recid, T.srcnode.as<int32_t>(), (int32_t)p0,
                                T.d_info, pp->x, pp->y, pp->z, ost, ctx->out3.as<double>(), ts);
         }
         }

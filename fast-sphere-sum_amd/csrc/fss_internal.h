@@ -212,6 +212,7 @@ struct Tree {
     DevBuf proxy_xyz;   // double4 [nn * p] static proxy positions (w unused)
     DevBuf src64;       // double4 [p0 + nn * p] source records (see above)
     DevBuf src32;       // float4 [p0 + nn * p], then float [nn * p] planar offsets
+    DevBuf srcnode;     // int32 [p0 + nn * p] node of every source position (mixed precision)
     int64_t pairs_near = 0, pairs_far = 0;
 };
 
