@@ -1274,21 +1274,47 @@ __global__ void __launch_bounds__(64) k_near_src_count(NearItem *items, const Ra
     }
 }
 
+// Writes the record positions of the ranges [beg, end) that `take` accepts (it
+// is given a range's count) to dst, one wave together; returns the end of the
+// list.  The lanes load 64 ranges at once and sum their counts; sixteen lanes
+// then write a range, four ranges at a time (ranges hold a leaf, or up to 45
+// proxies).  Range by range, every turn waited for its own load and wrote with ten
+// lanes: 200,003 particles, theta 0.6: near lists 61 us, far lists 31; now 29 and
+// 14 (level-10 grid, degree 7: 739 and 235, now 420 and 168).
+template <typename Take>
+__device__ inline int32_t *list_ranges(const Range *__restrict__ ranges, int beg, int end, int32_t *dst, Take take)
+{
+    const int lane = threadIdx.x & 63;
+    for (int b = beg; b < end; b += 64) {
+        int32_t start = 0, count = 0;
+        if (b + lane < end) {
+            const Range r = ranges[b + lane];
+            start = r.start;
+            count = take(r.count) ? r.count & ~FSS_SELF_BIT : 0;
+        }
+        int32_t sum = count;
+        for (int o = 1; o < 64; o <<= 1) {
+            const int32_t t = __shfl_up(sum, o, 64);
+            sum += lane >= o ? t : 0;
+        }
+        for (int l0 = 0; l0 < min(64, end - b); l0 += 4) {
+            const int l = l0 + (lane >> 4);
+            const int32_t s = __shfl(start, l, 64), c = __shfl(count, l, 64), o = __shfl(sum, l, 64) - c;
+            for (int i = lane & 15; i < c; i += 16) dst[o + i] = s + i;
+        }
+        dst += __shfl(sum, 63, 64);
+    }
+    return dst;
+}
+
 __global__ void __launch_bounds__(64) k_near_src_fill(NearItem *items, const Range *__restrict__ ranges,
                                                       const int64_t *__restrict__ off, int32_t *near_src)
 {
-    const int lane = threadIdx.x;
     const NearItem it = items[blockIdx.x];
-    int64_t o = off[blockIdx.x];
-    if (lane == 0) items[blockIdx.x].src_off = o;
-    for (int pass = 0; pass < 2; pass++)
-        for (int r = it.a_beg; r < it.a_end; r++) {
-            const Range rg = ranges[r];
-            if (((rg.count & FSS_SELF_BIT) != 0) != (pass == 1)) continue;
-            const int c = rg.count & ~FSS_SELF_BIT;
-            for (int i = lane; i < c; i += 64) near_src[o + i] = rg.start + i;
-            o += c;
-        }
+    const int64_t o = off[blockIdx.x];
+    if (threadIdx.x == 0) items[blockIdx.x].src_off = o;
+    int32_t *dst = list_ranges(ranges, it.a_beg, it.a_end, near_src + o, [](int32_t c) { return !(c & FSS_SELF_BIT); });
+    list_ranges(ranges, it.a_beg, it.a_end, dst, [](int32_t c) { return (c & FSS_SELF_BIT) != 0; });
 }
 
 // The near kernel hands each XCD a contiguous eighth of the items; inside every
@@ -1297,32 +1323,29 @@ __global__ void __launch_bounds__(64) k_near_src_fill(NearItem *items, const Ran
 // hold short items.  Cost of an item: its sources over the phases of a 4-target
 // tile.  One block ranks a window (equal costs keep their order).
 constexpr int NEAR_WINDOW = 512;
-__global__ void __launch_bounds__(256) k_near_order(NearItem *items, int64_t n, int wpe)
+__global__ void __launch_bounds__(NEAR_WINDOW) k_near_order(NearItem *items, int64_t n, int wpe)
 {
-    __shared__ int64_t cost[NEAR_WINDOW];
+    // cost, then place (earlier first): distinct keys, 0 beyond the window's end.
+    // Whole unrolled rounds, so that their LDS reads are in flight together
+    // (32 us with a read per turn of a loop of c turns).
+    __shared__ __align__(16) uint64_t key[NEAR_WINDOW];
     const int64_t q8 = n >> 3, r8 = n & 7;
     const int64_t xcd = blockIdx.x / wpe, win = blockIdx.x % wpe;
     const int64_t b = xcd * q8 + min(xcd, r8) + win * NEAR_WINDOW, e = (xcd + 1) * q8 + min(xcd + 1, r8);
-    const int c = (int)max((int64_t)0, min((int64_t)NEAR_WINDOW, e - b));
-    NearItem it[NEAR_WINDOW / 256];
-#pragma unroll
-    for (int k = 0; k < NEAR_WINDOW / 256; k++) {
-        const int i = threadIdx.x + 256 * k;
-        if (i >= c) continue;
-        it[k] = items[b + i];
-        const int tt = (it[k].tgt_cnt + 3) / 4, ph = 64 / tt;
-        cost[i] = ((int64_t)it[k].n_other + it[k].n_self + ph - 1) / ph;
+    const int c = (int)max((int64_t)0, min((int64_t)NEAR_WINDOW, e - b)), i = threadIdx.x;
+    NearItem it{};
+    uint64_t mine = 0;
+    if (i < c) {
+        it = items[b + i];
+        const int tt = (it.tgt_cnt + 3) / 4, ph = 64 / tt;
+        mine = (uint64_t)(((int64_t)it.n_other + it.n_self + ph - 1) / ph) * NEAR_WINDOW + (NEAR_WINDOW - 1 - i);
     }
+    key[i] = mine;
     __syncthreads();
-#pragma unroll
-    for (int k = 0; k < NEAR_WINDOW / 256; k++) {
-        const int i = threadIdx.x + 256 * k;
-        if (i >= c) continue;
-        const int64_t mine = cost[i];
-        int rank = 0;
-        for (int j = 0; j < c; j++) rank += cost[j] > mine || (cost[j] == mine && j < i) ? 1 : 0;
-        items[b + rank] = it[k];
-    }
+    int rank = 0;
+#pragma unroll 16
+    for (int j = 0; j < NEAR_WINDOW; j++) rank += key[j] > mine ? 1 : 0;
+    if (i < c) items[b + rank] = it;
 }
 
 // Source list of every proxy item: the records of its class-B ranges in order.
@@ -1344,16 +1367,9 @@ __global__ void __launch_bounds__(64) k_far_src_fill(const ProxyItem *__restrict
                                                      const Range *__restrict__ ranges,
                                                      const int64_t *__restrict__ off, int32_t *far_src)
 {
-    const int lane = threadIdx.x;
     if (nitems && (int)blockIdx.x >= *nitems) return;
     const ProxyItem it = items[blockIdx.x];
-    int64_t o = off[blockIdx.x];
-    for (int r = it.b_beg; r < it.b_end; r++) {
-        const Range rg = ranges[r];
-        const int c = rg.count & ~FSS_SELF_BIT;
-        for (int i = lane; i < c; i += 64) far_src[o + i] = rg.start + i;
-        o += c;
-    }
+    list_ranges(ranges, it.b_beg, it.b_end, far_src + off[blockIdx.x], [](int32_t) { return true; });
 }
 
 // Upward items: each charge node's records (main range, then exception range)
@@ -1428,7 +1444,7 @@ fss_status plan_finish(fss_ctx *ctx)
         hipLaunchKernelGGL(k_near_src_fill, dim3((unsigned)T.n_near), dim3(64), 0, s, T.near_items.as<NearItem>(),
                            T.ranges_a.as<Range>(), B.off.as<int64_t>(), T.near_src.as<int32_t>());
         const int wpe = (int)div_up((T.n_near >> 3) + 1, NEAR_WINDOW);
-        hipLaunchKernelGGL(k_near_order, dim3((unsigned)(8 * wpe)), dim3(256), 0, s, T.near_items.as<NearItem>(),
+        hipLaunchKernelGGL(k_near_order, dim3((unsigned)(8 * wpe)), dim3(NEAR_WINDOW), 0, s, T.near_items.as<NearItem>(),
                            T.n_near, wpe);
         FSS_HIP(hipGetLastError());
     }
