@@ -38,6 +38,7 @@
 #include <mutex>
 
 #include "fss_internal.h"
+#include "fss_rk4_dev.h"
 
 namespace fss {
 
@@ -317,7 +318,7 @@ __global__ void __launch_bounds__(256, 4) k_direct(DirectArgs a)
 // one thread per target would walk them alone), ways added in order
 __global__ void __launch_bounds__(256) k_direct_sum(const double *__restrict__ part, int64_t m, int nt, int64_t K,
                                                     int64_t B1, int64_t q1, int64_t q, double omega, double *u, double *v, double *w,
-                                                    double *dvort, uint64_t *ts)
+                                                    double *dvort, RkNext next, uint64_t *ts)
 {
     __shared__ double red[3][16][17];
     const int tl = threadIdx.x & 15, way = threadIdx.x >> 4;
@@ -340,10 +341,14 @@ __global__ void __launch_bounds__(256) k_direct_sum(const double *__restrict__ p
     }
     __syncthreads();
     if (way == 0 && (int64_t)blockIdx.x * 16 + tl < m) {
-        u[r] = red[0][0][tl];
-        v[r] = red[1][0][tl];
-        w[r] = red[2][0][tl];
-        dvort[r] = -2 * omega * red[2][0][tl];
+        const double a0 = red[0][0][tl], a1 = red[1][0][tl], a2 = red[2][0][tl], a3 = -2 * omega * a2;
+        if (next.mode != RkNext::STEP) {
+            u[r] = a0;
+            v[r] = a1;
+            w[r] = a2;
+            dvort[r] = a3;
+        }
+        rk_next(next, r, a0, a1, a2, a3);
     }
     stamp_end(ts);
 }
@@ -530,7 +535,7 @@ __global__ void __launch_bounds__(256, R == 4 ? 3 : 4) k_direct_sym(SymArgs a)
 // adds a slab's column and run sums of every target from its first row on, 16
 // targets x 16 ways per block, ways added in order; the velocities of a
 // target are written by the first slab and raised by the others
-template <int R> __global__ void __launch_bounds__(256) k_sym_sum(SymArgs a)
+template <int R> __global__ void __launch_bounds__(256) k_sym_sum(SymArgs a, RkNext next)
 {
     constexpr int T = 256 * R, RT = 4 * R;
     __shared__ double red[3][16][17];
@@ -573,10 +578,17 @@ template <int R> __global__ void __launch_bounds__(256) k_sym_sum(SymArgs a)
             v1 += a.v[j];
             v2 += a.w[j];
         }
-        a.u[j] = v0;
-        a.v[j] = v1;
-        a.w[j] = v2;
-        a.dvort[j] = -2 * a.omega * v2;
+        const double v3 = -2 * a.omega * v2;
+        // a target is done with its own row's slab, and later slabs read neither
+        // it nor its state
+        const bool done = row < a.r1;
+        if (!done || next.mode != RkNext::STEP) {
+            a.u[j] = v0;
+            a.v[j] = v1;
+            a.w[j] = v2;
+            a.dvort[j] = v3;
+        }
+        if (done) rk_next(next, j, v0, v1, v2, v3);
     }
     stamp_end(a.ts);
 }
@@ -712,7 +724,8 @@ static size_t sym_bytes(int64_t n, int R)
 }
 
 template <int R>
-static fss_status launch_sym(fss_ctx *ctx, const fss_particles *p, fss_velocity *out, void *buf, uint64_t *ts)
+static fss_status launch_sym(fss_ctx *ctx, const fss_particles *p, fss_velocity *out, void *buf, const RkNext &next,
+                             uint64_t *ts)
 {
     constexpr int64_t T = 256 * R;
     SymArgs a{};
@@ -728,7 +741,7 @@ static fss_status launch_sym(fss_ctx *ctx, const fss_particles *p, fss_velocity 
         a.ts = a.r0 == 0 ? ts : nullptr;
         hipLaunchKernelGGL(k_direct_sym<R>, dim3((unsigned)blocks), dim3(256), 0, ctx->stream, a);
         a.ts = ts;
-        hipLaunchKernelGGL(k_sym_sum<R>, dim3((unsigned)div_up(a.n - a.r0 * T, 16)), dim3(256), 0, ctx->stream, a);
+        hipLaunchKernelGGL(k_sym_sum<R>, dim3((unsigned)div_up(a.n - a.r0 * T, 16)), dim3(256), 0, ctx->stream, a, next);
     }
     FSS_HIP(hipGetLastError());
     return FSS_OK;
@@ -736,11 +749,11 @@ static fss_status launch_sym(fss_ctx *ctx, const fss_particles *p, fss_velocity 
 
 // buf: at least sym_bytes() or direct_plan().bytes; ts: the call's time stamps or null
 static fss_status launch_direct(fss_ctx *ctx, const fss_particles *p, const int64_t *idx, int64_t m,
-                                fss_velocity *out, bool mixed, void *buf, uint64_t *ts)
+                                fss_velocity *out, bool mixed, void *buf, const RkNext &next, uint64_t *ts)
 {
     hipStream_t s = ctx->stream;
     if (const int R = sym_targets(p, out, idx, mixed))
-        return R == 2 ? launch_sym<2>(ctx, p, out, buf, ts) : launch_sym<4>(ctx, p, out, buf, ts);
+        return R == 2 ? launch_sym<2>(ctx, p, out, buf, next, ts) : launch_sym<4>(ctx, p, out, buf, next, ts);
     const DirectPlan P = direct_plan(p->n, m, mixed);
     DirectArgs a{p->x, p->y, p->z, p->vort, p->area, nullptr, idx, p->n, m, P.K, P.U, P.B1, P.q1, P.q, -1.0 / (4.0 * M_PI),
                  ctx->cfg.omega, static_cast<double *>(buf), out->u, out->v, out->w, out->dvort, ts};
@@ -766,13 +779,15 @@ static fss_status launch_direct(fss_ctx *ctx, const fss_particles *p, const int6
     hipLaunchKernelGGL(k, dim3((unsigned)P.B), dim3(256), 0, s, a);
     if (P.split)
         hipLaunchKernelGGL(k_direct_sum, dim3((unsigned)div_up(m, 16)), dim3(256), 0, s, a.part, m, 64 * P.R, P.K, P.B1, P.q1,
-                           P.q, a.omega, out->u, out->v, out->w, out->dvort, ts);
+                           P.q, a.omega, out->u, out->v, out->w, out->dvort, next, ts);
+    else if (next.mode != RkNext::NONE)
+        FSS_TRY(rk4_next(ctx, next, *out)); // these kernels write every velocity where it is summed
     FSS_HIP(hipGetLastError());
     return FSS_OK;
 }
 
 fss_status velocity_direct(fss_ctx *ctx, const fss_particles *p, const int64_t *idx, int64_t m,
-                           fss_velocity *out, bool force_fp64)
+                           fss_velocity *out, bool force_fp64, const RkNext &next)
 {
     const int64_t n = p->n;
     if (n < 1) {
@@ -784,11 +799,11 @@ fss_status velocity_direct(fss_ctx *ctx, const fss_particles *p, const int64_t *
     DevBuf &buf = ctx->direct;
     const int R = sym_targets(p, out, idx, mixed);
     FSS_TRY(buf.ensure(R ? sym_bytes(n, R) : direct_plan(n, m, mixed).bytes));
-    if (ctx->capturing) return launch_direct(ctx, p, idx, m, out, mixed, buf.p, nullptr);
+    if (ctx->capturing) return launch_direct(ctx, p, idx, m, out, mixed, buf.p, next, nullptr);
     Timing &t = ctx->timing;
     timing_begin(t, ctx->stream);
     t.have[t.cur] = 1 << Timing::MAIN;
-    FSS_TRY(launch_direct(ctx, p, idx, m, out, mixed, buf.p, t.slot()));
+    FSS_TRY(launch_direct(ctx, p, idx, m, out, mixed, buf.p, next, t.slot()));
     t.valid = true;
     return FSS_OK;
 }
@@ -849,7 +864,7 @@ fss_status velocity_direct_noalloc(fss_ctx *ctx, const fss_particles *p, fss_vel
         set_error("velocity_direct_noalloc: scratch of device " + std::to_string(dev) + " not set up");
         return FSS_ERR_STATE;
     }
-    return launch_direct(ctx, p, nullptr, n, out, mixed, buf, nullptr);
+    return launch_direct(ctx, p, nullptr, n, out, mixed, buf, RkNext{}, nullptr);
 }
 
 } // namespace fss

@@ -31,6 +31,7 @@
 
 #include "fss_geom.h"
 #include "fss_internal.h"
+#include "fss_rk4_dev.h"
 
 namespace fss {
 
@@ -1136,7 +1137,7 @@ __global__ void k_combine(const int32_t *__restrict__ recid, const int32_t *__re
                           const typename Rec<Real>::T4 *__restrict__ src, const double *__restrict__ centres,
                           const Instance *__restrict__ inst, int ninst, int64_t nrec, int64_t ostride,
                           const double *__restrict__ out, int normalise, double scale, double omega,
-                          double *u, double *v, double *w, double *dvort, uint64_t *ts_first, uint64_t *ts)
+                          double *u, double *v, double *w, double *dvort, RkNext next, uint64_t *ts_first, uint64_t *ts)
 {
     stamp_start(ts_first, Timing::MAIN_END);
     int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
@@ -1217,11 +1218,14 @@ __global__ void k_combine(const int32_t *__restrict__ recid, const int32_t *__re
             add_interp_wave<D>(tinv, alpha, g, node_slot[g], pt, normalise, a0, a1, a2);
         }
     }
-    const double s2 = a2 * scale;
-    u[id] = a0 * scale;
-    v[id] = a1 * scale;
-    w[id] = s2;
-    dvort[id] = -2 * omega * s2;
+    const double s0 = a0 * scale, s1 = a1 * scale, s2 = a2 * scale, s3 = -2 * omega * s2;
+    if (next.mode != RkNext::STEP) {
+        u[id] = s0;
+        v[id] = s1;
+        w[id] = s2;
+        dvort[id] = s3;
+    }
+    rk_next(next, id, s0, s1, s2, s3);
     stamp_end(ts);
 }
 
@@ -1257,7 +1261,8 @@ static fss_status upward(fss_ctx *ctx, typename Rec<Real>::T4 *src)
 }
 
 template <int D>
-static fss_status run_degree(fss_ctx *ctx, const fss_particles *pp, fss_velocity *out, const int32_t *recid, uint64_t *ts)
+static fss_status run_degree(fss_ctx *ctx, const fss_particles *pp, fss_velocity *out, const int32_t *recid,
+                             const RkNext &next, uint64_t *ts)
 {
     Tree &T = ctx->tree;
     hipStream_t s = ctx->stream;
@@ -1323,7 +1328,7 @@ static fss_status run_degree(fss_ctx *ctx, const fss_particles *pp, fss_velocity
                            T.inv_active.as<int32_t>(), ctx->alpha.as<double>(), T.d_tinv,
                            T.src32.as<float4>(), T.d_info, T.inst.as<Instance>(), T.ninst, p0, ost,
                            ctx->out3.as<double>(), bltc ? 1 : 0, scale, ctx->cfg.omega, out->u, out->v, out->w,
-                           out->dvort, first, ts);
+                           out->dvort, next, first, ts);
     else
         hipLaunchKernelGGL((k_combine<double, D>), dim3((unsigned)div_up(p0, 256)), dim3(256), 0, s,
                            recid, T.recnode.as<int32_t>(), T.rinfo.as<uint8_t>(), T.nrange.as<int4>(),
@@ -1331,7 +1336,7 @@ static fss_status run_degree(fss_ctx *ctx, const fss_particles *pp, fss_velocity
                            T.inv_active.as<int32_t>(), ctx->alpha.as<double>(), T.d_tinv,
                            T.src64.as<double4>(), T.d_info, T.inst.as<Instance>(), T.ninst, p0, ost,
                            ctx->out3.as<double>(), bltc ? 1 : 0, scale, ctx->cfg.omega, out->u, out->v, out->w,
-                           out->dvort, first, ts);
+                           out->dvort, next, first, ts);
     FSS_HIP(hipGetLastError());
     return FSS_OK;
 }
@@ -1366,7 +1371,7 @@ fss_status tree_sources64(fss_ctx *ctx, const fss_particles *pp, uint64_t *ts)
     }
 }
 
-fss_status velocity_tree(fss_ctx *ctx, const fss_particles *pp, fss_velocity *out, bool tree_order)
+fss_status velocity_tree(fss_ctx *ctx, const fss_particles *pp, fss_velocity *out, bool tree_order, const RkNext &next)
 {
     Tree &T = ctx->tree;
     const int32_t *recid = tree_order ? nullptr : T.recid.as<int32_t>();
@@ -1388,14 +1393,14 @@ fss_status velocity_tree(fss_ctx *ctx, const fss_particles *pp, fss_velocity *ou
     }
     fss_status st;
     switch (ctx->interp.degree) {
-    case 1: st = run_degree<1>(ctx, pp, out, recid, ts); break;
-    case 2: st = run_degree<2>(ctx, pp, out, recid, ts); break;
-    case 3: st = run_degree<3>(ctx, pp, out, recid, ts); break;
-    case 4: st = run_degree<4>(ctx, pp, out, recid, ts); break;
-    case 5: st = run_degree<5>(ctx, pp, out, recid, ts); break;
-    case 6: st = run_degree<6>(ctx, pp, out, recid, ts); break;
-    case 7: st = run_degree<7>(ctx, pp, out, recid, ts); break;
-    case 8: st = run_degree<8>(ctx, pp, out, recid, ts); break;
+    case 1: st = run_degree<1>(ctx, pp, out, recid, next, ts); break;
+    case 2: st = run_degree<2>(ctx, pp, out, recid, next, ts); break;
+    case 3: st = run_degree<3>(ctx, pp, out, recid, next, ts); break;
+    case 4: st = run_degree<4>(ctx, pp, out, recid, next, ts); break;
+    case 5: st = run_degree<5>(ctx, pp, out, recid, next, ts); break;
+    case 6: st = run_degree<6>(ctx, pp, out, recid, next, ts); break;
+    case 7: st = run_degree<7>(ctx, pp, out, recid, next, ts); break;
+    case 8: st = run_degree<8>(ctx, pp, out, recid, next, ts); break;
     default: set_error("unsupported degree"); return FSS_ERR_INVALID;
     }
     if (st == FSS_OK && !ctx->capturing) ctx->timing.valid = true;

@@ -359,16 +359,31 @@ fss_status tree_export(fss_ctx *ctx, int32_t *loc, uint8_t *found, int32_t *coun
 // ---- interpolation constants (fss_api.cpp) ----
 fss_status interp_setup(fss_ctx *ctx);
 
+// ---- RK4 update at the end of an evaluation (fss_rk4_dev.h) ----
+struct RkNext {
+    enum { NONE = 0, STAGE = 1, STEP = 2 };
+    int mode = NONE;
+    double *x, *y, *z, *vort; // state of the step; STEP writes the new one here
+    const double *k;          // STEP: velocities of the first three stages, 4 n each
+    double *ys;               // STAGE: the next stage's state, 4 n
+    int64_t n;
+    double fac, omega;
+};
+// the update as a kernel of its own, from stored velocities (fss_rk4.hip)
+fss_status rk4_next(fss_ctx *ctx, const RkNext &r, const fss_velocity &k);
+
 // ---- evaluation (fss_eval.hip) ----
 // tree_order: the arrays are in tree order (element i belongs to main record i;
-// only for a tree without exception records)
-fss_status velocity_tree(fss_ctx *ctx, const fss_particles *p, fss_velocity *out, bool tree_order = false);
+// only for a tree without exception records).  next: an RK4 update to take with
+// the velocities; its state may be the evaluated one.  STEP leaves out unwritten.
+fss_status velocity_tree(fss_ctx *ctx, const fss_particles *p, fss_velocity *out, bool tree_order = false,
+                         const RkNext &next = RkNext{});
 // source records of a new plan (room for the particles', the proxies' laid down)
 fss_status proxy_records(fss_ctx *ctx);
 
 // ---- direct sum (fss_direct.hip) ----
 fss_status velocity_direct(fss_ctx *ctx, const fss_particles *p, const int64_t *idx, int64_t m,
-                           fss_velocity *out, bool force_fp64);
+                           fss_velocity *out, bool force_fp64, const RkNext &next = RkNext{});
 
 // allocation-free direct sum (fss_direct.hip): records packed into a
 // file-scope device array of FSS_DIRECT_SCRATCH_BYTES per GPU, whose address

@@ -6,71 +6,26 @@
 //   k1 = f(y); y1 = proj(y + dt/2 k1); k2 = f(y1); y2 = proj(y + dt/2 k2);
 //   k3 = f(y2); y3 = proj(y + dt k3); k4 = f(y3);
 //   y += dt/6 (k1 + 2 k2 + 2 k3 + k4); proj(y)
-// proj = project_points (helpers.h:362-372): x <- x/|x| and
-// omega += -2 Omega (z_new - z_old), which keeps omega + 2 Omega z per particle.
+// The updates are taken by the last kernel of each evaluation (fss_rk4_dev.h).
 // The tree is the t = 0 tree (new_dynamics.cpp:84-88 builds it once).
-// Compiled without FMA contraction: every product and sum of the update is
-// rounded separately, as the reference's scalar_mult and vec_add round them.
 #include <cmath>
 
 #include "fss_internal.h"
+#include "fss_rk4_dev.h"
 
 namespace fss {
 
-__device__ inline void project_one(double &x, double &y, double &z, double &vort, double omega)
-{
-    // project_to_sphere(p, 1.0): p[i] *= 1.0 / norm (helpers.h:82-85)
-    double s = 0.0;
-    s += x * x;
-    s += y * y;
-    s += z * z;
-    double nrm = sqrt(s);
-    double f = 1.0 / nrm;
-    double px = x * f, py = y * f, pz = z * f;
-    double dz = pz - z;
-    x = px;
-    y = py;
-    z = pz;
-    vort += -2 * omega * dz;
-}
-
-// ys = proj(y + fac * k)   (scalar_mult then vec_add, new_dynamics.cpp:174-184)
-__global__ void k_rk4_stage(const double *__restrict__ x, const double *__restrict__ y,
-                            const double *__restrict__ z, const double *__restrict__ vo,
-                            const double *__restrict__ k, int64_t n, double fac, double omega,
-                            double *ys)
+__global__ void k_rk4_next(RkNext r, fss_velocity k)
 {
     int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= n) return;
-    double a = k[i] * fac + x[i];
-    double b = k[n + i] * fac + y[i];
-    double c = k[2 * n + i] * fac + z[i];
-    double d = k[3 * n + i] * fac + vo[i];
-    project_one(a, b, c, d, omega);
-    ys[i] = a;
-    ys[n + i] = b;
-    ys[2 * n + i] = c;
-    ys[3 * n + i] = d;
+    if (i < r.n) rk_next(r, i, k.u[i], k.v[i], k.w[i], k.dvort[i]);
 }
 
-// y += dt/6 (k1 + 2 k2 + 2 k3 + k4); proj(y)   (new_dynamics.cpp:205-229)
-__global__ void k_rk4_final(double *x, double *y, double *z, double *vo, const double *__restrict__ k,
-                            int64_t n, double dt, double omega)
+fss_status rk4_next(fss_ctx *ctx, const RkNext &r, const fss_velocity &k)
 {
-    int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= n) return;
-    double *f[4] = {x, y, z, vo};
-    double v[4];
-    for (int c = 0; c < 4; c++) {
-        double a = k[(int64_t)c * n + i];
-        a += k[4 * n + (int64_t)c * n + i] * 2;
-        a += k[8 * n + (int64_t)c * n + i] * 2;
-        a += k[12 * n + (int64_t)c * n + i];
-        a *= dt / 6;
-        v[c] = f[c][i] + a;
-    }
-    project_one(v[0], v[1], v[2], v[3], omega);
-    for (int c = 0; c < 4; c++) f[c][i] = v[c];
+    hipLaunchKernelGGL(k_rk4_next, dim3((unsigned)div_up(r.n, 256)), dim3(256), 0, ctx->stream, r, k);
+    FSS_HIP(hipGetLastError());
+    return FSS_OK;
 }
 
 // Tree order: with a tree the step runs on copies in the order of the source
@@ -132,28 +87,23 @@ struct State {
 };
 
 static fss_status eval(fss_ctx *ctx, const double *x, const double *y, const double *z,
-                       const double *vo, const State &S, int64_t n, double *k, int use_tree)
+                       const double *vo, const State &S, int64_t n, double *k, int use_tree, const RkNext &next)
 {
     fss_particles p{x, y, z, vo, S.area, n};
     fss_velocity o{k, k + n, k + 2 * n, k + 3 * n};
-    if (use_tree) return velocity_tree(ctx, &p, &o, S.tree_order);
-    return velocity_direct(ctx, &p, nullptr, n, &o, false);
+    if (use_tree) return velocity_tree(ctx, &p, &o, S.tree_order, next);
+    return velocity_direct(ctx, &p, nullptr, n, &o, false, next);
 }
 
 static fss_status step(fss_ctx *ctx, const State &S, int64_t n, double dt, int use_tree)
 {
-    hipStream_t s = ctx->stream;
     double *K = ctx->rk_k.as<double>(), *Y = ctx->rk_y.as<double>();
-    unsigned g = (unsigned)div_up(n, 256);
-    const double fac[3] = {dt / 2, dt / 2, dt};
-    FSS_TRY(eval(ctx, S.x, S.y, S.z, S.vort, S, n, K, use_tree));
-    for (int st = 1; st < 4; st++) {
-        hipLaunchKernelGGL(k_rk4_stage, dim3(g), dim3(256), 0, s, S.x, S.y, S.z, S.vort, K + 4 * n * (st - 1),
-                           n, fac[st - 1], ctx->cfg.omega, Y);
-        FSS_TRY(eval(ctx, Y, Y + n, Y + 2 * n, Y + 3 * n, S, n, K + 4 * n * st, use_tree));
+    const double fac[4] = {dt / 2, dt / 2, dt, dt / 6};
+    for (int st = 0; st < 4; st++) {
+        const RkNext next{st < 3 ? RkNext::STAGE : RkNext::STEP, S.x, S.y, S.z, S.vort, K, Y, n, fac[st], ctx->cfg.omega};
+        if (st == 0) FSS_TRY(eval(ctx, S.x, S.y, S.z, S.vort, S, n, K, use_tree, next));
+        else FSS_TRY(eval(ctx, Y, Y + n, Y + 2 * n, Y + 3 * n, S, n, K + 4 * n * st, use_tree, next));
     }
-    hipLaunchKernelGGL(k_rk4_final, dim3(g), dim3(256), 0, s, S.x, S.y, S.z, S.vort, K, n, dt, ctx->cfg.omega);
-    FSS_HIP(hipGetLastError());
     return FSS_OK;
 }
 
