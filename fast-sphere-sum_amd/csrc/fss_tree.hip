@@ -564,18 +564,18 @@ __global__ void __launch_bounds__(TRAV_BLOCKS) k_trav_types(const int4 *__restri
 }
 
 // Proxy items: the class-B ranges of every interpolant slot cut into parts of
-// about FSS_PROXY_CHUNK sources, in range order (a part closes at the range
+// about `chunk` sources, in range order (a part closes at the range
 // that takes its count to the chunk size, or at the slot's last range).  One
 // wave per slot, counting first and writing after the scan of the counts; a
 // slot with fewer sources than the chunk size in all is one part.
-__device__ inline int32_t chunk_parts(const ProxyItem &it, const Range *__restrict__ rb, ProxyItem *out,
+__device__ inline int32_t chunk_parts(const ProxyItem &it, const Range *__restrict__ rb, int chunk, ProxyItem *out,
                                       int32_t slot)
 {
     int32_t np = 0, b = it.b_beg;
     int64_t acc = 0;
     for (int32_t r = it.b_beg; r < it.b_end; r++) {
         acc += rb[r].count & ~FSS_SELF_BIT;
-        if (acc >= FSS_PROXY_CHUNK || r + 1 == it.b_end) {
+        if (acc >= chunk || r + 1 == it.b_end) {
             if (out) out[np] = ProxyItem{it.node, b, r + 1, slot};
             np++;
             b = r + 1;
@@ -583,6 +583,20 @@ __device__ inline int32_t chunk_parts(const ProxyItem &it, const Range *__restri
         }
     }
     return np;
+}
+
+// Sources per part: FSS_PROXY_CHUNK, or so many that a small tree's parts are 1.5
+// for each SIMD (a wave takes a part, and the longest ends the kernel): FP64 fast
+// sum as the reference has it, N = 10,242, one context alone, 53.7 us with parts of
+// 4,096, 43.1 of 2,048, 38.9 of 1,024, 38.4 of 512; trees of 30,000 particles and more
+// have the items anyway.  Mixed precision keeps 4,096, since the parts' starts
+// decide which FP32 values share a partial sum; so do a batch's instances, which
+// fill the chip together.
+static int proxy_chunk(const fss_ctx *ctx)
+{
+    if (ctx->cfg.precision == FSS_MIXED || ctx->batch_part) return FSS_PROXY_CHUNK;
+    const int64_t c = 128 * div_up(ctx->tree.n_far_src, 128 * 1536);
+    return (int)std::min<int64_t>(FSS_PROXY_CHUNK, std::max<int64_t>(512, c));
 }
 
 // sources of the slot (all lanes hold the sum)
@@ -595,25 +609,25 @@ __device__ inline int64_t slot_sources(const ProxyItem &it, const Range *__restr
 }
 
 __global__ void __launch_bounds__(256) k_chunk_count(const ProxyItem *__restrict__ one, int64_t nslot,
-                                                     const Range *__restrict__ rb, int32_t *cnt)
+                                                     const Range *__restrict__ rb, int chunk, int32_t *cnt)
 {
     const int64_t q = (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6);
     if (q >= nslot) return;
     const ProxyItem it = one[q];
-    const bool split = slot_sources(it, rb) >= FSS_PROXY_CHUNK;
-    if ((threadIdx.x & 63) == 0) cnt[q] = split ? chunk_parts(it, rb, nullptr, (int32_t)q) : it.b_end > it.b_beg ? 1 : 0;
+    const bool split = slot_sources(it, rb) >= chunk;
+    if ((threadIdx.x & 63) == 0) cnt[q] = split ? chunk_parts(it, rb, chunk, nullptr, (int32_t)q) : it.b_end > it.b_beg ? 1 : 0;
 }
 
 __global__ void __launch_bounds__(256) k_chunk_fill(const ProxyItem *__restrict__ one, int64_t nslot,
                                                     const Range *__restrict__ rb, const int32_t *__restrict__ pos,
-                                                    ProxyItem *parts, ProxySlot *slots, BuildInfo *info)
+                                                    int chunk, ProxyItem *parts, ProxySlot *slots, BuildInfo *info)
 {
     const int64_t q = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
     if (q >= nslot) return;
     const int32_t p0 = pos[q], np = pos[q + 1] - p0;
     const ProxyItem it = one[q];
     if (np == 1) parts[p0] = ProxyItem{it.node, it.b_beg, it.b_end, (int32_t)q};
-    else chunk_parts(it, rb, parts + p0, (int32_t)q);
+    else chunk_parts(it, rb, chunk, parts + p0, (int32_t)q);
     slots[q] = ProxySlot{it.node, p0, p0 + np, 0};
     if (q == nslot - 1) info->n_proxy = pos[nslot];
 }
@@ -1203,11 +1217,12 @@ fss_status tree_build(fss_ctx *ctx, const double *x, const double *y, const doub
     hipLaunchKernelGGL(k_plan_items, dim3(gn), dim3(256), 0, s, beg, end, T.nrange.as<int4>(), B.pos.as<int4>(), nn,
                        nA, T.near_items.as<NearItem>(), B.prox_one.as<ProxyItem>(), T.node_slot.as<int32_t>(),
                        T.oslot.as<int32_t>(), T.charge_nodes.as<int32_t>());
-    // Long class-B lists split into chunks of about FSS_PROXY_CHUNK sources
+    // Long class-B lists split into chunks of about `chunk` sources
     // (order inside a node is kept).  Every chunk but a slot's last holds that
     // many, so this many items are room enough; their number stays on the
     // device until the build's last synchronisation.
-    const int64_t proxy_room = T.n_slot + T.n_far_src / FSS_PROXY_CHUNK;
+    const int chunk = proxy_chunk(ctx);
+    const int64_t proxy_room = T.n_slot + T.n_far_src / chunk;
     FSS_TRY(T.proxy_slots.ensure(sizeof(ProxySlot) * std::max<int64_t>(1, T.n_slot)));
     FSS_TRY(T.proxy_items.ensure(sizeof(ProxyItem) * std::max<int64_t>(1, proxy_room)));
     if (T.n_slot > 0) {
@@ -1215,11 +1230,11 @@ fss_status tree_build(fss_ctx *ctx, const double *x, const double *y, const doub
         FSS_TRY(B.rpos.ensure(sizeof(int32_t) * (T.n_slot + 1)));
         FSS_HIP(hipMemsetAsync(B.rcnt.as<int32_t>() + T.n_slot, 0, sizeof(int32_t), s));
         hipLaunchKernelGGL(k_chunk_count, dim3((unsigned)div_up(T.n_slot, 4)), dim3(256), 0, s,
-                           B.prox_one.as<ProxyItem>(), T.n_slot, T.ranges_b.as<Range>(), B.rcnt.as<int32_t>());
+                           B.prox_one.as<ProxyItem>(), T.n_slot, T.ranges_b.as<Range>(), chunk, B.rcnt.as<int32_t>());
         FSS_TRY(cub_exclusive_sum(B.cub, B.rcnt.as<int32_t>(), B.rpos.as<int32_t>(), T.n_slot + 1, s));
         hipLaunchKernelGGL(k_chunk_fill, dim3((unsigned)div_up(T.n_slot, 256)), dim3(256), 0, s,
                            B.prox_one.as<ProxyItem>(), T.n_slot, T.ranges_b.as<Range>(), B.rpos.as<int32_t>(),
-                           T.proxy_items.as<ProxyItem>(), T.proxy_slots.as<ProxySlot>(), info);
+                           chunk, T.proxy_items.as<ProxyItem>(), T.proxy_slots.as<ProxySlot>(), info);
     }
     T.n_proxy = proxy_room;
     // maps of the memberships outside the main paths
