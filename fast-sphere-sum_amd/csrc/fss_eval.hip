@@ -667,6 +667,49 @@ __device__ inline void near_tile_pairwise(const float4 *xt, const float4 &s, Acc
 }
 
 // ------------------------------------------------------------------
+// interpolants: sum the chunks of each node in order and solve alpha = V^{-1} phi
+// (dgetrs, fast_rhs.h:217): one thread per (slot, component); the row
+// interchanges are applied while summing (perm: the composed ipiv sequence)
+// ------------------------------------------------------------------
+struct SolveArgs {
+    const ProxySlot *__restrict__ slots;
+    int64_t nslot;
+    const double *__restrict__ phi;
+    const double *__restrict__ lu;
+    const int32_t *__restrict__ perm;
+    double *alpha;
+    int blocks; // of 64 threads that k_near gives to it, a multiple of 8
+};
+template <int D> __device__ inline void solve_slot(const SolveArgs &a, int64_t i)
+{
+    constexpr int P = npts<D>();
+    if (i >= 3 * a.nslot) return;
+    int64_t q = i / 3;
+    int c = (int)(i % 3);
+    ProxySlot sl = a.slots[q];
+    double b[P];
+#pragma unroll
+    for (int k = 0; k < P; k++) b[k] = 0.0;
+    for (int part = sl.part_beg; part < sl.part_end; part++) {
+        const double *o = a.phi + (int64_t)part * 3 * P + c * P;
+#pragma unroll
+        for (int k = 0; k < P; k++) b[k] += o[a.perm[k]];
+    }
+#pragma unroll
+    for (int k = 0; k < P; k++)
+#pragma unroll
+        for (int r = k + 1; r < P; r++) b[r] = b[r] - b[k] * a.lu[r + k * P];
+#pragma unroll
+    for (int k = P - 1; k >= 0; k--) {
+        b[k] = b[k] / a.lu[k + k * P];
+#pragma unroll
+        for (int r = 0; r < k; r++) b[r] = b[r] - b[k] * a.lu[r + k * P];
+    }
+    double *o = a.alpha + q * 3 * P + c * P;
+#pragma unroll
+    for (int k = 0; k < P; k++) o[k] = b[k];
+}
+// ------------------------------------------------------------------
 // near field (class A): direct pairs, R targets per lane
 // ------------------------------------------------------------------
 // The item's source list (records of the ranges that cannot hold one of its
@@ -675,7 +718,14 @@ __device__ inline void near_tile_pairwise(const float4 *xt, const float4 &s, Acc
 // record loads of a chunk are independent and issued together.  Self sources
 // stage their particle ids too and run a masked evaluation that skips the
 // self pair; the others run the branch-free loop.
-template <typename Real, int R, bool SPH>
+//
+// DS > 0: the first blocks solve the interpolants of degree DS, which need the
+// proxy values of the kernel before and are needed by the one after.  A launch
+// of their own costs the host 3.5 us and the chip a tail (5 us at degree 2 on the
+// level-8 grid, 16 for 24 instances).  Degrees above 3 keep it: their right-hand
+// sides do not fit beside the FP32 kernel's 64 registers.
+constexpr int solve_in_near(int d) { return d <= 3 ? d : 0; }
+template <typename Real, int R, bool SPH, int DS>
 __global__ void __launch_bounds__(64, sizeof(Real) == 4 && R == 2 ? 8 : 4) k_near(const NearItem *__restrict__ items,
                                              const int32_t *__restrict__ near_src,
                                              const typename Rec<Real>::T4 *__restrict__ src,
@@ -685,9 +735,15 @@ __global__ void __launch_bounds__(64, sizeof(Real) == 4 && R == 2 ? 8 : 4) k_nea
                                              const double *__restrict__ x,
                                              const double *__restrict__ y,
                                              const double *__restrict__ z, int64_t ostride, double *out,
-                                             uint64_t *ts)
+                                             SolveArgs solve, uint64_t *ts)
 {
     stamp_start(ts, Timing::MAIN);
+    if constexpr (DS > 0) {
+        if ((int)blockIdx.x < solve.blocks) {
+            solve_slot<DS>(solve, (int64_t)blockIdx.x * 64 + threadIdx.x);
+            return;
+        }
+    }
     using T4 = typename Rec<Real>::T4;
     // staged records and their particle ids, or after the last chunk the
     // phase partials [64][3R] and sums [T][3R] (T <= 64 / R + 1); one buffer
@@ -701,7 +757,8 @@ __global__ void __launch_bounds__(64, sizeof(Real) == 4 && R == 2 ? 8 : 4) k_nea
     int32_t *lid = reinterpret_cast<int32_t *>(smem + sizeof(T4) * NCH);
     // Blocks go round-robin to the 8 XCDs: give every XCD a contiguous run of
     // items (neighbouring leaves, largely the same sources) for its own L2.
-    const int nb = gridDim.x, q8 = nb >> 3, r8 = nb & 7, xcd = blockIdx.x & 7, loc = blockIdx.x >> 3;
+    const int sb = DS > 0 ? solve.blocks : 0;
+    const int nb = gridDim.x - sb, q8 = nb >> 3, r8 = nb & 7, xcd = blockIdx.x & 7, loc = (blockIdx.x - sb) >> 3;
     const NearItem it = items[(xcd < r8 ? xcd * (q8 + 1) : r8 * (q8 + 1) + (xcd - r8) * q8) + loc];
     const int lane = threadIdx.x;
     const int cnt = it.tgt_cnt;
@@ -1026,42 +1083,10 @@ __global__ void __launch_bounds__(256) k_proxy_list(const ProxyItem *__restrict_
     }
 }
 
-// sum the chunks of each node in order and solve alpha = V^{-1} phi
-// (dgetrs, fast_rhs.h:217): one thread per (slot, component); the row
-// interchanges are applied while summing (perm: the composed ipiv sequence)
-template <int D>
-__global__ void __launch_bounds__(128) k_solve(const ProxySlot *__restrict__ slots, int64_t nslot,
-                        const double *__restrict__ phi, const double *__restrict__ lu,
-                        const int32_t *__restrict__ perm, double *alpha, uint64_t *ts)
+template <int D> __global__ void __launch_bounds__(128) k_solve(SolveArgs a, uint64_t *ts)
 {
     stamp_start(ts, Timing::MAIN_END);
-    constexpr int P = npts<D>();
-    int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= 3 * nslot) return;
-    int64_t q = i / 3;
-    int c = (int)(i % 3);
-    ProxySlot sl = slots[q];
-    double b[P];
-#pragma unroll
-    for (int k = 0; k < P; k++) b[k] = 0.0;
-    for (int part = sl.part_beg; part < sl.part_end; part++) {
-        const double *o = phi + (int64_t)part * 3 * P + c * P;
-#pragma unroll
-        for (int k = 0; k < P; k++) b[k] += o[perm[k]];
-    }
-#pragma unroll
-    for (int k = 0; k < P; k++)
-#pragma unroll
-        for (int r = k + 1; r < P; r++) b[r] = b[r] - b[k] * lu[r + k * P];
-#pragma unroll
-    for (int k = P - 1; k >= 0; k--) {
-        b[k] = b[k] / lu[k + k * P];
-#pragma unroll
-        for (int r = 0; r < k; r++) b[r] = b[r] - b[k] * lu[r + k * P];
-    }
-    double *o = alpha + q * 3 * P + c * P;
-#pragma unroll
-    for (int k = 0; k < P; k++) o[k] = b[k];
+    solve_slot<D>(a, (int64_t)blockIdx.x * blockDim.x + threadIdx.x);
 }
 
 // ------------------------------------------------------------------
@@ -1275,6 +1300,11 @@ static fss_status run_degree(fss_ctx *ctx, const fss_particles *pp, fss_velocity
     FSS_TRY(ctx->out3.ensure(sizeof(double) * 3 * ost));
     FSS_TRY(ctx->phi.ensure(sizeof(double) * 3 * p * std::max<int64_t>(1, T.n_proxy)));
     FSS_TRY(ctx->alpha.ensure(sizeof(double) * 3 * p * std::max<int64_t>(1, T.n_slot)));
+    constexpr int DS = solve_in_near(D);
+    SolveArgs sol{T.proxy_slots.as<ProxySlot>(), T.n_slot, ctx->phi.as<double>(), ctx->d_lu.as<double>(),
+                  ctx->d_perm.as<int32_t>(), ctx->alpha.as<double>(), 0};
+    if (DS > 0 && T.n_near > 0) sol.blocks = 8 * (int)div_up(3 * T.n_slot, 8 * 64);
+    const dim3 gn((unsigned)(sol.blocks + T.n_near));
     const dim3 gs((unsigned)div_up(p0, 256));
     if (!mixed) {
         double4 *src = T.src64.as<double4>();
@@ -1290,11 +1320,11 @@ static fss_status run_degree(fss_ctx *ctx, const fss_particles *pp, fss_velocity
         }
             if (T.n_near > 0) {
             // default 4 targets per lane; the treecode's near pairs use the sphere form
-            auto kn = bltc ? (ctx->near_r == 2 ? k_near<double, 2, true> : k_near<double, 4, true>)
-                           : (ctx->near_r == 2 ? k_near<double, 2, false> : k_near<double, 4, false>);
-            hipLaunchKernelGGL(kn, dim3((unsigned)T.n_near), dim3(64), 0, s, T.near_items.as<NearItem>(),
+            auto kn = bltc ? (ctx->near_r == 2 ? k_near<double, 2, true, DS> : k_near<double, 4, true, DS>)
+                           : (ctx->near_r == 2 ? k_near<double, 2, false, DS> : k_near<double, 4, false, DS>);
+            hipLaunchKernelGGL(kn, gn, dim3(64), 0, s, T.near_items.as<NearItem>(),
                                T.near_src.as<int32_t>(), src, recid, T.srcnode.as<int32_t>(), (int32_t)p0,
-                               T.d_info, pp->x, pp->y, pp->z, ost, ctx->out3.as<double>(), ts);
+                               T.d_info, pp->x, pp->y, pp->z, ost, ctx->out3.as<double>(), sol, ts);
         }
         } else {
         float4 *src = T.src32.as<float4>();
@@ -1310,17 +1340,16 @@ static fss_status run_degree(fss_ctx *ctx, const fss_particles *pp, fss_velocity
                                T.proxy_xyz.as<double4>(), ctx->phi.as<double>(), ts);
         }
             if (T.n_near > 0) {
-            auto kn = ctx->near_r == 4 ? k_near<float, 4, false> : k_near<float, 2, false>; // default 2
-            hipLaunchKernelGGL(kn, dim3((unsigned)T.n_near), dim3(64), 0, s, T.near_items.as<NearItem>(),
+            auto kn = ctx->near_r == 4 ? k_near<float, 4, false, DS> : k_near<float, 2, false, DS>; // default 2
+            hipLaunchKernelGGL(kn, gn, dim3(64), 0, s, T.near_items.as<NearItem>(),
                                T.near_src.as<int32_t>(), src, recid, T.srcnode.as<int32_t>(), (int32_t)p0,
-                               T.d_info, pp->x, pp->y, pp->z, ost, ctx->out3.as<double>(), ts);
+                               T.d_info, pp->x, pp->y, pp->z, ost, ctx->out3.as<double>(), sol, ts);
         }
         }
-    if (T.n_slot > 0)
-        hipLaunchKernelGGL((k_solve<D>), dim3((unsigned)div_up(3 * T.n_slot, 128)), dim3(128), 0, s,
-                           T.proxy_slots.as<ProxySlot>(), T.n_slot, ctx->phi.as<double>(),
-                           ctx->d_lu.as<double>(), ctx->d_perm.as<int32_t>(), ctx->alpha.as<double>(), ts);
-    uint64_t *first = T.n_slot > 0 ? nullptr : ts;
+    const bool solve = T.n_slot > 0 && sol.blocks == 0; // not done by k_near
+    if (solve)
+        hipLaunchKernelGGL((k_solve<D>), dim3((unsigned)div_up(3 * T.n_slot, 128)), dim3(128), 0, s, sol, ts);
+    uint64_t *first = solve ? nullptr : ts;
     if (mixed)
         hipLaunchKernelGGL((k_combine<float, D>), dim3((unsigned)div_up(p0, 256)), dim3(256), 0, s,
                            recid, T.recnode.as<int32_t>(), T.rinfo.as<uint8_t>(), T.nrange.as<int4>(),
