@@ -8,6 +8,7 @@
 #include <cmath>
 #include <cstring>
 #include <exception>
+#include <mutex>
 #include <new>
 #include <string>
 #include <vector>
@@ -49,6 +50,65 @@ void DevBuf::release()
     }
     p = nullptr;
     bytes = 0;
+}
+
+// ---- page-locked words (HostWords) ----
+constexpr size_t WORDS_WAITING = 16;
+// blocks that wait for a context, page-locked for all devices; never destroyed, as
+// a context may end after the library's static objects
+struct WordsPool {
+    std::mutex mu;
+    std::vector<void *> free;
+    WordsPool() { free.reserve(WORDS_WAITING); }
+};
+static WordsPool &words_pool()
+{
+    static WordsPool *pool = new WordsPool;
+    return *pool;
+}
+
+static void *words_take()
+{
+    {
+        WordsPool &pool = words_pool();
+        std::lock_guard<std::mutex> lock(pool.mu);
+        if (!pool.free.empty()) {
+            void *p = pool.free.back();
+            pool.free.pop_back();
+            return p;
+        }
+    }
+    void *p = nullptr;
+    if (hipHostMalloc(&p, HostWords::BYTES, hipHostMallocPortable) != hipSuccess) {
+        (void)hipGetLastError();
+        return nullptr;
+    }
+    return p;
+}
+
+// the context's stream has been waited for
+HostWords::~HostWords()
+{
+    if (!p) return;
+    {
+        WordsPool &pool = words_pool();
+        std::lock_guard<std::mutex> lock(pool.mu);
+        if (pool.free.size() < WORDS_WAITING) {
+            pool.free.push_back(p);
+            return;
+        }
+    }
+    (void)hipHostFree(p);
+}
+
+fss_status read_back(fss_ctx *ctx, void *dst, const void *src, size_t bytes)
+{
+    if (bytes <= HostWords::BYTES && !ctx->words.p) ctx->words.p = words_take();
+    const bool words = bytes <= HostWords::BYTES && ctx->words.p;
+    FSS_HIP(hipMemcpyAsync(words ? ctx->words.p : dst, src, bytes, hipMemcpyDeviceToHost, ctx->stream));
+    FSS_HIP(hipStreamSynchronize(ctx->stream));
+    if (words) std::memcpy(dst, ctx->words.p, bytes);
+    return FSS_OK;
 }
 
 // ---- interpolation constants (interp_utils.h:12-75) ----

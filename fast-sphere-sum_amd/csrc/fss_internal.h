@@ -243,12 +243,13 @@ struct Geo {
 
 // Scratch of tree_build, kept between builds while it is small (BUILD_SCRATCH_KEEP).
 struct BuildScratch {
-    DevBuf info, cub, ecnt, k0, k1, v0, v1, ek0, ek1, ev0, ev1, f0, f1, act, blk, types, begend, charge, per, pos, keys,
+    // info: BuildInfo, then the build's other arrays that start at zero (ZeroParts, fss_tree.hip)
+    DevBuf info, cub, k0, k1, v0, v1, ek0, ek1, ev0, ev1, f0, f1, act, blk, per, pos, keys,
         keys2, vals, vals2, rcnt, rpos, rkeys, prox_one, cnt, off;
     std::vector<DevBuf *> all()
     {
-        return {&info, &cub,    &ecnt, &k0,  &k1,  &v0,   &v1,    &ek0,  &ek1,   &ev0,  &ev1,  &f0,    &f1,       &act, &blk,
-                &types, &begend, &charge, &per, &pos, &keys, &keys2, &vals, &vals2, &rcnt, &rpos, &rkeys, &prox_one, &cnt, &off};
+        return {&info, &cub, &k0,  &k1,  &v0,   &v1,    &ek0,  &ek1,   &ev0,  &ev1,  &f0,    &f1,       &act, &blk,
+                &per, &pos, &keys, &keys2, &vals, &vals2, &rcnt, &rpos, &rkeys, &prox_one, &cnt, &off};
     }
 };
 
@@ -257,6 +258,22 @@ struct BuildScratch {
 struct Remesh {
     DevBuf miss, cnt, tri, count, start, scan, place, cap, bin, odd;
 };
+
+// Page-locked host memory for the few words that a call reads back: a copy to
+// pageable memory takes 23 us with its wait, one to page-locked memory 15.  Taking
+// it costs 70 us, so contexts hand theirs on (words_take, words_give in
+// fss_api.cpp: at most 16 wait, the others are freed).
+struct HostWords {
+    static constexpr size_t BYTES = 4096;
+    void *p = nullptr;
+    HostWords() = default;
+    HostWords(const HostWords &) = delete;
+    HostWords &operator=(const HostWords &) = delete;
+    ~HostWords();
+};
+// bytes from the device after everything before them on the context's stream;
+// waits for them
+fss_status read_back(fss_ctx *ctx, void *dst, const void *src, size_t bytes);
 
 // Device time stamps of each velocity call in a ring of RING slots, kept without
 // synchronizing; the mean over the slots since the last reset is read with
@@ -315,6 +332,7 @@ struct fss_ctx {
     fss::Remesh remesh;
     fss::Geo geo;
     fss::BuildScratch build;
+    fss::HostWords words;
 
     // device constants
     fss::DevBuf d_lu, d_perm, d_vinv, d_pts;

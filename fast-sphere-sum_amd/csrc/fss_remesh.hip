@@ -318,8 +318,7 @@ fss_status remesh(fss_ctx *ctx, const double *ax, const double *ay, const double
                        atr, tris, vt_off, vt_idx, x, y, z, omega, vort, tr, to, miss, c);
     FSS_HIP(hipGetLastError());
     unsigned long long h[2] = {0, 0};
-    FSS_HIP(hipMemcpyAsync(h, c, sizeof(unsigned long long), hipMemcpyDeviceToHost, s));
-    FSS_HIP(hipStreamSynchronize(s));
+    FSS_TRY(read_back(ctx, h, c, sizeof(unsigned long long)));
     if (h[0] > 0) {
         const RmGrid g = rm_grid(ntri);
         const int64_t nc = (int64_t)g.G * g.G * g.G;
@@ -345,8 +344,7 @@ fss_status remesh(fss_ctx *ctx, const double *ax, const double *ay, const double
                            ax, ay, az, avort, atr, tris, g, W.start.as<int32_t>(), W.bin.as<int32_t>(),
                            W.cap.as<float4>(), W.odd.as<int32_t>(), nodd, x, y, z, omega, vort, tr, to, c + 1);
         FSS_HIP(hipGetLastError());
-        FSS_HIP(hipMemcpyAsync(h + 1, c + 1, sizeof(unsigned long long), hipMemcpyDeviceToHost, s));
-        FSS_HIP(hipStreamSynchronize(s));
+        FSS_TRY(read_back(ctx, h + 1, c + 1, sizeof(unsigned long long)));
     }
     if (n_fallback) *n_fallback = (int64_t)h[0];
     if (n_missing) *n_missing = (int64_t)h[1];

@@ -897,12 +897,19 @@ static fss_status cub_exclusive_add4(DevBuf &tmp, const int4 *in, int4 *out, int
     return FSS_OK;
 }
 
-static fss_status d2h(void *dst, const void *src, size_t bytes, hipStream_t s)
-{
-    FSS_HIP(hipMemcpyAsync(dst, src, bytes, hipMemcpyDeviceToHost, s));
-    FSS_HIP(hipStreamSynchronize(s));
-    return FSS_OK;
-}
+// The build's arrays that start at zero, in one buffer cleared by one memset (six
+// of them took 3 us each of the host)
+struct ZeroParts {
+    size_t types, ecnt, begend, charge, bytes; // after the BuildInfo
+    explicit ZeroParts(int64_t nn)
+    {
+        types = (sizeof(BuildInfo) + 15) / 16 * 16;
+        ecnt = types + sizeof(int4) * TRAV_BLOCKS;
+        begend = ecnt + sizeof(int32_t) * nn;
+        charge = begend + sizeof(int32_t) * 4 * nn;
+        bytes = charge + nn;
+    }
+};
 
 // The build's scratch arrays stay with the context while they are small
 // (allocating and freeing about forty of them was 5 of a 13 ms build) and are
@@ -950,7 +957,7 @@ static fss_status geo_ensure(fss_ctx *ctx, int levels)
 // point location and tree order of the main records (keys of type Key)
 template <typename Key>
 static fss_status locate_and_sort(fss_ctx *ctx, const double *x, const double *y, const double *z, int64_t n,
-                                  uint64_t maxkey, const Pow5 &pw)
+                                  uint64_t maxkey, const Pow5 &pw, int32_t *ecnt)
 {
     Tree &T = ctx->tree;
     BuildScratch &B = ctx->build;
@@ -962,7 +969,7 @@ static fss_status locate_and_sort(fss_ctx *ctx, const double *x, const double *y
     FSS_TRY(B.v1.ensure(sizeof(int32_t) * n));
     hipLaunchKernelGGL((k_locate<Key>), dim3(gp), dim3(256), 0, s, x, y, z, n, T.L, T.d_xyz, T.d_tinv,
                        ctx->cfg.assign_mode == FSS_ASSIGN_ROBUST ? 1 : 0, T.loc.as<int32_t>(), T.found.as<uint8_t>(),
-                       B.k0.as<Key>(), B.v0.as<int32_t>(), B.ecnt.as<int32_t>(), B.info.as<BuildInfo>());
+                       B.k0.as<Key>(), B.v0.as<int32_t>(), ecnt, B.info.as<BuildInfo>());
     FSS_TRY(cub_sort_pairs(B.cub, B.k0.as<Key>(), B.k1.as<Key>(), B.v0.as<int32_t>(), B.v1.as<int32_t>(), n,
                            bits_for64(maxkey), s));
     hipLaunchKernelGGL((k_main_ranges<Key>), dim3(gp), dim3(256), 0, s, B.k1.as<Key>(), B.v1.as<int32_t>(),
@@ -1020,8 +1027,8 @@ fss_status tree_build(fss_ctx *ctx, const double *x, const double *y, const doub
     T.d_tinv = ctx->geo.tinv.as<double>();
 
     // ---- point location, tree order of the source records, list lengths ----
-    FSS_TRY(B.info.ensure(sizeof(BuildInfo)));
-    FSS_TRY(B.ecnt.ensure(sizeof(int32_t) * T.nn));
+    const ZeroParts Z(T.nn);
+    FSS_TRY(B.info.ensure(Z.bytes));
     FSS_TRY(T.loc.ensure(sizeof(int32_t) * L * n));
     FSS_TRY(T.found.ensure((size_t)L * n));
     FSS_TRY(T.counts.ensure(sizeof(int32_t) * T.nn));
@@ -1031,8 +1038,12 @@ fss_status tree_build(fss_ctx *ctx, const double *x, const double *y, const doub
     FSS_TRY(T.rinfo.ensure(n));
     FSS_TRY(T.ipos.ensure(sizeof(int32_t) * n));
     BuildInfo *info = B.info.as<BuildInfo>();
-    FSS_HIP(hipMemsetAsync(B.info.p, 0, sizeof(BuildInfo), s));
-    FSS_HIP(hipMemsetAsync(B.ecnt.p, 0, sizeof(int32_t) * T.nn, s));
+    char *const zero = B.info.as<char>();
+    int4 *const types = reinterpret_cast<int4 *>(zero + Z.types);
+    int32_t *const ecnt = reinterpret_cast<int32_t *>(zero + Z.ecnt);
+    int32_t *const beg = reinterpret_cast<int32_t *>(zero + Z.begend), *const end = beg + 2 * T.nn;
+    uint8_t *const charge = reinterpret_cast<uint8_t *>(zero + Z.charge);
+    FSS_HIP(hipMemsetAsync(zero, 0, Z.bytes, s));
     FSS_HIP(hipMemsetAsync(T.nrange.p, 0, sizeof(int4) * T.nn, s));
     uint64_t maxkey = 21;
     Pow5 pw{};
@@ -1041,11 +1052,11 @@ fss_status tree_build(fss_ctx *ctx, const double *x, const double *y, const doub
     for (int l = 1; l < L; l++) maxkey *= 5;
     const bool key32 = maxkey <= UINT32_MAX;
     auto sorted_records = [&]() -> fss_status {
-        return key32 ? locate_and_sort<uint32_t>(ctx, x, y, z, n, maxkey, pw)
-                     : locate_and_sort<unsigned long long>(ctx, x, y, z, n, maxkey, pw);
+        return key32 ? locate_and_sort<uint32_t>(ctx, x, y, z, n, maxkey, pw, ecnt)
+                     : locate_and_sort<unsigned long long>(ctx, x, y, z, n, maxkey, pw, ecnt);
     };
     FSS_TRY(sorted_records());
-    hipLaunchKernelGGL(k_nrange_counts, dim3((unsigned)div_up(T.nn, 256)), dim3(256), 0, s, B.ecnt.as<int32_t>(), T.nn,
+    hipLaunchKernelGGL(k_nrange_counts, dim3((unsigned)div_up(T.nn, 256)), dim3(256), 0, s, ecnt, T.nn,
                        T.nrange.as<int4>(), T.counts.as<int32_t>());
 
     // ---- traversal ----
@@ -1061,28 +1072,26 @@ fss_status tree_build(fss_ctx *ctx, const double *x, const double *y, const doub
         int64_t capF = std::max<int64_t>(cap, (int64_t)(B.f0.bytes / sizeof(int4)));
         const int gens = 2 * L - 1; // every split takes one of the pair's two nodes a level down
         FSS_TRY(B.blk.ensure(sizeof(int2) * TRAV_BLOCKS));
-        FSS_TRY(B.types.ensure(sizeof(int4) * TRAV_BLOCKS));
         for (;;) {
             FSS_TRY(B.f0.ensure(sizeof(int4) * capF));
             FSS_TRY(B.f1.ensure(sizeof(int4) * capF));
             FSS_TRY(B.act.ensure(capF));
             FSS_TRY(T.inter.ensure(sizeof(int32_t) * 7 * capI));
-            FSS_HIP(hipMemsetAsync(B.types.p, 0, sizeof(int4) * TRAV_BLOCKS, s));
             hipLaunchKernelGGL(k_trav_init, dim3(2), dim3(256), 0, s, B.f0.as<int4>(), info);
             int4 *F = B.f0.as<int4>(), *Fn = B.f1.as<int4>();
             for (int g = 0; g < gens; g++) {
                 hipLaunchKernelGGL(k_trav_classify, dim3(TRAV_BLOCKS), dim3(256), 0, s, F, info, g,
                                    T.counts.as<int32_t>(), T.d_info, ctx->geo.aux.as<double2>(),
                                    mac_thetas(L, cfg.theta, cfg.theta_decay), cfg.many_count, L, cfg.radius,
-                                   bltc ? 1 : 0, B.act.as<int8_t>(), B.blk.as<int2>(), B.types.as<int4>());
+                                   bltc ? 1 : 0, B.act.as<int8_t>(), B.blk.as<int2>(), types);
                 hipLaunchKernelGGL(k_trav_scatter, dim3(TRAV_BLOCKS), dim3(256), 0, s, F, info, g,
                                    B.act.as<int8_t>(), B.blk.as<int2>(), T.counts.as<int32_t>(),
                                    T.inter.as<int32_t>(), capI, Fn, capF);
                 std::swap(F, Fn);
             }
-            hipLaunchKernelGGL(k_trav_types, dim3(1), dim3(TRAV_BLOCKS), 0, s, B.types.as<int4>(), info);
+            hipLaunchKernelGGL(k_trav_types, dim3(1), dim3(TRAV_BLOCKS), 0, s, types, info);
             FSS_HIP(hipGetLastError());
-            FSS_TRY(d2h(&h, info, sizeof(h), s));
+            FSS_TRY(read_back(ctx, &h, info, sizeof(h)));
             if (!h.overflow) break;
             if ((int64_t)h.needI > INT32_MAX / 2) return too_many((int64_t)h.needI);
             if ((int64_t)h.needF > INT32_MAX) return too_many((int64_t)h.needF);
@@ -1090,6 +1099,7 @@ fss_status tree_build(fss_ctx *ctx, const double *x, const double *y, const doub
             if ((int64_t)h.needF > capF) capF = std::max<int64_t>(2 * capF, (int64_t)h.needF);
             // sizes of the generations and the overflow marks start again
             FSS_HIP(hipMemsetAsync(info->nF, 0, offsetof(BuildInfo, types) - offsetof(BuildInfo, nF), s));
+            FSS_HIP(hipMemsetAsync(types, 0, sizeof(int4) * TRAV_BLOCKS, s));
         }
     }
     const int64_t ninter = (int64_t)*std::max_element(h.nE, h.nE + 28);
@@ -1118,9 +1128,9 @@ fss_status tree_build(fss_ctx *ctx, const double *x, const double *y, const doub
         FSS_TRY(T.rinfo.ensure(T.p0));
         FSS_HIP(hipMemsetAsync(T.rinfo.p, 0, T.p0, s));
         FSS_HIP(hipMemsetAsync(T.nrange.p, 0, sizeof(int4) * T.nn, s));
-        FSS_HIP(hipMemsetAsync(B.ecnt.p, 0, sizeof(int32_t) * T.nn, s));
+        FSS_HIP(hipMemsetAsync(ecnt, 0, sizeof(int32_t) * T.nn, s));
         FSS_TRY(sorted_records());
-        hipLaunchKernelGGL(k_nrange_counts, dim3((unsigned)div_up(T.nn, 256)), dim3(256), 0, s, B.ecnt.as<int32_t>(),
+        hipLaunchKernelGGL(k_nrange_counts, dim3((unsigned)div_up(T.nn, 256)), dim3(256), 0, s, ecnt,
                            T.nn, T.nrange.as<int4>(), T.counts.as<int32_t>());
         // exception memberships, sorted by (node, particle)
         using u64 = unsigned long long;
@@ -1146,13 +1156,8 @@ fss_status tree_build(fss_ctx *ctx, const double *x, const double *y, const doub
                        ctx->d_pts.as<double>(), p, T.nn, bltc ? 1 : 0, T.proxy_xyz.as<double4>());
     const int64_t m = ninter;
     const int64_t mA = T.stats.n_type[0] + T.stats.n_type[1]; // class-A interactions (sorted first)
-    FSS_TRY(B.begend.ensure(sizeof(int32_t) * 4 * T.nn));
-    FSS_TRY(B.charge.ensure(T.nn));
     FSS_TRY(B.per.ensure(sizeof(int4) * (T.nn + 1)));
     FSS_TRY(B.pos.ensure(sizeof(int4) * (T.nn + 1)));
-    FSS_HIP(hipMemsetAsync(B.begend.p, 0, sizeof(int32_t) * 4 * T.nn, s));
-    FSS_HIP(hipMemsetAsync(B.charge.p, 0, T.nn, s));
-    int32_t *beg = B.begend.as<int32_t>(), *end = beg + 2 * T.nn;
     int64_t nA = mA, nR = m; // ranges: one per interaction, two where a particle source node has exception members
     if (m > 0) {
         const unsigned gb = (unsigned)div_up(m, 256);
@@ -1175,8 +1180,8 @@ fss_status tree_build(fss_ctx *ctx, const double *x, const double *y, const doub
                                B.rcnt.as<int32_t>());
             FSS_TRY(cub_exclusive_sum(B.cub, B.rcnt.as<int32_t>(), rpos, m + 1, s));
             int32_t a = 0, r = 0;
-            FSS_TRY(d2h(&a, rpos + mA, 4, s));
-            FSS_TRY(d2h(&r, rpos + m, 4, s));
+            FSS_TRY(read_back(ctx, &a, rpos + mA, 4));
+            FSS_TRY(read_back(ctx, &r, rpos + m, 4));
             nA = a;
             nR = r;
             FSS_TRY(B.rkeys.ensure(sizeof(uint32_t) * nR));
@@ -1187,7 +1192,7 @@ fss_status tree_build(fss_ctx *ctx, const double *x, const double *y, const doub
         hipLaunchKernelGGL(k_plan_ranges, dim3((unsigned)std::min<int64_t>(gb, 512)), dim3(256), 0, s,
                            T.inter.as<int32_t>(), B.vals2.as<int32_t>(), B.keys2.as<uint32_t>(), rpos, m, nA,
                            T.nrange.as<int4>(), bltc ? 1 : 0, p, T.p0, T.ranges_a.as<Range>(), T.ranges_b.as<Range>(),
-                           rkeys, B.charge.as<uint8_t>(), info);
+                           rkeys, charge, info);
         hipLaunchKernelGGL(k_plan_segments, dim3((unsigned)div_up(nR, 256)), dim3(256), 0, s,
                            rkeys ? rkeys : B.keys2.as<uint32_t>(), nR, nn, beg, end);
     } else {
@@ -1197,10 +1202,10 @@ fss_status tree_build(fss_ctx *ctx, const double *x, const double *y, const doub
     T.n_ra = nA;
     T.n_rb = nR - nA;
     hipLaunchKernelGGL(k_plan_nodes, dim3(gn), dim3(256), 0, s, beg, end, T.nrange.as<int4>(),
-                       B.charge.as<uint8_t>(), nn, B.per.as<int4>());
+                       charge, nn, B.per.as<int4>());
     FSS_TRY(cub_exclusive_add4(B.cub, B.per.as<int4>(), B.pos.as<int4>(), T.nn + 1, s));
     FSS_HIP(hipMemcpyAsync(&info->totals, B.pos.as<int4>() + T.nn, sizeof(int4), hipMemcpyDeviceToDevice, s));
-    FSS_TRY(d2h(&h, info, sizeof(h), s));
+    FSS_TRY(read_back(ctx, &h, info, sizeof(h)));
     T.pairs_near = T.stats.pairs_near = (int64_t)h.pairs[0];
     T.pairs_far = T.stats.pairs_far = (int64_t)h.pairs[1];
     T.n_near_src = (int64_t)h.pairs[2];
@@ -1254,7 +1259,7 @@ fss_status tree_build(fss_ctx *ctx, const double *x, const double *y, const doub
     FSS_HIP(hipGetLastError());
     if (ctx->batch_part) {
         // the merged plan is finished by the caller, who needs the item count
-        FSS_TRY(d2h(&h, info, sizeof(h), s));
+        FSS_TRY(read_back(ctx, &h, info, sizeof(h)));
         T.n_proxy = h.n_proxy;
     } else {
         FSS_TRY(plan_finish(ctx));
@@ -1497,7 +1502,7 @@ fss_status plan_finish(fss_ctx *ctx)
     }
     FSS_TRY(proxy_records(ctx));
     BuildInfo h;
-    FSS_TRY(d2h(&h, info, sizeof(h), s));
+    FSS_TRY(read_back(ctx, &h, info, sizeof(h)));
     if (!T.batched) T.n_proxy = T.n_slot > 0 ? h.n_proxy : 0;
     if (T.n_charge > 0) {
         T.n_up_small = h.up.x;
@@ -1518,7 +1523,7 @@ static fss_status export_lists(fss_ctx *ctx, int32_t *offsets, int32_t *ids)
     DevBuf off, keys, sorted, vals, out, tmp;
     FSS_TRY(off.ensure(sizeof(int32_t) * T.nn));
     FSS_TRY(cub_exclusive_sum(tmp, T.counts.as<int32_t>(), off.as<int32_t>(), T.nn, s));
-    if (offsets) FSS_TRY(d2h(offsets, off.p, sizeof(int32_t) * T.nn, s));
+    if (offsets) FSS_TRY(read_back(ctx, offsets, off.p, sizeof(int32_t) * T.nn));
     if (!ids) return FSS_OK;
     FSS_TRY(keys.ensure(sizeof(uint32_t) * n));
     FSS_TRY(sorted.ensure(sizeof(uint32_t) * n));
@@ -1532,7 +1537,7 @@ static fss_status export_lists(fss_ctx *ctx, int32_t *offsets, int32_t *ids)
                            (uint32_t)level_size(l), keys.as<uint32_t>(), vals.as<int32_t>());
         FSS_TRY(cub_sort_pairs(tmp, keys.as<uint32_t>(), sorted.as<uint32_t>(), vals.as<int32_t>(), out.as<int32_t>(),
                                n, bits_for64((uint64_t)level_size(l)), s));
-        if (cnt > 0) FSS_TRY(d2h(ids + base, out.p, sizeof(int32_t) * cnt, s));
+        if (cnt > 0) FSS_TRY(read_back(ctx, ids + base, out.p, sizeof(int32_t) * cnt));
         base += cnt;
     }
     return FSS_OK;
@@ -1542,7 +1547,6 @@ fss_status tree_export(fss_ctx *ctx, int32_t *loc, uint8_t *found, int32_t *coun
                        int32_t *ids, int32_t *inter, double *tri_info, double *tri_xyz)
 {
     Tree &T = ctx->tree;
-    hipStream_t s = ctx->stream;
     if (!T.built) {
         set_error("tree_export before tree_build");
         return FSS_ERR_STATE;
@@ -1551,13 +1555,13 @@ fss_status tree_export(fss_ctx *ctx, int32_t *loc, uint8_t *found, int32_t *coun
         set_error("tree_export is not available for a batch");
         return FSS_ERR_STATE;
     }
-    if (loc) FSS_TRY(d2h(loc, T.loc.p, sizeof(int32_t) * T.L * T.n, s));
-    if (found) FSS_TRY(d2h(found, T.found.p, (size_t)T.L * T.n, s));
-    if (counts) FSS_TRY(d2h(counts, T.counts.p, sizeof(int32_t) * T.nn, s));
+    if (loc) FSS_TRY(read_back(ctx, loc, T.loc.p, sizeof(int32_t) * T.L * T.n));
+    if (found) FSS_TRY(read_back(ctx, found, T.found.p, (size_t)T.L * T.n));
+    if (counts) FSS_TRY(read_back(ctx, counts, T.counts.p, sizeof(int32_t) * T.nn));
     if (offsets || (ids && T.nlist > 0)) FSS_TRY(export_lists(ctx, offsets, T.nlist > 0 ? ids : nullptr));
-    if (inter && T.ninter > 0) FSS_TRY(d2h(inter, T.inter.p, sizeof(int32_t) * 7 * T.ninter, s));
-    if (tri_info) FSS_TRY(d2h(tri_info, T.d_info, sizeof(double) * 4 * T.ntri_all, s));
-    if (tri_xyz) FSS_TRY(d2h(tri_xyz, T.d_xyz, sizeof(double) * 9 * T.ntri_all, s));
+    if (inter && T.ninter > 0) FSS_TRY(read_back(ctx, inter, T.inter.p, sizeof(int32_t) * 7 * T.ninter));
+    if (tri_info) FSS_TRY(read_back(ctx, tri_info, T.d_info, sizeof(double) * 4 * T.ntri_all));
+    if (tri_xyz) FSS_TRY(read_back(ctx, tri_xyz, T.d_xyz, sizeof(double) * 9 * T.ntri_all));
     return FSS_OK;
 }
 
