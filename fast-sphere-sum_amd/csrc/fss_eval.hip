@@ -337,7 +337,7 @@ __device__ inline void write_charge(const double *M, const double *__restrict__ 
 // normalised barycentric b_j; an item that covers its whole node writes the
 // charges (lane k < P charge k), the others write partial moments
 template <typename Real, int D>
-__global__ void __launch_bounds__(256) k_upward(const int4 *__restrict__ items, int64_t nitems,
+__global__ void __launch_bounds__(256, npts<D>() <= 36 ? 4 : 3) k_upward(const int4 *__restrict__ items, int64_t nitems,
                                                const int32_t *__restrict__ recnode,
                                                const double *__restrict__ centres,
                                                const double *__restrict__ tinv,
@@ -440,32 +440,34 @@ __global__ void __launch_bounds__(256) k_upward_pair(const int4 *__restrict__ it
     }
 }
 
-// nodes with several items: one wave per node sums the partial moments (in
-// a fixed order) and lanes k < P write q_k
+// Nodes with several items: one block per node sums their partial moments, thread
+// (group, moment) every G-th of them, coalesced, the groups in order, and P threads
+// write q_k.  One wave per node with a lane per partial (strided reads, the lane sum
+// of k_upward) took 95 us at degree 7 on the level-10 grid, where a root node has
+// 1,024 partials; now 30.
 template <typename Real, int D>
-__global__ void __launch_bounds__(256) k_upward_finish(const int4 *__restrict__ multi, int64_t nmulti,
-                                                       const double *__restrict__ partial,
+__global__ void __launch_bounds__(256) k_upward_finish(const int4 *__restrict__ multi, const double *__restrict__ partial,
                                                        const double *__restrict__ vinv, int64_t p0,
                                                        typename Rec<Real>::T4 *src)
 {
-    constexpr int P = npts<D>();
-    // wave index within the block, made wave-uniform for the compiler (item
-    // and node data then come through scalar loads)
-    const int64_t wi = (int64_t)blockIdx.x * 4 + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    if (wi >= nmulti) return;
-    const int4 mn = multi[wi];
-    const int lane = threadIdx.x & 63;
-    double M[P];
-#pragma unroll
-    for (int k = 0; k < P; k++) M[k] = 0.0;
-    for (int32_t j = mn.y + lane; j < mn.z; j += 64) {
-        const double *o = partial + (int64_t)j * P;
-#pragma unroll
-        for (int k = 0; k < P; k++) M[k] += o[k];
+    constexpr int P = npts<D>(), G = 256 / P;
+    __shared__ double sum[G * P], M[P];
+    const int4 mn = multi[blockIdx.x];
+    const int g = threadIdx.x / P, k = threadIdx.x - g * P;
+    if (g < G) {
+        double a = 0.0;
+#pragma unroll 4
+        for (int32_t j = mn.y + g; j < mn.z; j += G) a += partial[(int64_t)j * P + k];
+        sum[threadIdx.x] = a;
     }
-    __shared__ double lds_up[4][UP_LDS<P, 64>];
-    group_sum<P, 64>(M, lds_up[threadIdx.x >> 6]);
-    if (lane < P) write_charge<Real, D>(M, vinv, p0, mn.x, lane, src);
+    __syncthreads();
+    if (g == 0) {
+        double a = 0.0;
+        for (int h = 0; h < min(G, mn.z - mn.y); h++) a += sum[h * P + k];
+        M[k] = a;
+    }
+    __syncthreads();
+    if (g == 0) write_charge<Real, D>(M, vinv, p0, mn.x, k, src);
 }
 
 // ------------------------------------------------------------------
@@ -672,40 +674,45 @@ __device__ inline void near_tile_pairwise(const float4 *xt, const float4 &s, Acc
 // interchanges are applied while summing (perm: the composed ipiv sequence)
 // ------------------------------------------------------------------
 struct SolveArgs {
-    const ProxySlot *__restrict__ slots;
+    const ProxySlot *slots;
     int64_t nslot;
-    const double *__restrict__ phi;
-    const double *__restrict__ lu;
-    const int32_t *__restrict__ perm;
+    const double *phi, *lu;
+    const int32_t *perm;
     double *alpha;
     int blocks; // of 64 threads that k_near gives to it, a multiple of 8
 };
-template <int D> __device__ inline void solve_slot(const SolveArgs &a, int64_t i)
+// (k_solve takes its pointers one by one: from a struct, without restrict, the
+// factors go through vector registers, 254 of them and 162 us in place of 115 at
+// degree 7)
+template <int D>
+__device__ inline void solve_slot(int64_t i, const ProxySlot *__restrict__ slots, int64_t nslot,
+                                  const double *__restrict__ phi, const double *__restrict__ lu,
+                                  const int32_t *__restrict__ perm, double *__restrict__ alpha)
 {
     constexpr int P = npts<D>();
-    if (i >= 3 * a.nslot) return;
+    if (i >= 3 * nslot) return;
     int64_t q = i / 3;
     int c = (int)(i % 3);
-    ProxySlot sl = a.slots[q];
+    ProxySlot sl = slots[q];
     double b[P];
 #pragma unroll
     for (int k = 0; k < P; k++) b[k] = 0.0;
     for (int part = sl.part_beg; part < sl.part_end; part++) {
-        const double *o = a.phi + (int64_t)part * 3 * P + c * P;
+        const double *o = phi + (int64_t)part * 3 * P + c * P;
 #pragma unroll
-        for (int k = 0; k < P; k++) b[k] += o[a.perm[k]];
+        for (int k = 0; k < P; k++) b[k] += o[perm[k]];
     }
 #pragma unroll
     for (int k = 0; k < P; k++)
 #pragma unroll
-        for (int r = k + 1; r < P; r++) b[r] = b[r] - b[k] * a.lu[r + k * P];
+        for (int r = k + 1; r < P; r++) b[r] = b[r] - b[k] * lu[r + k * P];
 #pragma unroll
     for (int k = P - 1; k >= 0; k--) {
-        b[k] = b[k] / a.lu[k + k * P];
+        b[k] = b[k] / lu[k + k * P];
 #pragma unroll
-        for (int r = 0; r < k; r++) b[r] = b[r] - b[k] * a.lu[r + k * P];
+        for (int r = 0; r < k; r++) b[r] = b[r] - b[k] * lu[r + k * P];
     }
-    double *o = a.alpha + q * 3 * P + c * P;
+    double *o = alpha + q * 3 * P + c * P;
 #pragma unroll
     for (int k = 0; k < P; k++) o[k] = b[k];
 }
@@ -740,7 +747,8 @@ __global__ void __launch_bounds__(64, sizeof(Real) == 4 && R == 2 ? 8 : 4) k_nea
     stamp_start(ts, Timing::MAIN);
     if constexpr (DS > 0) {
         if ((int)blockIdx.x < solve.blocks) {
-            solve_slot<DS>(solve, (int64_t)blockIdx.x * 64 + threadIdx.x);
+            solve_slot<DS>((int64_t)blockIdx.x * 64 + threadIdx.x, solve.slots, solve.nslot, solve.phi, solve.lu,
+                           solve.perm, solve.alpha);
             return;
         }
     }
@@ -1083,10 +1091,14 @@ __global__ void __launch_bounds__(256) k_proxy_list(const ProxyItem *__restrict_
     }
 }
 
-template <int D> __global__ void __launch_bounds__(128) k_solve(SolveArgs a, uint64_t *ts)
+template <int D>
+__global__ void __launch_bounds__(128) k_solve(const ProxySlot *__restrict__ slots, int64_t nslot,
+                                               const double *__restrict__ phi, const double *__restrict__ lu,
+                                               const int32_t *__restrict__ perm, double *__restrict__ alpha,
+                                               uint64_t *ts)
 {
     stamp_start(ts, Timing::MAIN_END);
-    solve_slot<D>(a, (int64_t)blockIdx.x * blockDim.x + threadIdx.x);
+    solve_slot<D>((int64_t)blockIdx.x * blockDim.x + threadIdx.x, slots, nslot, phi, lu, perm, alpha);
 }
 
 // ------------------------------------------------------------------
@@ -1279,8 +1291,8 @@ static fss_status upward(fss_ctx *ctx, typename Rec<Real>::T4 *src)
                            T.up_items.as<int4>() + ns, nl, T.recnode.as<int32_t>(), T.d_info,
                            T.d_tinv, ctx->d_vinv.as<double>(), p0, src, part);
     if (T.n_up_multi > 0)
-        hipLaunchKernelGGL((k_upward_finish<Real, D>), dim3((unsigned)div_up(T.n_up_multi, 4)), dim3(256), 0, s,
-                           T.up_multi.as<int4>(), T.n_up_multi, part, ctx->d_vinv.as<double>(), p0, src);
+        hipLaunchKernelGGL((k_upward_finish<Real, D>), dim3((unsigned)T.n_up_multi), dim3(256), 0, s,
+                           T.up_multi.as<int4>(), part, ctx->d_vinv.as<double>(), p0, src);
     FSS_HIP(hipGetLastError());
     return FSS_OK;
 }
@@ -1348,7 +1360,8 @@ static fss_status run_degree(fss_ctx *ctx, const fss_particles *pp, fss_velocity
         }
     const bool solve = T.n_slot > 0 && sol.blocks == 0; // not done by k_near
     if (solve)
-        hipLaunchKernelGGL((k_solve<D>), dim3((unsigned)div_up(3 * T.n_slot, 128)), dim3(128), 0, s, sol, ts);
+        hipLaunchKernelGGL((k_solve<D>), dim3((unsigned)div_up(3 * T.n_slot, 128)), dim3(128), 0, s, sol.slots, sol.nslot,
+                           sol.phi, sol.lu, sol.perm, sol.alpha, ts);
     uint64_t *first = solve ? nullptr : ts;
     if (mixed)
         hipLaunchKernelGGL((k_combine<float, D>), dim3((unsigned)div_up(p0, 256)), dim3(256), 0, s,
