@@ -139,7 +139,7 @@ def rel_errors(got, ref):
 def time_stage(torch, ctx, call, steps, warmup):
     """Host-clock time per call over `steps` calls between two
     synchronisations, and the mean near-field and far-field kernel times
-    from the HIP events the library records on its stream."""
+    from the time stamps that the library's kernels write."""
     for _ in range(warmup):
         call()
     torch.cuda.synchronize()
@@ -356,7 +356,7 @@ def run_batch(args, W, fss, torch):
                     unit="TFLOP/s", frac=achieved / PEAK_FP32_TFLOPS,
                     traffic=traffic, flops_per_launch=alg_pairs * FLOPS_PAIR_FP32,
                     note=f"compute bound (vector ALU): {alg_pairs} near pairs x {FLOPS_PAIR_FP32} flops / mean "
-                         f"k_near<float,{tile},false> duration (HIP events on the context stream); traffic: "
+                         f"k_near<float,{tile},false> duration (the kernels' time stamps); traffic: "
                          + traffic_note(tfile, key))
     cpu = None
     if not args.no_cpu:
@@ -584,7 +584,7 @@ def run_single(args, W, fss, torch):
                     flops_per_launch=units * flp,
                     note=f"compute bound (bound 'mfma' = the compute peak; this kernel runs on the vector ALU, "
                          f"no matrix instructions): {units} {what} x {flp} flops / mean {kname} duration "
-                         f"{ms:.3f} ms (HIP events on the context stream); traffic: ")
+                         f"{ms:.3f} ms (the kernels' time stamps); traffic: ")
     roofline["traffic"], tfile = traffic_from_profiles(kfile, W["name"], key)
     roofline["note"] += traffic_note(tfile, key)
 
