@@ -663,8 +663,12 @@ static DirectPlan direct_plan(int64_t n, int64_t m, bool mixed)
     return p;
 }
 
-// Workspace of the sum over unordered pairs, within FSS_DIRECT_SCRATCH_BYTES.
-constexpr int64_t SYM_BYTES = (int64_t)30 << 20;
+// Workspace of the sum over unordered pairs, within the allocation-free variant's
+// scratch.  With 30 MiB 20,011 particles have room for equal runs only (187 us,
+// now 165) and 100,003 take 10 slabs (3,904 us, now 3 and 3,730); 126 MiB gave 0.5
+// to 4 % more.
+constexpr int64_t DIRECT_SCRATCH = (int64_t)64 << 20, SYM_BYTES = (int64_t)62 << 20;
+static_assert(DIRECT_SCRATCH >= (int64_t)FSS_DIRECT_SCRATCH_BYTES, "records of the largest sum");
 
 // Targets per lane of the sum over unordered pairs, or 0 where k_direct does
 // the call: chosen targets and mixed precision (whose FP32 partial sums keep
@@ -672,13 +676,14 @@ constexpr int64_t SYM_BYTES = (int64_t)30 << 20;
 // and more than one row's column sums have room for.  Us a call, k_direct
 // against two / four targets a lane: N = 2,562 14.3, 17.3 / 22.1; 3,500 21.7, 18.6 /
 // 23.6; 10,242 75.3, 59.8 / 60.5; 15,000 146.7, 105.9 / 116.7; 20,011 233.4, 197.1 /
-// 186.3; 40,009 824, 705 / 630; 100,003 5,045, 4,361 / 3,902.
+// 186.3; 40,009 824, 705 / 630; 100,003 5,045, 4,361 / 3,902 (with 30 MiB); 655,362
+// 228,600, - / 159,600.
 // Outputs that overlap the inputs stay with k_direct, whose last kernel alone
 // writes them.
 static int sym_targets(const fss_particles *p, const fss_velocity *o, const int64_t *idx, bool mixed)
 {
     const int64_t n = p->n;
-    if (idx || mixed || n < 3300 || n > 500000) return 0;
+    if (idx || mixed || n < 3300 || n > 1900000) return 0;
     for (const double *in : {p->x, p->y, p->z, p->vort, p->area})
         for (const double *out : {o->u, o->v, o->w, o->dvort})
             if (std::less<const double *>()(in, out + n) && std::less<const double *>()(out, in + n)) return 0;
@@ -816,7 +821,7 @@ fss_status velocity_direct(fss_ctx *ctx, const fss_particles *p, const int64_t *
 // that GPU's copy, so calls that overlap on one GPU (two streams, two threads)
 // race; calls in one stream order are safe.  Nothing in it needs clearing: a
 // call reads only what it wrote.
-static __device__ __align__(256) unsigned char scratch[FSS_DIRECT_SCRATCH_BYTES];
+static __device__ __align__(256) unsigned char scratch[DIRECT_SCRATCH];
 
 constexpr int SCRATCH_MAX_DEVICES = 64;
 static std::mutex g_scratch_mu;
@@ -854,7 +859,7 @@ fss_status velocity_direct_noalloc(fss_ctx *ctx, const fss_particles *p, fss_vel
     if (n < 1 || (size_t)n > FSS_DIRECT_SCRATCH_BYTES / rec) {
         set_error("velocity_direct_noalloc: n must be in [1, " +
                   std::to_string(FSS_DIRECT_SCRATCH_BYTES / rec) + "] in " + (mixed ? "mixed" : "FP64") +
-                  " precision (" + std::to_string(FSS_DIRECT_SCRATCH_BYTES >> 20) + " MiB of scratch), got " +
+                  " precision (" + std::to_string(FSS_DIRECT_SCRATCH_BYTES >> 20) + " MiB of records), got " +
                   std::to_string(n));
         return FSS_ERR_INVALID;
     }

@@ -403,8 +403,8 @@ fss_status proxy_records(fss_ctx *ctx);
 fss_status velocity_direct(fss_ctx *ctx, const fss_particles *p, const int64_t *idx, int64_t m,
                            fss_velocity *out, bool force_fp64, const RkNext &next = RkNext{});
 
-// allocation-free direct sum (fss_direct.hip): records packed into a
-// file-scope device array of FSS_DIRECT_SCRATCH_BYTES per GPU, whose address
+// allocation-free direct sum (fss_direct.hip): workspace in a file-scope device
+// array per GPU (FSS_DIRECT_SCRATCH_BYTES of records and more), whose address
 // direct_scratch_setup resolves once per device (that device current)
 fss_status direct_scratch_setup(int device);
 fss_status velocity_direct_noalloc(fss_ctx *ctx, const fss_particles *p, fss_velocity *out);
