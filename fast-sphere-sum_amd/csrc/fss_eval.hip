@@ -729,9 +729,10 @@ __device__ inline void solve_slot(int64_t i, const ProxySlot *__restrict__ slots
 // DS > 0: the first blocks solve the interpolants of degree DS, which need the
 // proxy values of the kernel before and are needed by the one after.  A launch
 // of their own costs the host 3.5 us and the chip a tail (5 us at degree 2 on the
-// level-8 grid, 16 for 24 instances).  Degrees above 3 keep it: their right-hand
-// sides do not fit beside the FP32 kernel's 64 registers.
-constexpr int solve_in_near(int d) { return d <= 3 ? d : 0; }
+// level-8 grid, 16 for 24 instances).  Degrees above 2 keep it: at degree 3 a
+// stage of 963,564 particles is 2 % slower without it (mixed 436 against 427 us,
+// FP64 567 against 561).
+constexpr int solve_in_near(int d) { return d <= 2 ? d : 0; }
 template <typename Real, int R, bool SPH, int DS>
 __global__ void __launch_bounds__(64, sizeof(Real) == 4 && R == 2 ? 8 : 4) k_near(const NearItem *__restrict__ items,
                                              const int32_t *__restrict__ near_src,
@@ -742,13 +743,15 @@ __global__ void __launch_bounds__(64, sizeof(Real) == 4 && R == 2 ? 8 : 4) k_nea
                                              const double *__restrict__ x,
                                              const double *__restrict__ y,
                                              const double *__restrict__ z, int64_t ostride, double *out,
-                                             SolveArgs solve, uint64_t *ts)
+                                             const ProxySlot *__restrict__ slots, int64_t nslot,
+                                             const double *__restrict__ phi, const double *__restrict__ lu,
+                                             const int32_t *__restrict__ perm, double *__restrict__ alpha,
+                                             int sblocks, uint64_t *ts)
 {
     stamp_start(ts, Timing::MAIN);
     if constexpr (DS > 0) {
-        if ((int)blockIdx.x < solve.blocks) {
-            solve_slot<DS>((int64_t)blockIdx.x * 64 + threadIdx.x, solve.slots, solve.nslot, solve.phi, solve.lu,
-                           solve.perm, solve.alpha);
+        if ((int)blockIdx.x < sblocks) {
+            solve_slot<DS>((int64_t)blockIdx.x * 64 + threadIdx.x, slots, nslot, phi, lu, perm, alpha);
             return;
         }
     }
@@ -765,7 +768,7 @@ __global__ void __launch_bounds__(64, sizeof(Real) == 4 && R == 2 ? 8 : 4) k_nea
     int32_t *lid = reinterpret_cast<int32_t *>(smem + sizeof(T4) * NCH);
     // Blocks go round-robin to the 8 XCDs: give every XCD a contiguous run of
     // items (neighbouring leaves, largely the same sources) for its own L2.
-    const int sb = DS > 0 ? solve.blocks : 0;
+    const int sb = DS > 0 ? sblocks : 0;
     const int nb = gridDim.x - sb, q8 = nb >> 3, r8 = nb & 7, xcd = blockIdx.x & 7, loc = (blockIdx.x - sb) >> 3;
     const NearItem it = items[(xcd < r8 ? xcd * (q8 + 1) : r8 * (q8 + 1) + (xcd - r8) * q8) + loc];
     const int lane = threadIdx.x;
@@ -1165,7 +1168,9 @@ __device__ inline void add_interp_wave(const double *__restrict__ tinv, const do
 // default cap of 128 VGPRs (a few spilled at degree 6-8) four waves fit per
 // SIMD, which measured faster than 159 VGPRs and three (degree 8, level-10
 // grid: 1.23 against 1.47 ms).
-template <typename Real, int D>
+// RK: with the RK4 update (rk_next); without it the kernel has the registers of the
+// velocities alone (degree 3, FP64, N = 2,000,003: 1.4 % of the stage).
+template <typename Real, int D, bool RK>
 __global__ void k_combine(const int32_t *__restrict__ recid, const int32_t *__restrict__ recnode,
                           const uint8_t *__restrict__ rinfo, const int4 *__restrict__ nrange,
                           const int32_t *__restrict__ oslot, const int32_t *__restrict__ node_slot,
@@ -1256,13 +1261,13 @@ __global__ void k_combine(const int32_t *__restrict__ recid, const int32_t *__re
         }
     }
     const double s0 = a0 * scale, s1 = a1 * scale, s2 = a2 * scale, s3 = -2 * omega * s2;
-    if (next.mode != RkNext::STEP) {
+    if (!RK || next.mode != RkNext::STEP) {
         u[id] = s0;
         v[id] = s1;
         w[id] = s2;
         dvort[id] = s3;
     }
-    rk_next(next, id, s0, s1, s2, s3);
+    if constexpr (RK) rk_next(next, id, s0, s1, s2, s3);
     stamp_end(ts);
 }
 
@@ -1336,7 +1341,8 @@ static fss_status run_degree(fss_ctx *ctx, const fss_particles *pp, fss_velocity
                            : (ctx->near_r == 2 ? k_near<double, 2, false, DS> : k_near<double, 4, false, DS>);
             hipLaunchKernelGGL(kn, gn, dim3(64), 0, s, T.near_items.as<NearItem>(),
                                T.near_src.as<int32_t>(), src, recid, T.srcnode.as<int32_t>(), (int32_t)p0,
-                               T.d_info, pp->x, pp->y, pp->z, ost, ctx->out3.as<double>(), sol, ts);
+                               T.d_info, pp->x, pp->y, pp->z, ost, ctx->out3.as<double>(), sol.slots, sol.nslot, sol.phi,
+                               sol.lu, sol.perm, sol.alpha, sol.blocks, ts);
         }
         } else {
         float4 *src = T.src32.as<float4>();
@@ -1355,7 +1361,8 @@ static fss_status run_degree(fss_ctx *ctx, const fss_particles *pp, fss_velocity
             auto kn = ctx->near_r == 4 ? k_near<float, 4, false, DS> : k_near<float, 2, false, DS>; // default 2
             hipLaunchKernelGGL(kn, gn, dim3(64), 0, s, T.near_items.as<NearItem>(),
                                T.near_src.as<int32_t>(), src, recid, T.srcnode.as<int32_t>(), (int32_t)p0,
-                               T.d_info, pp->x, pp->y, pp->z, ost, ctx->out3.as<double>(), sol, ts);
+                               T.d_info, pp->x, pp->y, pp->z, ost, ctx->out3.as<double>(), sol.slots, sol.nslot, sol.phi,
+                               sol.lu, sol.perm, sol.alpha, sol.blocks, ts);
         }
         }
     const bool solve = T.n_slot > 0 && sol.blocks == 0; // not done by k_near
@@ -1363,8 +1370,9 @@ static fss_status run_degree(fss_ctx *ctx, const fss_particles *pp, fss_velocity
         hipLaunchKernelGGL((k_solve<D>), dim3((unsigned)div_up(3 * T.n_slot, 128)), dim3(128), 0, s, sol.slots, sol.nslot,
                            sol.phi, sol.lu, sol.perm, sol.alpha, ts);
     uint64_t *first = solve ? nullptr : ts;
+    const bool rk = next.mode != RkNext::NONE;
     if (mixed)
-        hipLaunchKernelGGL((k_combine<float, D>), dim3((unsigned)div_up(p0, 256)), dim3(256), 0, s,
+        hipLaunchKernelGGL((rk ? k_combine<float, D, true> : k_combine<float, D, false>), dim3((unsigned)div_up(p0, 256)), dim3(256), 0, s,
                            recid, T.recnode.as<int32_t>(), T.rinfo.as<uint8_t>(), T.nrange.as<int4>(),
                            T.oslot.as<int32_t>(), T.node_slot.as<int32_t>(), T.nodeof.as<int32_t>(),
                            T.inv_active.as<int32_t>(), ctx->alpha.as<double>(), T.d_tinv,
@@ -1372,7 +1380,7 @@ static fss_status run_degree(fss_ctx *ctx, const fss_particles *pp, fss_velocity
                            ctx->out3.as<double>(), bltc ? 1 : 0, scale, ctx->cfg.omega, out->u, out->v, out->w,
                            out->dvort, next, first, ts);
     else
-        hipLaunchKernelGGL((k_combine<double, D>), dim3((unsigned)div_up(p0, 256)), dim3(256), 0, s,
+        hipLaunchKernelGGL((rk ? k_combine<double, D, true> : k_combine<double, D, false>), dim3((unsigned)div_up(p0, 256)), dim3(256), 0, s,
                            recid, T.recnode.as<int32_t>(), T.rinfo.as<uint8_t>(), T.nrange.as<int4>(),
                            T.oslot.as<int32_t>(), T.node_slot.as<int32_t>(), T.nodeof.as<int32_t>(),
                            T.inv_active.as<int32_t>(), ctx->alpha.as<double>(), T.d_tinv,
