@@ -77,13 +77,16 @@ __device__ inline double table_at(const SalTab &t, double x, bool u)
     return fma(fma(fma(c3, f, c2), f, 0.5 * e1), f, a.y);
 }
 
-// square root of q >= 0 from v_rsq_f64 (relative error below 1e-7) and two
-// Newton steps: within an ulp or two, without the scaling that the library's needs
-// for the smallest and largest numbers (q in [0, 4] here; 0 gives 1e-100)
+// square root of q >= 0 from v_rsq_f64 (relative error below 1e-7), one coupled
+// Newton step for the root and half its reciprocal (Goldschmidt's iteration) and
+// a last correction by the residual (Markstein 1990): within an ulp or two,
+// without the scaling that the library's needs for the smallest and largest numbers
+// (q in [0, 4] here; 0 gives 0).  Only the estimate's argument is kept off zero, by
+// a maximum that would turn a NaN into a number: a NaN in q goes through to the
+// root.
 __device__ inline double sqrt_plain(double q)
 {
-    q = fmax(q, 1e-200);
-    const double r = __builtin_amdgcn_rsq(q);
+    const double r = __builtin_amdgcn_rsq(fmax(q, 1e-200));
     double g = q * r, h = 0.5 * r;
     const double e = fma(-h, g, 0.5);
     g = fma(g, e, g);
@@ -98,12 +101,14 @@ __device__ inline double table_eval(const SalTab &t, double s)
     return table_at(t, u ? sqrt(fmax(0.0, (1.0 - s) * (1.0 + s))) : s, u);
 }
 
-// G at s = sqrt(q) / 2 from the squared distance: s^2 = q / 4, u^2 = 1 - q / 4, one
-// square root for either half of the table
+// G at s = sqrt(q) / 2 from the squared distance: s^2 = q / 4, u^2 = 1 - q / 4 (not
+// below 0 where points off the sphere are further apart than a diameter), one
+// square root for either half of the table.  A q that is no number takes the half
+// without the maximum and comes out as one.
 __device__ inline double table_eval_dist2(const SalTab &t, double q)
 {
     const bool u = q > 2.0;
-    return table_at(t, sqrt_plain(u ? fma(-0.25, q, 1.0) : 0.25 * q), u);
+    return table_at(t, sqrt_plain(u ? fmax(fma(-0.25, q, 1.0), 0.0) : 0.25 * q), u);
 }
 
 // ------------------------------------------------------------------

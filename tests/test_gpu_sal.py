@@ -358,3 +358,20 @@ def test_sal_treecode_proxy_layouts(fsslib, sal, degree, bar):
     for kind in (0, 2):
         got = ctx.sal_tree(*d, kind=kind).cpu().numpy()
         assert np.linalg.norm(got - ref) <= bar * np.linalg.norm(ref)
+
+
+@pytest.mark.parametrize("n,levels", [(700, 2), (3001, 3)])
+def test_sal_table_keeps_nan(fsslib, sal, n, levels):
+    """A particle whose position is not a number leaves no finite sum anywhere:
+    every target's separation from it is NaN, in the direct sum and in the
+    treecode (near pairs, proxy values and modified charges alike)."""
+    ctx, c, A, torch = sal
+    x, y, z = fsslib.grid_random(n, 4)
+    x[7] = np.nan
+    d = [torch.from_numpy(a).cuda() for a in (x, y, z, np.random.default_rng(n).normal(size=n), np.full(n, 4 * np.pi / n))]
+    t = fsslib.Context(tree_levels=levels, theta=0.6, degree=2, eval_mode=1, assign_mode=1, node_rule=1)
+    t.sal_set_series(c, table_points=1 << 22, A=A)
+    t.tree_build(*d[:3])
+    print(f"sal NaN n={n} levels={levels}", flush=True)
+    assert np.all(np.isnan(ctx.sal_direct(*d, kind=0).cpu().numpy()))
+    assert np.all(np.isnan(t.sal_tree(*d, kind=0).cpu().numpy()))
