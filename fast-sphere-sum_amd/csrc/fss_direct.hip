@@ -678,15 +678,23 @@ static_assert(DIRECT_SCRATCH >= (int64_t)FSS_DIRECT_SCRATCH_BYTES, "records of t
 // 23.6; 10,242 75.3, 59.8 / 60.5; 15,000 146.7, 105.9 / 116.7; 20,011 233.4, 197.1 /
 // 186.3; 40,009 824, 705 / 630; 100,003 5,045, 4,361 / 3,902 (with 30 MiB); 655,362
 // 228,600, - / 159,600.
-// Outputs that overlap the inputs stay with k_direct, whose last kernel alone
-// writes them.
+// Outputs that overlap the inputs or each other stay with k_direct, whose last
+// kernel alone writes them and reads none: a later slab reads the inputs again and
+// adds to the velocities.
 static int sym_targets(const fss_particles *p, const fss_velocity *o, const int64_t *idx, bool mixed)
 {
     const int64_t n = p->n;
     if (idx || mixed || n < 3300 || n > 1900000) return 0;
-    for (const double *in : {p->x, p->y, p->z, p->vort, p->area})
-        for (const double *out : {o->u, o->v, o->w, o->dvort})
-            if (std::less<const double *>()(in, out + n) && std::less<const double *>()(out, in + n)) return 0;
+    const double *const outs[4] = {o->u, o->v, o->w, o->dvort};
+    auto overlap = [n](const double *a, const double *b) {
+        return std::less<const double *>()(a, b + n) && std::less<const double *>()(b, a + n);
+    };
+    for (int k = 0; k < 4; k++) {
+        for (const double *in : {p->x, p->y, p->z, p->vort, p->area})
+            if (overlap(in, outs[k])) return 0;
+        for (int j = 0; j < k; j++)
+            if (overlap(outs[j], outs[k])) return 0;
+    }
     return n < 18000 ? 2 : 4;
 }
 

@@ -8,6 +8,7 @@ is the reciprocals' last bits and summation order)."""
 import numpy as np
 import pytest
 
+from conftest import rel_l2
 from test_gpu_direct_layouts import _case, _dev, _err
 
 pytestmark = pytest.mark.gpu
@@ -45,3 +46,19 @@ def test_pair_sum_outputs_over_inputs(fsslib, orc):
     d = _dev(*c)
     got = fsslib.Context().velocity_direct(*d, out=(d[3], d[0], d[1], d[2]))
     assert _err([t.cpu().numpy() for t in got], orc.rhs_direct(*c, nthreads=8)) <= 1e-12
+
+
+@pytest.mark.parametrize("n", [41023, 70001])
+def test_pair_sum_outputs_over_each_other(fsslib, orc, n):
+    """One array for two outputs (a caller without use for one of them) holds the
+    component written last, and the others are as with arrays of their own."""
+    c = _case(n, 6)
+    d = _dev(*c)
+    ctx = fsslib.Context()
+    want = [t.clone() for t in ctx.velocity_direct(*d)]
+    for pick in ((0, 1, 2, 2), (0, 0, 2, 3), (0, 1, 1, 3), (0, 1, 2, 0)):
+        buf = [want[0].new_full((n,), float("nan")) for _ in range(4)]
+        got = ctx.velocity_direct(*d, out=[buf[k] for k in pick])
+        for k in range(4):
+            last = max(j for j in range(4) if pick[j] == pick[k])
+            assert rel_l2(got[k].cpu().numpy(), want[last].cpu().numpy()) <= 1e-12, (pick, k)
