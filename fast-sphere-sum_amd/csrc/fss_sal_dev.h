@@ -63,12 +63,13 @@ inline SalTab sal_tab(const double *tab, int64_t M)
 // A lane reads its four samples as two 16-byte loads: the lanes of a wave read
 // unrelated cells, and each of their loads is a lookup of its own in the L1
 // (as four 8-byte loads the near pairs of a level-8 grid took 3.31 ms, now 2.76,
-// the proxy values 2.00, now 1.49).
+// the proxy values 2.00, now 1.49).  Outside the table the cubic of the first or
+// the last cell goes on.
 __device__ inline double table_at(const SalTab &t, double x, bool u)
 {
     typedef double pair8 __attribute__((ext_vector_type(2), aligned(8)));
     const double v = x * (u ? t.inv2 : t.inv1);
-    const double k = fmin(floor(v), (double)((u ? t.n2 : t.n1) - 2)), f = v - k;
+    const double k = fmax(0.0, fmin(floor(v), (double)((u ? t.n2 : t.n1) - 2))), f = v - k;
     const pair8 *q = reinterpret_cast<const pair8 *>(t.tab + (u ? t.n1 + 2 : 0) + (t.wide ? (int64_t)k : (int64_t)(uint32_t)k));
     const pair8 a = q[0], b = q[1];
     // the cubic with slopes (p2 - p0) / 2 and (p3 - p1) / 2

@@ -375,3 +375,25 @@ def test_sal_table_keeps_nan(fsslib, sal, n, levels):
     print(f"sal NaN n={n} levels={levels}", flush=True)
     assert np.all(np.isnan(ctx.sal_direct(*d, kind=0).cpu().numpy()))
     assert np.all(np.isnan(t.sal_tree(*d, kind=0).cpu().numpy()))
+
+
+@pytest.mark.parametrize("points", [8, 4096])
+def test_table_kernel_outside_the_table(fsslib, sal, points):
+    """Separations below 0 (rounding in a caller's own formula) continue the cubic
+    of the first cell, those above 1 take the antipode's value, and a NaN stays
+    one.  Samples of the first cells from the series: an ulp of s moves it by less
+    than 4000^2 ulps, 4e-9 of 1 and 1e-11 of the sum of 4000 terms at s = 0."""
+    _, c, A, torch = sal
+    ctx = fsslib.Context()
+    ctx.sal_set_series(c, table_points=points, A=A)
+    n1 = points // 2
+    cell = 0.75 / (n1 - 1)
+    p = ctx.sal_kernel(torch.tensor([0.0, cell, 2 * cell], dtype=torch.float64), kind=0).cpu().numpy()
+    f = np.array([-1.0, -0.25, -1e-3, -1e-9])
+    print(f"sal table outside, {points} points", flush=True)
+    got = ctx.sal_kernel(torch.tensor(list(f * cell) + [1.0, 1.5, 3.0, float("nan")], dtype=torch.float64), kind=2).cpu().numpy()
+    # Catmull-Rom with the first sample twice
+    p0, p1, p2, p3 = p[0], p[0], p[1], p[2]
+    want = p1 + 0.5 * f * ((p2 - p0) + f * ((2 * p0 - 5 * p1 + 4 * p2 - p3) + f * (3 * (p1 - p2) + p3 - p0)))
+    assert np.abs(got[:4] - want).max() <= 1e-10 * np.abs(p).max()
+    assert got[5] == got[4] and got[6] == got[4] and np.isnan(got[7])
