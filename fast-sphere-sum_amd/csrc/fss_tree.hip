@@ -1258,13 +1258,15 @@ fss_status tree_build(fss_ctx *ctx, const double *x, const double *y, const doub
     FSS_HIP(hipMemcpyAsync(T.inst.p, &one, sizeof(Instance), hipMemcpyHostToDevice, s));
     FSS_HIP(hipGetLastError());
     if (ctx->batch_part) {
-        // the merged plan is finished by the caller, who needs the item count
+        // the merged plan is finished by the caller, who needs the item count;
+        // without its source lists this one serves no evaluation, so it is not
+        // built, should a later instance be refused
         FSS_TRY(read_back(ctx, &h, info, sizeof(h)));
         T.n_proxy = h.n_proxy;
-    } else {
-        FSS_TRY(plan_finish(ctx));
-        build_scratch_trim(B);
+        return FSS_OK;
     }
+    FSS_TRY(plan_finish(ctx));
+    build_scratch_trim(B);
     T.built = true;
     return FSS_OK;
 }

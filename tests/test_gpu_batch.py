@@ -132,3 +132,25 @@ def test_autotune_picks_the_node_set(fsslib):
     c1.tree_build(*d[:3])
     for g, r in zip(got, [t.cpu().numpy() for t in c1.velocity_tree(*d)]):
         np.testing.assert_array_equal(g, r)
+
+
+def test_refused_batch_leaves_no_tree(fsslib):
+    """A batch refused at its second instance leaves no half-built plan of the
+    first behind: calls on it are refused until the next build, which works."""
+    import torch
+    x, y, z = fsslib.grid_random(3000, 5)
+    d = [torch.from_numpy(a).cuda() for a in (x, y, z, np.sin(3 * x), np.full(3000, 4 * np.pi / 3000))]
+    ctx = fsslib.Context(tree_levels=4, eval_mode=1, assign_mode=1, node_rule=1)
+    with pytest.raises(fsslib.FssError):
+        ctx.batch_build(*d[:3], [3000, 0])
+    with pytest.raises(fsslib.FssError):
+        ctx.stats()
+    with pytest.raises(fsslib.FssError):
+        ctx.velocity_tree(*d)
+    with pytest.raises(fsslib.FssError):
+        ctx.rk4_step(*d, 0.01, use_tree=True)
+    with pytest.raises(fsslib.FssError):
+        ctx.sal_tree(*d, kind=2)
+    ctx.batch_build(*d[:3], [2000, 1000])
+    got = ctx.velocity_tree(*d)
+    assert all(bool(torch.isfinite(t).all()) for t in got)
