@@ -110,15 +110,21 @@ fss_status autotune(fss_ctx *ctx, const fss_particles *pp, const fss_tune_point 
 {
     if (ncand < 1 || m < 1 || reps < 1 || !(max_rel_l2 > 0))
         return set_error("autotune: need candidates, targets, reps >= 1 and a positive bar"), FSS_ERR_INVALID;
+    const int64_t n = pp->n;
     for (int k = 0; k < ncand; k++) {
         const fss_tune_point &c = cand[k];
         if (c.degree < 1 || c.degree > FSS_MAX_DEGREE || !(c.theta > 0) || c.tree_levels < 1 ||
             c.tree_levels > 13 || c.many_count < 0 || (c.near_tile != 0 && c.near_tile != 2 && c.near_tile != 4) ||
             c.node_rule < -1 || c.node_rule > FSS_NODES_WARP_BLEND || !(c.theta_decay >= 0 && c.theta_decay <= 1))
             return set_error("autotune: candidate " + std::to_string(k) + " is out of range"), FSS_ERR_INVALID;
+        // what tree_build refuses before it gives the present tree up: found only
+        // there, a tree of the candidate before would stay with the kept degree
+        if (n > (int64_t)INT32_MAX || c.tree_levels * n > (int64_t)INT32_MAX)
+            return set_error("autotune: candidate " + std::to_string(k) +
+                             ": particle count out of range for 32-bit list offsets"),
+                   FSS_ERR_INVALID;
     }
     hipStream_t s = ctx->stream;
-    const int64_t n = pp->n;
     // FP64 direct sum at the targets: the reference of every candidate
     DevBuf ref, out, take;
     FSS_TRY(ref.ensure(sizeof(double) * 4 * m));

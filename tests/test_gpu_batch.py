@@ -154,3 +154,24 @@ def test_refused_batch_leaves_no_tree(fsslib):
     ctx.batch_build(*d[:3], [2000, 1000])
     got = ctx.velocity_tree(*d)
     assert all(bool(torch.isfinite(t).all()) for t in got)
+
+
+def test_autotune_refuses_a_candidate_before_it_builds(fsslib):
+    """A depth at which tree_build refuses the particles (levels x n beyond 32 bits)
+    is refused before any candidate is built, and the tree that was there still
+    serves."""
+    import torch
+    x, y, z = fsslib.grid_random(3000, 5)
+    d = [torch.from_numpy(a).cuda() for a in (x, y, z, np.sin(3 * x), np.full(3000, 4 * np.pi / 3000))]
+    ctx = fsslib.Context(tree_levels=4, degree=3, eval_mode=1, assign_mode=1, node_rule=1)
+    ctx.tree_build(*d[:3])
+    want = [t.clone() for t in ctx.velocity_tree(*d)]
+    n = 2 ** 31 // 13 + 1
+    big = torch.zeros(n, dtype=torch.float64, device="cuda")
+    cands = [dict(degree=2, theta=0.7, tree_levels=12, many_count=10), dict(degree=2, theta=0.7, tree_levels=13, many_count=10)]
+    with pytest.raises(fsslib.FssError) as e:
+        ctx.autotune(*[big] * 5, cands, torch.zeros(1, dtype=torch.int64), 1e-6, reps=1)
+    assert e.value.status == 1 and "candidate 1" in str(e.value)
+    assert ctx.stats().n == 3000
+    for g, w in zip(ctx.velocity_tree(*d), want):
+        np.testing.assert_array_equal(g.cpu().numpy(), w.cpu().numpy())
