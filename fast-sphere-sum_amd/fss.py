@@ -335,9 +335,11 @@ class Context:
     def _out(self, m, out=None):
         import torch
         if out is None:
-            out = torch.empty((4, m), dtype=torch.float64, device=self.device).unbind(0)
-        for t in out:
-            assert t.numel() == m and t.dtype == torch.float64 and t.is_contiguous()
+            # four tensors: views of one would share its storage and its autograd version
+            out = [torch.empty(m, dtype=torch.float64, device=self.device) for _ in range(4)]
+        else:
+            for t in out:
+                assert t.numel() == m and t.dtype == torch.float64 and t.is_contiguous()
         return out, Velocity(*(t.data_ptr() for t in out))
 
     def tree_build(self, x, y, z):
