@@ -335,7 +335,10 @@ fss_status timing_read(fss_ctx *ctx, int64_t first, int64_t count, double *stage
 {
     Timing &t = ctx->timing;
     std::vector<uint64_t> h((size_t)count * Timing::SLOT);
-    if (t.stream != ctx->stream) FSS_HIP(hipDeviceSynchronize()); // the calls ran on another stream
+    if (t.streams || t.stream != ctx->stream) {
+        FSS_HIP(hipSetDevice(ctx->cfg.device));
+        FSS_HIP(hipDeviceSynchronize());
+    }
     FSS_HIP(hipMemcpyAsync(h.data(), t.stamps.as<uint64_t>() + first * Timing::SLOT, sizeof(uint64_t) * h.size(),
                            hipMemcpyDeviceToHost, ctx->stream));
     FSS_HIP(hipStreamSynchronize(ctx->stream));

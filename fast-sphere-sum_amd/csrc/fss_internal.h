@@ -290,18 +290,21 @@ struct Timing {
     int cur = -1;       // slot of the current call
     bool valid = false;
     hipStream_t stream = nullptr; // of the last timed call
+    bool streams = false; // the window's calls ran on more than one stream
     uint64_t *slot() const { return stamps.as<uint64_t>() + (int64_t)cur * SLOT; }
 };
 
 // begin a timed call: picks the next ring slot
 inline void timing_begin(Timing &t, hipStream_t s)
 {
+    t.streams = t.calls > 0 && (t.streams || t.stream != s);
     t.stream = s;
     t.cur = (int)(t.calls % Timing::RING);
     t.calls++;
     t.have[t.cur] = 0;
 }
-// a stage's milliseconds: total, main kernel, far kernel (0 without one).  Waits for the stream.
+// a stage's milliseconds: total, main kernel, far kernel (0 without one).  Waits for
+// the context's stream, or for the device where calls ran on another.
 fss_status timing_read(fss_ctx *ctx, int64_t first, int64_t count, double *stage, double *main, double *far);
 
 // Time stamps by the kernels themselves (ts null: none).  The first block of a
