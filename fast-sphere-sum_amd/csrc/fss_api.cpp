@@ -690,7 +690,7 @@ fss_status fss_last_timing(fss_ctx *ctx, double *stage_ms, double *main_ms)
 {
     if (!ctx) return set_error("null context"), FSS_ERR_INVALID;
     if (!ctx->timing.valid || ctx->timing.cur < 0) return set_error("no timed call yet"), FSS_ERR_STATE;
-    return timing_read(ctx, ctx->timing.cur, 1, stage_ms, main_ms, nullptr);
+    FSS_GUARD(return timing_read(ctx, ctx->timing.cur, 1, stage_ms, main_ms, nullptr);)
 }
 
 fss_status fss_sal_set_series(fss_ctx *ctx, const double *c, int nmax, int64_t table_points, double A)
@@ -792,9 +792,9 @@ fss_status fss_timing_mean(fss_ctx *ctx, int64_t *calls, double *stage_ms, doubl
     Timing &t = ctx->timing;
     if (!t.valid || t.calls < 1) return set_error("no timed call yet"), FSS_ERR_STATE;
     if (t.calls > Timing::RING)
-        return set_error("more timed calls than event slots; reset more often"), FSS_ERR_STATE;
+        return set_error("more timed calls than slots; reset more often"), FSS_ERR_STATE;
     if (calls) *calls = t.calls;
-    return timing_read(ctx, 0, t.calls, stage_ms, main_ms, nullptr);
+    FSS_GUARD(return timing_read(ctx, 0, t.calls, stage_ms, main_ms, nullptr);)
 }
 
 fss_status fss_timing_far_mean(fss_ctx *ctx, double *far_ms)
@@ -803,8 +803,8 @@ fss_status fss_timing_far_mean(fss_ctx *ctx, double *far_ms)
     Timing &t = ctx->timing;
     if (!t.valid || t.calls < 1) return set_error("no timed call yet"), FSS_ERR_STATE;
     if (t.calls > Timing::RING)
-        return set_error("more timed calls than event slots; reset more often"), FSS_ERR_STATE;
-    return timing_read(ctx, 0, t.calls, nullptr, nullptr, far_ms);
+        return set_error("more timed calls than slots; reset more often"), FSS_ERR_STATE;
+    FSS_GUARD(return timing_read(ctx, 0, t.calls, nullptr, nullptr, far_ms);)
 }
 
 } // extern "C"

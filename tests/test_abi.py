@@ -64,3 +64,16 @@ def test_host_grid_and_field_entry_points(fsslib):
     area = np.full(500, 4 * np.pi / 500)
     v = fsslib.gauss_vortices(xr, yr, zr, area, 6, 2.0, 0.05, 0.3, seed=2)
     assert abs((v * area).sum()) < 1e-12  # mean removed
+
+
+def test_entries_that_use_containers_are_guarded():
+    """No exception crosses the ABI: an entry point whose work takes host memory
+    from a container (the tree, the tuners, the read-back of the stage times, ...)
+    runs it in FSS_GUARD."""
+    src = open(os.path.join(ROOT, "fast-sphere-sum_amd", "csrc", "fss_api.cpp")).read()
+    bodies = re.findall(r"^fss_status (fss_\w+)\([^{]*\)\n\{\n(.*?)^\}", src, flags=re.S | re.M)
+    assert len(bodies) > 20
+    work = r"\b(timing_read|tree_build|batch_build|tree_export|autotune\w*|sal_mlp_train|sal_mlp_grad)\("
+    found = [n for n, b in bodies if re.search(work, b)]
+    assert {"fss_last_timing", "fss_timing_mean", "fss_timing_far_mean", "fss_tree_build"} <= set(found)
+    assert [n for n, b in bodies if re.search(work, b) and "FSS_GUARD(" not in b] == []
