@@ -1062,10 +1062,13 @@ fss_status tree_build(fss_ctx *ctx, const double *x, const double *y, const doub
     // ---- traversal ----
     // Capacities: what an earlier build on this context held, at least an
     // estimate of the interactions from the acceptance criterion (about 30 / theta^2
-    // per occupied node with one theta, twice that with a tightened one).
+    // per occupied node with one theta, twice that with a tightened one), and never
+    // more than there can be: a pair of occupied nodes comes up once, to be
+    // emitted or split in four.
     BuildInfo h;
     {
-        const double est = 60.0 / (cfg.theta * cfg.theta) * (double)std::min<int64_t>(T.nn, (int64_t)L * n);
+        const double occupied = (double)std::min<int64_t>(T.nn, (int64_t)L * n);
+        const double est = std::min(60.0 / (cfg.theta * cfg.theta) * occupied, 4.0 * occupied * occupied);
         int64_t cap = (int64_t)std::min(est, 16777216.0);
         cap = std::max<int64_t>(cap, 1 << 16);
         int64_t capI = std::max<int64_t>(cap, (int64_t)(T.inter.bytes / (7 * sizeof(int32_t))));
