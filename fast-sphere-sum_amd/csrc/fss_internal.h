@@ -237,6 +237,7 @@ struct Geo {
     int levels = 0;
     DevBuf xyz;  // 9 doubles per triangle (vertex coordinates, tree_tri_verts order)
     DevBuf info; // 4 doubles per triangle (centre, radius)
+    // of the nodes, levels 0 .. levels-2
     DevBuf tinv; // 9 doubles: rows r_m with barycentric c_m = r_m . p
     DevBuf aux;  // double2: norm of the centre, arc radius of the cap
 };

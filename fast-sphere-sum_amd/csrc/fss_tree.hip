@@ -926,18 +926,20 @@ void build_scratch_trim(BuildScratch &B)
 
 // Triangles of levels 0 .. levels-1: fixed by the depth alone (the sphere has
 // radius 1), and the triangles of a shallower tree are the first ones of a
-// deeper, so a context computes them once for its deepest tree.
+// deeper, so a context computes them once for its deepest tree.  Matrices and caps
+// are of the nodes, which end a level earlier (on all levels they were 88 bytes a
+// triangle in place of 22: 1.85 GB at 10 levels).
 static fss_status geo_ensure(fss_ctx *ctx, int levels)
 {
     Geo &G = ctx->geo;
     hipStream_t s = ctx->stream;
     if (G.levels >= levels) return FSS_OK;
     G.levels = 0;
-    const int64_t nt = level_offset(levels);
+    const int64_t nt = level_offset(levels), nn = level_offset(levels - 1);
     FSS_TRY(G.xyz.ensure(sizeof(double) * 9 * nt));
     FSS_TRY(G.info.ensure(sizeof(double) * 4 * nt));
-    FSS_TRY(G.tinv.ensure(sizeof(double) * 9 * nt));
-    FSS_TRY(G.aux.ensure(sizeof(double2) * nt));
+    FSS_TRY(G.tinv.ensure(sizeof(double) * 9 * nn));
+    FSS_TRY(G.aux.ensure(sizeof(double2) * nn));
     const double radius = ctx->cfg.radius;
     hipLaunchKernelGGL(k_geom_level0, dim3(1), dim3(64), 0, s, G.xyz.as<double>(), G.info.as<double>(), radius);
     for (int l = 0; l + 1 < levels; l++) {
@@ -945,9 +947,9 @@ static fss_status geo_ensure(fss_ctx *ctx, int levels)
         hipLaunchKernelGGL(k_geom_children, dim3((unsigned)div_up(np, 256)), dim3(256), 0, s, G.xyz.as<double>(),
                            G.info.as<double>(), level_offset(l), level_offset(l + 1), np, radius);
     }
-    hipLaunchKernelGGL(k_tinv, dim3((unsigned)div_up(nt, 256)), dim3(256), 0, s, G.xyz.as<double>(), nt,
+    hipLaunchKernelGGL(k_tinv, dim3((unsigned)div_up(nn, 256)), dim3(256), 0, s, G.xyz.as<double>(), nn,
                        G.tinv.as<double>());
-    hipLaunchKernelGGL(k_geo_aux, dim3((unsigned)div_up(nt, 256)), dim3(256), 0, s, G.info.as<double>(), nt,
+    hipLaunchKernelGGL(k_geo_aux, dim3((unsigned)div_up(nn, 256)), dim3(256), 0, s, G.info.as<double>(), nn,
                        G.aux.as<double2>());
     FSS_HIP(hipGetLastError());
     G.levels = levels;

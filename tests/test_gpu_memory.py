@@ -26,3 +26,13 @@ def test_lists_are_sized_by_the_pairs_there_can_be(fsslib):
     ctx, held = _held(fsslib, _case(100), 6, theta=0.05)
     print(f"held {held / 1e6:.0f} MB for {ctx.stats().n_interactions} interactions", flush=True)
     assert held <= 200e6
+
+
+def test_inverse_matrices_for_nodes_only(fsslib):
+    """Triangles go one level deeper than the nodes: 104 bytes each of those, and per
+    node the inverse matrix, cap, proxies, records and ranges (308 bytes at degree 1)."""
+    L = 10
+    ctx, held = _held(fsslib, _case(1000), L, degree=1, theta=0.7)
+    nodes, tris = [20 * (4 ** k - 1) // 3 for k in (L, L + 1)]
+    print(f"held {held / 1e9:.2f} GB", flush=True)
+    assert held <= 1.1 * (104 * tris + 308 * nodes)
