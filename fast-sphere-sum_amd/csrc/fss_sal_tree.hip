@@ -20,7 +20,9 @@ namespace fss {
 
 namespace {
 
-constexpr int NCH_S = 128; // 4.6 KiB a one-wave block: eight waves per SIMD
+// sources staged at a time: 4.6 KiB a one-wave block for the table, eight waves per
+// SIMD in place of four
+constexpr int sal_chunk_size(int kind) { return kind == 2 ? 256 : 128; }
 
 template <int D> constexpr int npts_s() { return (D + 1) * (D + 2) / 2; }
 
@@ -77,8 +79,12 @@ __device__ inline void sal_chunk(const KernelArgs &ka, const double4 *xt, const 
 // 7: 9.97 / 10.63 / 12.61 / 9.63).  Contiguous runs of items per XCD are slower (6.1
 // against 4.3 ms), and so are two lanes sharing each window of the table (half the
 // loads' lines, but the exchange costs more: 4.0 ms).
-constexpr int SAL_NEAR_R = 4;
-constexpr int sal_proxy_r(int pp) { return pp <= 10 ? pp : pp / 3; }
+// The Clenshaw series is arithmetic alone, and the targets that fill up a lane's
+// count cost as much as others: one a lane (200,003 particles, 6 levels, 65 terms,
+// degree 1 / 3 / 5: 8.9 / 21.4 / 59.0 ms; with the table's counts and chunks 10.6 / 23.7 /
+// 69.4).
+constexpr int sal_near_r(int kind) { return kind == 2 ? 1 : 4; }
+constexpr int sal_proxy_r(int kind, int pp) { return kind == 2 ? 1 : pp <= 10 ? pp : pp / 3; }
 
 // near field: one wave per near item, R targets per lane and phase; the
 // item's source list (the self ranges too: j = i is part of the sum) staged in
@@ -89,6 +95,7 @@ __global__ void __launch_bounds__(64) k_sal_near(const NearItem *__restrict__ it
                                                  const double4 *__restrict__ src, KernelArgs ka, double *out)
 {
     stamp_start(ka.ts_near, Timing::MAIN);
+    constexpr int NCH_S = sal_chunk_size(KIND);
     __shared__ double4 lds[NCH_S];
     __shared__ double red[64 * R];
     const NearItem it = items[blockIdx.x];
@@ -138,6 +145,7 @@ __global__ void __launch_bounds__(64) k_sal_proxy(const ProxyItem *__restrict__ 
     stamp_start(ka.ts_proxy, Timing::MAIN);
     constexpr int PP = npts_s<D>();
     constexpr int T = (PP + R - 1) / R, P = 64 / T;
+    constexpr int NCH_S = sal_chunk_size(KIND);
     __shared__ double4 lds[NCH_S];
     __shared__ double red[64 * R];
     const int64_t item = blockIdx.x;
@@ -456,9 +464,9 @@ template <int KIND, int D> fss_status run(fss_ctx *ctx, const KernelArgs &ka, do
                                T.proxy_items.as<ProxyItem>(), T.n_proxy, T.far_off.as<int64_t>(),
                                T.far_src.as<int32_t>(), src, p0, ka, ctx->phi.as<double>());
     } else {
-        constexpr int RF = sal_proxy_r(npts_s<D>());
+        constexpr int RN = sal_near_r(KIND), RF = sal_proxy_r(KIND, npts_s<D>());
         if (T.n_near > 0)
-            hipLaunchKernelGGL((k_sal_near<KIND, SAL_NEAR_R>), dim3((unsigned)T.n_near), dim3(64), 0, s,
+            hipLaunchKernelGGL((k_sal_near<KIND, RN>), dim3((unsigned)T.n_near), dim3(64), 0, s,
                                T.near_items.as<NearItem>(), T.near_src.as<int32_t>(), src, ka, ctx->out3.as<double>());
         if (T.n_proxy > 0)
             hipLaunchKernelGGL((k_sal_proxy<KIND, D, RF>), dim3((unsigned)T.n_proxy), dim3(64), 0, s,

@@ -397,3 +397,19 @@ def test_table_kernel_outside_the_table(fsslib, sal, points):
     want = p1 + 0.5 * f * ((p2 - p0) + f * ((2 * p0 - 5 * p1 + 4 * p2 - p3) + f * (3 * (p1 - p2) + p3 - p0)))
     assert np.abs(got[:4] - want).max() <= 1e-10 * np.abs(p).max()
     assert got[5] == got[4] and got[6] == got[4] and np.isnan(got[7])
+
+
+@pytest.mark.parametrize("n,levels", [(5, 1), (30, 2), (257, 2), (1280, 1), (3001, 3)])
+def test_sal_treecode_series_near_layouts(fsslib, sal, n, levels):
+    """The series kernel takes one target a lane: as above, against the table's
+    direct sum (the two kernels agree to 1e-8 of max(|G|, 1); n of them against a
+    sum that grows like its root)."""
+    ctx, c, A, torch = sal
+    x, y, z = fsslib.grid_random(n, 3)
+    d = [torch.from_numpy(a).cuda() for a in (x, y, z, np.random.default_rng(n).normal(size=n), np.full(n, 4 * np.pi / n))]
+    t = fsslib.Context(tree_levels=levels, theta=1e-6, degree=2, eval_mode=1, assign_mode=1, node_rule=1, many_count=1)
+    t.sal_set_series(c, table_points=1 << 22, A=A)
+    t.tree_build(*d[:3])
+    print(f"sal series near n={n} levels={levels}", flush=True)
+    got, ref = t.sal_tree(*d, kind=2).cpu().numpy(), ctx.sal_direct(*d, kind=0).cpu().numpy()
+    assert np.linalg.norm(got - ref) <= 1e-6 * np.linalg.norm(ref)
