@@ -73,3 +73,26 @@ def test_direct_coincident_points(fsslib, orc, n):
     assert _err([g[keep] for g in got], [r[keep] for r in ref]) <= 1e-12
     for g, r in zip(got[:3], ref[:3]):
         assert np.isfinite(g[[i, j]]).tolist() == np.isfinite(r[[i, j]]).tolist()
+
+
+@pytest.mark.parametrize("n,precision,bar", [(33, 0, 1e-12), (47, 0, 1e-12), (300, 1, 1e-6), (513, 1, 1e-6), (767, 1, 1e-6)])
+def test_direct_groups_of_few_tiles_match_oracle(fsslib, orc, n, precision, bar):
+    """Two or three tiles a target group: a block per group."""
+    c = _case(n, 5)
+    print(f"direct few tiles n={n} precision={precision}", flush=True)
+    ctx = fsslib.Context(precision=precision)
+    ref = orc.rhs_direct(*c, nthreads=8)
+    for call in (ctx.velocity_direct, ctx.velocity_direct_noalloc):
+        assert _err([t.cpu().numpy() for t in call(*_dev(*c))], ref) <= bar
+
+
+@pytest.mark.parametrize("n,m", [(40, 40003), (40, 140001), (200, 400001)])
+def test_direct_many_targets_of_few_tiles_match_oracle(fsslib, orc, n, m):
+    """Few sources and more target groups than blocks: long and short runs over
+    groups of three or four tiles."""
+    import torch
+    c = _case(n, 2)
+    idx = np.random.default_rng(7).integers(0, n, m)
+    print(f"direct targets few tiles n={n} m={m}", flush=True)
+    got = [t.cpu().numpy() for t in fsslib.Context().velocity_direct_targets(*_dev(*c), torch.from_numpy(idx))]
+    assert _err(got, [r[idx] for r in orc.rhs_direct(*c, nthreads=8)]) <= 1e-12
