@@ -96,3 +96,40 @@ def test_direct_many_targets_of_few_tiles_match_oracle(fsslib, orc, n, m):
     print(f"direct targets few tiles n={n} m={m}", flush=True)
     got = [t.cpu().numpy() for t in fsslib.Context().velocity_direct_targets(*_dev(*c), torch.from_numpy(idx))]
     assert _err(got, [r[idx] for r in orc.rhs_direct(*c, nthreads=8)]) <= 1e-12
+
+
+def _layout(n, m):
+    """(targets a lane, sources a wave tile) of a call with chosen targets below
+    655,361: direct_plan's choice from the measured table in the source."""
+    import os
+    import re
+    from conftest import ROOT
+    src = open(os.path.join(ROOT, "fast-sphere-sum_amd", "csrc", "fss_direct.hip")).read()
+    table = re.search(r"kDirect64\[4\] = \{(.*?)\};", src, flags=re.S).group(1)
+    lays = [[float(v) for v in r.split(",")] for r in re.findall(r"\{([^{}]*)\}", table)]
+    R, wt, _, _ = min(lays, key=lambda a: a[2] + -(-m // (64 * a[0])) * 64 * a[0] * n / a[3])
+    return int(R), int(wt)
+
+
+@pytest.mark.parametrize("n,m,layout", [(20011, 301, (1, 16)), (20011, 1501, (1, 64)), (20011, 3001, (2, 64)),
+                                        (60000, 6001, (4, 64)), (30011, 20011, (4, 64))])
+def test_direct_targets_every_layout_matches_oracle(fsslib, orc, n, m, layout):
+    import torch
+    assert _layout(n, m) == layout
+    c = _case(n, 2)
+    idx = np.random.default_rng(8).permutation(n)[:m]
+    print(f"direct targets n={n} m={m} layout={layout}", flush=True)
+    got = [t.cpu().numpy() for t in fsslib.Context().velocity_direct_targets(*_dev(*c), torch.from_numpy(idx))]
+    assert _err(got, orc.rhs_direct(*c, idx=idx, nthreads=8)) <= 1e-12
+
+
+def test_direct_whole_groups_of_many_tiles(fsslib, orc):
+    """A block per target group, which walks the tiles of 700 sources: 655,361
+    targets in FP64."""
+    import torch
+    n = 700
+    c = _case(n, 9)
+    idx = np.random.default_rng(9).integers(0, n, 655361)
+    print(f"direct whole groups n={n}", flush=True)
+    got = [t.cpu().numpy() for t in fsslib.Context().velocity_direct_targets(*_dev(*c), torch.from_numpy(idx))]
+    assert _err(got, [r[idx] for r in orc.rhs_direct(*c, nthreads=8)]) <= 1e-12

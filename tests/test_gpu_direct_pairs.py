@@ -62,3 +62,74 @@ def test_pair_sum_outputs_over_each_other(fsslib, orc, n):
         for k in range(4):
             last = max(j for j in range(4) if pick[j] == pick[k])
             assert rel_l2(got[k].cpu().numpy(), want[last].cpu().numpy()) <= 1e-12, (pick, k)
+
+
+def _slabs(n):
+    """Rows of every slab of the sum over n particles and how its units are cut
+    (one unit a run, equal runs, or long and short ones): sym_slab's arithmetic, with
+    the workspace that the source gives it."""
+    import os
+    import re
+    from conftest import ROOT
+    src = open(os.path.join(ROOT, "fast-sphere-sum_amd", "csrc", "fss_direct.hip")).read()
+    room = (int(re.search(r"SYM_BYTES = \(int64_t\)(\d+) << 20", src).group(1)) << 20) // 24
+    R = 2 if n < 18000 else 4
+    T, RT, slots, K = 256 * R, 4 * R, 768 if R == 4 else 1024, -(-n // 64)
+    rows, r0, out = -(-n // T), 0, []
+
+    def cols(r):
+        return (r - r0) * 64 * K - T * (r * (r + 1) - r0 * (r0 + 1)) // 2
+
+    while r0 < rows:
+        r1 = r0 + 1
+        while r1 < rows and cols(r1 + 1) + (r1 + 1 - r0 + slots) * T <= room:
+            r1 += 1
+        units = (r1 - r0) * K - RT * (r1 * (r1 - 1) - r0 * (r0 - 1)) // 2
+        runs = (room - cols(min(r1, rows - 1))) // T - (r1 - r0)
+        out.append((r1 - r0, "one" if units <= min(2 * slots, runs) else "equal" if runs < 2 * slots else "long"))
+        r0 = r1
+    return out
+
+
+# particles, and the slabs that they are meant to take (asserted below, so that
+# another workspace does not leave a cut untested)
+SLABS = {50021: ["equal"], 62208: ["equal"], 62209: ["equal", "one"], 70001: ["equal", "long"],
+         100003: ["equal"] * 3}
+
+
+def _sampled(orc, c, m=400):
+    idx = np.unique(np.concatenate([np.random.default_rng(1).integers(0, len(c[0]), m), [0, len(c[0]) - 1]]))
+    return idx, orc.rhs_direct(*c, idx=idx, nthreads=8)
+
+
+@pytest.mark.parametrize("n", sorted(SLABS))
+def test_pair_sum_in_slabs_matches_oracle(fsslib, orc, n):
+    """One and several slabs of rows, and each cut of a slab's units; the
+    allocation-free entry takes the same plan, so the same bits."""
+    assert [k for _, k in _slabs(n)] == SLABS[n]
+    c = _case(n, 6)
+    print(f"direct pairs n={n} slabs={_slabs(n)}", flush=True)
+    d = _dev(*c)
+    ctx = fsslib.Context()
+    got = [t.cpu().numpy() for t in ctx.velocity_direct(*d)]
+    idx, ref = _sampled(orc, c)
+    assert _err([g[idx] for g in got], ref) <= 1e-12
+    for g, h in zip(got, ctx.velocity_direct_noalloc(*d)):
+        np.testing.assert_array_equal(g, h.cpu().numpy())
+
+
+@pytest.mark.parametrize("shift", [0, 37])
+def test_pair_sum_outputs_over_inputs_in_slabs(fsslib, orc, shift):
+    """Outputs over the inputs, element by element and shifted: with several slabs
+    the inputs are read again after the first velocities are known."""
+    n = 70001
+    assert len(_slabs(n)) > 1
+    c = _case(n, 6)
+    buf = [t.new_zeros(n + shift) for t in _dev(*c[:4])]
+    d = [b[:n] for b in buf]
+    for a, b in zip(d, _dev(*c[:4])):
+        a.copy_(b)
+    out = [buf[k][shift:] for k in (3, 0, 1, 2)]
+    got = [t.cpu().numpy() for t in fsslib.Context().velocity_direct(*d, *_dev(c[4]), out=out)]
+    idx, ref = _sampled(orc, c)
+    assert _err([g[idx] for g in got], ref) <= 1e-12

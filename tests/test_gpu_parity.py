@@ -361,3 +361,26 @@ def test_tree_theta_one_keeps_touching_caps_apart(fsslib, orc):
         np.testing.assert_array_equal(ctx.tree_export()["inter"], T.interactions())
         got = _host(*ctx.velocity_tree(*d))
         assert all(np.isfinite(g).all() for g in got)
+
+
+@pytest.mark.parametrize("theta,decay", [(1.0, 0.3), (1.0, 0.2)])
+def test_traversal_beyond_its_first_lists(fsslib, orc, theta, decay):
+    """A theta tightened that much towards the root leaves most pairs to the leaves:
+    more interactions than the first list holds (60 / theta^2 a node, at least
+    65,536), so the traversal runs again with larger lists."""
+    L, n = 4, 3000
+    x, y, z = fsslib.grid_random(n, 21)
+    vort, area = np.sin(3 * x) + y, np.full(n, 4 * np.pi / n)
+    kw = dict(theta=theta, theta_decay=decay, many_count=1, degree=2, node_rule=1)
+    T = orc.Tree(x, y, z, L, assign=1, eval_mode=1, **kw)
+    first = max(60 / theta ** 2 * orc.level_offset(L), 65536)
+    assert T.ninter > first
+    print(f"traversal again: {T.ninter} interactions, first list {first:.0f}", flush=True)
+    ctx = fsslib.Context(tree_levels=L, assign_mode=1, eval_mode=1, **kw)
+    d = _dev(x, y, z, vort, area)
+    for _ in range(2):  # the second build starts with the first one's lists
+        ctx.tree_build(*d[:3])
+        assert ctx.stats().n_interactions == T.ninter
+        np.testing.assert_array_equal(ctx.tree_export()["inter"], T.interactions())
+    eu, ew = _vel_err(_host(*ctx.velocity_tree(*d)), T.rhs(vort, area, nthreads=8))
+    assert eu <= TOL_FP64 and ew <= TOL_FP64
