@@ -157,7 +157,6 @@ struct Interp {
 
 struct Tree {
     bool built = false;
-    uint64_t builds = 0;  // builds begun on this context: names the plan (see fss_ctx::graph_build)
     int L = 0;            // tree levels used (0..L-1)
     int64_t n = 0;        // particles
     int64_t nn = 0;       // nodes on levels 0..L-1
@@ -362,7 +361,6 @@ struct fss_ctx {
     int graph_tree = -1;
     int graph_near_r = -1;
     uint64_t graph_epoch = 0; // alloc_epoch() when the graph was captured
-    uint64_t graph_build = 0; // Tree::builds when the graph was captured
     bool capturing = false; // inside hipStreamBeginCapture: no event records
 };
 

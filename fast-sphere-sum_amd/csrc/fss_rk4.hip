@@ -155,13 +155,12 @@ fss_status rk4_run_graph(fss_ctx *ctx, double *x, double *y, double *z, double *
     FSS_TRY(begin(ctx, x, y, z, vort, area, n, use_tree, S));
     // the graph holds the addresses of the state and of the workspace and the
     // plan's launch shapes of its capture: any reallocation since then (a larger
-    // direct sum on this context), a rebuilt tree (a rebuild of no more particles
-    // keeps its buffers, but not the plan's sizes) or another near tile means
-    // capturing again
+    // direct sum on this context) or another near tile means capturing again; the
+    // entries that build or tune a tree drop the graph themselves
     const void *key[6] = {S.x, S.y, S.z, S.vort, S.area, nullptr};
     bool same = ctx->graph_exec && ctx->graph_n == n && ctx->graph_dt == dt &&
                 ctx->graph_tree == use_tree && ctx->graph_near_r == ctx->near_r &&
-                ctx->graph_epoch == alloc_epoch() && (!use_tree || ctx->graph_build == ctx->tree.builds);
+                ctx->graph_epoch == alloc_epoch();
     for (int i = 0; i < 5 && same; i++) same = ctx->graph_key[i] == key[i];
     int done = 0;
     if (!same) {
@@ -195,7 +194,6 @@ fss_status rk4_run_graph(fss_ctx *ctx, double *x, double *y, double *z, double *
         ctx->graph_tree = use_tree;
         ctx->graph_near_r = ctx->near_r;
         ctx->graph_epoch = alloc_epoch();
-        ctx->graph_build = ctx->tree.builds;
     }
     for (int i = done; i < steps; i++) FSS_HIP(hipGraphLaunch(ctx->graph_exec, ctx->stream));
     return finish(ctx, S, x, y, z, vort, n);

@@ -1008,7 +1008,6 @@ fss_status tree_build(fss_ctx *ctx, const double *x, const double *y, const doub
         return FSS_ERR_INVALID;
     }
     T.built = false;
-    T.builds++;
     T.L = L;
     T.n = n;
     T.nn = level_offset(L);
