@@ -673,17 +673,8 @@ __device__ inline void near_tile_pairwise(const float4 *xt, const float4 &s, Acc
 // (dgetrs, fast_rhs.h:217): one thread per (slot, component); the row
 // interchanges are applied while summing (perm: the composed ipiv sequence)
 // ------------------------------------------------------------------
-struct SolveArgs {
-    const ProxySlot *slots;
-    int64_t nslot;
-    const double *phi, *lu;
-    const int32_t *perm;
-    double *alpha;
-    int blocks; // of 64 threads that k_near gives to it, a multiple of 8
-};
-// (k_solve takes its pointers one by one: from a struct, without restrict, the
-// factors go through vector registers, 254 of them and 162 us in place of 115 at
-// degree 7)
+// (Pointers one by one: from a struct, without restrict, the factors go through
+// vector registers, 254 of them and 162 us in place of 115 at degree 7.)
 template <int D>
 __device__ inline void solve_slot(int64_t i, const ProxySlot *__restrict__ slots, int64_t nslot,
                                   const double *__restrict__ phi, const double *__restrict__ lu,
@@ -716,6 +707,7 @@ __device__ inline void solve_slot(int64_t i, const ProxySlot *__restrict__ slots
 #pragma unroll
     for (int k = 0; k < P; k++) o[k] = b[k];
 }
+
 // ------------------------------------------------------------------
 // near field (class A): direct pairs, R targets per lane
 // ------------------------------------------------------------------
@@ -1318,57 +1310,56 @@ static fss_status run_degree(fss_ctx *ctx, const fss_particles *pp, fss_velocity
     FSS_TRY(ctx->phi.ensure(sizeof(double) * 3 * p * std::max<int64_t>(1, T.n_proxy)));
     FSS_TRY(ctx->alpha.ensure(sizeof(double) * 3 * p * std::max<int64_t>(1, T.n_slot)));
     constexpr int DS = solve_in_near(D);
-    SolveArgs sol{T.proxy_slots.as<ProxySlot>(), T.n_slot, ctx->phi.as<double>(), ctx->d_lu.as<double>(),
-                  ctx->d_perm.as<int32_t>(), ctx->alpha.as<double>(), 0};
-    if (DS > 0 && T.n_near > 0) sol.blocks = 8 * (int)div_up(3 * T.n_slot, 8 * 64);
-    const dim3 gn((unsigned)(sol.blocks + T.n_near));
+    const ProxySlot *slots = T.proxy_slots.as<ProxySlot>();
+    const double *lu = ctx->d_lu.as<double>();
+    const int32_t *perm = ctx->d_perm.as<int32_t>();
+    double *phi = ctx->phi.as<double>(), *alpha = ctx->alpha.as<double>();
+    // blocks of 64 threads that k_near gives to the solves: a multiple of 8, one per XCD
+    const int sblocks = DS > 0 && T.n_near > 0 ? 8 * (int)div_up(3 * T.n_slot, 8 * 64) : 0;
+    const dim3 gn((unsigned)(sblocks + T.n_near));
     const dim3 gs((unsigned)div_up(p0, 256));
     if (!mixed) {
         double4 *src = T.src64.as<double4>();
         hipLaunchKernelGGL(k_gather64, gs, dim3(256), 0, s, pp->x, pp->y, pp->z, pp->vort, pp->area, recid, p0, src,
                            ts);
         if (bltc) FSS_TRY((upward<double, D>(ctx, src)));
-            if (T.n_proxy > 0)
-        {
+        if (T.n_proxy > 0)
             hipLaunchKernelGGL((k_proxy_list<double, D>), dim3((unsigned)div_up(T.n_proxy, 4)), dim3(256), 0, s,
                                T.proxy_items.as<ProxyItem>(), T.n_proxy, T.far_off.as<int64_t>(), T.far_src.as<int32_t>(), src,
                                T.recnode.as<int32_t>(), (const float *)nullptr, p0, T.d_info,
-                               T.proxy_xyz.as<double4>(), ctx->phi.as<double>(), ts);
-        }
-            if (T.n_near > 0) {
+                               T.proxy_xyz.as<double4>(), phi, ts);
+        if (T.n_near > 0) {
             // default 4 targets per lane; the treecode's near pairs use the sphere form
             auto kn = bltc ? (ctx->near_r == 2 ? k_near<double, 2, true, DS> : k_near<double, 4, true, DS>)
                            : (ctx->near_r == 2 ? k_near<double, 2, false, DS> : k_near<double, 4, false, DS>);
             hipLaunchKernelGGL(kn, gn, dim3(64), 0, s, T.near_items.as<NearItem>(),
                                T.near_src.as<int32_t>(), src, recid, T.srcnode.as<int32_t>(), (int32_t)p0,
-                               T.d_info, pp->x, pp->y, pp->z, ost, ctx->out3.as<double>(), sol.slots, sol.nslot, sol.phi,
-                               sol.lu, sol.perm, sol.alpha, sol.blocks, ts);
+                               T.d_info, pp->x, pp->y, pp->z, ost, ctx->out3.as<double>(), slots, T.n_slot, phi, lu, perm,
+                               alpha, sblocks, ts);
         }
-        } else {
+    } else {
         float4 *src = T.src32.as<float4>();
         float *aoff = reinterpret_cast<float *>(src + nsrc);
         hipLaunchKernelGGL(k_gather32, gs, dim3(256), 0, s, pp->x, pp->y, pp->z, pp->vort, pp->area, recid, p0,
                            T.recnode.as<int32_t>(), T.d_info, src, ts);
         if (bltc) FSS_TRY((upward<float, D>(ctx, src)));
-            if (T.n_proxy > 0)
-        {
+        if (T.n_proxy > 0)
             hipLaunchKernelGGL((k_proxy_list<float, D>), dim3((unsigned)div_up(T.n_proxy, 4)), dim3(256), 0, s,
                                T.proxy_items.as<ProxyItem>(), T.n_proxy, T.far_off.as<int64_t>(), T.far_src.as<int32_t>(), src,
                                T.recnode.as<int32_t>(), (const float *)aoff, p0, T.d_info,
-                               T.proxy_xyz.as<double4>(), ctx->phi.as<double>(), ts);
-        }
-            if (T.n_near > 0) {
+                               T.proxy_xyz.as<double4>(), phi, ts);
+        if (T.n_near > 0) {
             auto kn = ctx->near_r == 4 ? k_near<float, 4, false, DS> : k_near<float, 2, false, DS>; // default 2
             hipLaunchKernelGGL(kn, gn, dim3(64), 0, s, T.near_items.as<NearItem>(),
                                T.near_src.as<int32_t>(), src, recid, T.srcnode.as<int32_t>(), (int32_t)p0,
-                               T.d_info, pp->x, pp->y, pp->z, ost, ctx->out3.as<double>(), sol.slots, sol.nslot, sol.phi,
-                               sol.lu, sol.perm, sol.alpha, sol.blocks, ts);
+                               T.d_info, pp->x, pp->y, pp->z, ost, ctx->out3.as<double>(), slots, T.n_slot, phi, lu, perm,
+                               alpha, sblocks, ts);
         }
-        }
-    const bool solve = T.n_slot > 0 && sol.blocks == 0; // not done by k_near
+    }
+    const bool solve = T.n_slot > 0 && sblocks == 0; // not done by k_near
     if (solve)
-        hipLaunchKernelGGL((k_solve<D>), dim3((unsigned)div_up(3 * T.n_slot, 128)), dim3(128), 0, s, sol.slots, sol.nslot,
-                           sol.phi, sol.lu, sol.perm, sol.alpha, ts);
+        hipLaunchKernelGGL((k_solve<D>), dim3((unsigned)div_up(3 * T.n_slot, 128)), dim3(128), 0, s, slots, T.n_slot, phi,
+                           lu, perm, alpha, ts);
     uint64_t *first = solve ? nullptr : ts;
     const bool rk = next.mode != RkNext::NONE;
     if (mixed)
