@@ -336,7 +336,8 @@ class Context:
         import torch
         if out is None:
             # four tensors: views of one would share its storage and its autograd version
-            out = [torch.empty(m, dtype=torch.float64, device=self.device) for _ in range(4)]
+            u = torch.empty(m, dtype=torch.float64, device=self.device)
+            out = [u, torch.empty_like(u), torch.empty_like(u), torch.empty_like(u)]
         else:
             for t in out:
                 assert t.numel() == m and t.dtype == torch.float64 and t.is_contiguous()
