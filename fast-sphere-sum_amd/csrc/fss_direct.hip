@@ -12,13 +12,14 @@
 // velocities itself.
 //
 // FP64 sums of all particles are taken over unordered pairs from 3,300
-// particles on (k_direct_sym).
+// particles on (k_direct_sym); these kernels do smaller ones, chosen targets and
+// mixed precision.
 //
-// Bound by FP64 issue (17 four-cycle slots a pair at four targets a lane: 822 us
-// at N = 40,009, 1.95e12 pairs/s at about 2 GHz).  One target a lane, one block
-// per 256 targets and a reciprocal with two Newton steps per pair took 2,036
-// us there, 525 us at N = 10,242 (41 blocks on 256 CUs; now 79) and 42.6 ms for
-// 10,000 targets of N = 655,362 (now 3.4).
+// Bound by FP64 issue (17 four-cycle slots a pair at four targets a lane: 10,000
+// targets of N = 655,362 in 3.4 ms, 1.95e12 pairs/s at about 2 GHz).  One target a
+// lane, one block per 256 targets and a reciprocal with two Newton steps per pair
+// took 42.6 ms there, and for the full sums that k_direct_sym now takes 2,036 us
+// at N = 40,009 (these kernels 822) and 525 us at N = 10,242 (79).
 //
 // The self pair j == i is skipped as the reference does (rhs_eval.h:20); only
 // tiles that hold a target of the wave pay for the index test.

@@ -261,7 +261,7 @@ struct Remesh {
 
 // Page-locked host memory for the few words that a call reads back: a copy to
 // pageable memory takes 23 us with its wait, one to page-locked memory 15.  Taking
-// it costs 70 us, so contexts hand theirs on (words_take, words_give in
+// it costs 70 us, so contexts hand theirs on (words_take and ~HostWords in
 // fss_api.cpp: at most 16 wait, the others are freed).
 struct HostWords {
     static constexpr size_t BYTES = 4096;
@@ -361,7 +361,7 @@ struct fss_ctx {
     int graph_tree = -1;
     int graph_near_r = -1;
     uint64_t graph_epoch = 0; // alloc_epoch() when the graph was captured
-    bool capturing = false; // inside hipStreamBeginCapture: no event records
+    bool capturing = false; // inside hipStreamBeginCapture: no time stamps
 };
 
 namespace fss {

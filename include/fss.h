@@ -224,7 +224,7 @@ fss_status fss_velocity_direct_targets(fss_ctx *ctx, const fss_particles *p, con
  * (1,048,576 and 2,097,152); larger n fails with FSS_ERR_INVALID.  Every call
  * on one GPU shares that scratch: calls that overlap on one GPU (other
  * streams, other threads) race.  Results equal fss_velocity_direct's bit for
- * bit; no timing events are recorded. */
+ * bit; the call's time is not recorded. */
 #define FSS_DIRECT_SCRATCH_BYTES ((uint64_t)32 << 20)
 fss_status fss_velocity_direct_noalloc(fss_ctx *ctx, const fss_particles *p, fss_velocity *out);
 
