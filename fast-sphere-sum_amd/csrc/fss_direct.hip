@@ -648,15 +648,14 @@ static DirectPlan direct_plan(int64_t n, int64_t m, bool mixed)
     // 1,024 resident blocks one quad each; above, three quarters of the work in
     // one round of long runs and the rest in short ones, so that the blocks that
     // end last are short (equal runs in two rounds: 872 us at N = 40,009, in
-    // four 841).  The partials of all of them stay within 30 MiB.  A group of fewer
-    // than four tiles is a run of its own while there are as many blocks: in a quad
+    // four 841).  A group of fewer than four tiles is a run of its own: in a quad
     // with the next group's tiles it would wait for them (mixed, N = 257: a call of
-    // 24 us, now 15).
+    // 24 us, now 15).  The partials of all of them stay within 30 MiB.
     const int64_t V = div_up(p.U, 4), slots = 1024;
-    const int64_t most = ((int64_t)30 << 20) / (1536 * p.R) - p.G, few = std::min<int64_t>(2 * slots, most);
-    if (p.K < 4 && p.G <= few) {
+    const int64_t most = ((int64_t)30 << 20) / (1536 * p.R) - p.G; // no fewer than the groups
+    if (p.K < 4) {
         p.q = p.K;
-    } else if (V <= few) {
+    } else if (V <= std::min<int64_t>(2 * slots, most)) {
         p.q = 4;
     } else {
         p.B1 = slots;
