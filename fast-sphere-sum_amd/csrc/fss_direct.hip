@@ -598,7 +598,6 @@ struct DirectPlan {
     int R, wt; // targets per lane, sources per wave tile
     bool split;
     int64_t K, G, U, B1, q1, q, B;
-    size_t bytes; // partials or packed records
 };
 
 // Layout of a call.  A lane's targets share a reciprocal and each LDS read, but
@@ -617,31 +616,35 @@ struct DirectLayout {
 static const DirectLayout kDirect64[4] = {
     {1, 16, 4, 0.9e6}, {1, 64, 15, 1.5e6}, {2, 64, 20, 1.84e6}, {4, 64, 27, 1.95e6}};
 static const DirectLayout kDirect32[2] = {{1, 256, 20, 4.0e6}, {2, 256, 34, 4.4e6}};
+struct Layouts {
+    const DirectLayout *first, *last;
+    const DirectLayout *begin() const { return first; }
+    const DirectLayout *end() const { return last; }
+};
+static Layouts direct_layouts(bool mixed) { return mixed ? Layouts{kDirect32, kDirect32 + 2} : Layouts{kDirect64, kDirect64 + 4}; }
 
 static DirectPlan direct_plan(int64_t n, int64_t m, bool mixed)
 {
     DirectPlan p{};
-    const DirectLayout *lay = mixed ? kDirect32 : kDirect64;
-    const int nl = mixed ? 2 : 4;
+    const Layouts lay = direct_layouts(mixed);
     p.split = div_up(m, 256) < DIRECT_SPLIT_GROUPS;
-    int pick = nl - 1;
+    const DirectLayout *pick = lay.last - 1;
     double best = INFINITY;
-    for (int k = 0; k < nl && p.split; k++) {
-        const double t = lay[k].lone + (double)(div_up(m, 64 * lay[k].R) * 64 * lay[k].R) * (double)n / lay[k].rate;
+    for (const DirectLayout *l = lay.first; l < lay.last && p.split; l++) {
+        const double t = l->lone + (double)(div_up(m, 64 * l->R) * 64 * l->R) * (double)n / l->rate;
         if (t < best) {
             best = t;
-            pick = k;
+            pick = l;
         }
     }
-    p.R = lay[pick].R;
-    p.wt = lay[pick].wt;
+    p.R = pick->R;
+    p.wt = pick->wt;
     p.K = div_up(n, p.wt);
     p.G = div_up(m, 64 * p.R);
     p.U = p.G * p.K;
     if (!p.split) {
         p.q = p.K;
         p.B = p.G;
-        p.bytes = (mixed ? sizeof(float4) : sizeof(double4)) * (size_t)n;
         return p;
     }
     // Runs, in quads of units (one per wave): up to about two rounds of the
@@ -664,8 +667,23 @@ static DirectPlan direct_plan(int64_t n, int64_t m, bool mixed)
         p.q = 4 * div_up(rest, std::min<int64_t>(3 * slots, most - slots));
     }
     p.B = p.B1 + div_up(std::max<int64_t>(0, p.U - p.B1 * p.q1), p.q);
-    p.bytes = sizeof(double) * 3 * 64 * p.R * (size_t)(p.B + p.G);
     return p;
+}
+
+// Bytes of workspace that serve every plan of n particles and m targets or fewer of
+// either, in whatever layout: a call may be captured after an eager one that was no
+// smaller, and must not allocate then.  Partials: a run has at least four units or
+// a group's, and a plan at most 4,096 runs or one per group.
+static size_t direct_bytes(int64_t n, int64_t m, bool mixed)
+{
+    const bool whole = div_up(m, 256) >= DIRECT_SPLIT_GROUPS;
+    int64_t bytes = whole ? (mixed ? sizeof(float4) : sizeof(double4)) * n : 0;
+    const int64_t ms = std::min<int64_t>(m, 256 * (DIRECT_SPLIT_GROUPS - 1));
+    for (const DirectLayout &l : direct_layouts(mixed)) {
+        const int64_t G = div_up(ms, 64 * l.R), V = div_up(G * div_up(n, l.wt), 4);
+        bytes = std::max(bytes, std::min((int64_t)30 << 20, 1536 * l.R * (std::max(G, std::min<int64_t>(V, 4096)) + G)));
+    }
+    return (size_t)bytes;
 }
 
 // Workspace of the sum over unordered pairs, within the allocation-free variant's
@@ -683,32 +701,36 @@ static_assert(DIRECT_SCRATCH >= (int64_t)FSS_DIRECT_SCRATCH_BYTES, "records of t
 // 23.6; 10,242 75.3, 59.8 / 60.5; 15,000 146.7, 105.9 / 116.7; 20,011 233.4, 197.1 /
 // 186.3; 40,009 824, 705 / 630; 100,003 5,045, 4,361 / 3,902 (with 30 MiB); 655,362
 // 228,600, - / 159,600.
+static int sym_targets(int64_t n, const int64_t *idx, bool mixed)
+{
+    if (idx || mixed || n < 3300 || n > 1900000) return 0;
+    return n < 18000 ? 2 : 4;
+}
+
 // Outputs that overlap the inputs or each other stay with k_direct, whose last
 // kernel alone writes them and reads none: a later slab reads the inputs again and
 // adds to the velocities.
-static int sym_targets(const fss_particles *p, const fss_velocity *o, const int64_t *idx, bool mixed)
+static bool outputs_apart(const fss_particles *p, const fss_velocity *o)
 {
     const int64_t n = p->n;
-    if (idx || mixed || n < 3300 || n > 1900000) return 0;
     const double *const outs[4] = {o->u, o->v, o->w, o->dvort};
     auto overlap = [n](const double *a, const double *b) {
         return std::less<const double *>()(a, b + n) && std::less<const double *>()(b, a + n);
     };
     for (int k = 0; k < 4; k++) {
         for (const double *in : {p->x, p->y, p->z, p->vort, p->area})
-            if (overlap(in, outs[k])) return 0;
+            if (overlap(in, outs[k])) return false;
         for (int j = 0; j < k; j++)
-            if (overlap(outs[j], outs[k])) return 0;
+            if (overlap(outs[j], outs[k])) return false;
     }
-    return n < 18000 ? 2 : 4;
+    return true;
 }
 
 // The next slab from row a.r0: as many rows as leave room for their column sums
 // beside the run sums of one round of resident blocks.  Its runs: one unit each
 // up to two rounds; beyond that three quarters of the work in one round of long
 // runs and the rest in short ones, as far as there is room for their sums.
-// Returns the doubles that it needs of the workspace.
-static int64_t sym_slab(int64_t n, int R, SymArgs &a, int64_t *blocks)
+static void sym_slab(int64_t n, int R, SymArgs &a, int64_t *blocks)
 {
     const int64_t T = 256 * R, RT = 4 * R, rows = div_up(n, T), slots = R == 4 ? 768 : 1024;
     const int64_t room = SYM_BYTES / 24;
@@ -730,15 +752,15 @@ static int64_t sym_slab(int64_t n, int R, SymArgs &a, int64_t *blocks)
     }
     *blocks = a.B1 + div_up(std::max<int64_t>(0, a.U - a.B1 * a.q1), a.q);
     a.part = a.col + 3 * cols;
-    return 3 * (cols + (*blocks + a.r1 - a.r0) * T);
 }
 
+// bytes of workspace that serve the sums of n particles and fewer (direct_bytes):
+// what one slab of all rows would take, with three rounds of runs
 static size_t sym_bytes(int64_t n, int R)
 {
-    SymArgs a{};
-    int64_t most = 0, blocks;
-    for (; a.r0 * 256 * R < n; a.r0 = a.r1) most = std::max(most, sym_slab(n, R, a, &blocks));
-    return sizeof(double) * (size_t)most;
+    const int64_t T = 256 * R, RT = 4 * R, rows = div_up(n, T), slots = R == 4 ? 768 : 1024, K = div_up(n, 64);
+    const int64_t runs = std::min<int64_t>(sym_first(rows, 0, K, RT), 3 * slots) + rows;
+    return (size_t)std::min<int64_t>(SYM_BYTES, 24 * (sym_col_first(rows - 1, 0, K, T) + runs * T));
 }
 
 template <int R>
@@ -765,12 +787,13 @@ static fss_status launch_sym(fss_ctx *ctx, const fss_particles *p, fss_velocity 
     return FSS_OK;
 }
 
-// buf: at least sym_bytes() or direct_plan().bytes; ts: the call's time stamps or null
+// buf: at least direct_bytes() and, for the sums that sym_targets takes, sym_bytes(); ts: the call's time stamps or null
 static fss_status launch_direct(fss_ctx *ctx, const fss_particles *p, const int64_t *idx, int64_t m,
                                 fss_velocity *out, bool mixed, void *buf, const RkNext &next, uint64_t *ts)
 {
     hipStream_t s = ctx->stream;
-    if (const int R = sym_targets(p, out, idx, mixed))
+    const int R = sym_targets(p->n, idx, mixed);
+    if (R && outputs_apart(p, out))
         return R == 2 ? launch_sym<2>(ctx, p, out, buf, next, ts) : launch_sym<4>(ctx, p, out, buf, next, ts);
     const DirectPlan P = direct_plan(p->n, m, mixed);
     DirectArgs a{p->x, p->y, p->z, p->vort, p->area, nullptr, idx, p->n, m, P.K, P.U, P.B1, P.q1, P.q, -1.0 / (4.0 * M_PI),
@@ -815,8 +838,8 @@ fss_status velocity_direct(fss_ctx *ctx, const fss_particles *p, const int64_t *
     if (!idx) m = n;
     const bool mixed = !force_fp64 && ctx->cfg.precision == FSS_MIXED;
     DevBuf &buf = ctx->direct;
-    const int R = sym_targets(p, out, idx, mixed);
-    FSS_TRY(buf.ensure(R ? sym_bytes(n, R) : direct_plan(n, m, mixed).bytes));
+    const int R = sym_targets(n, idx, mixed);
+    FSS_TRY(buf.ensure(std::max(direct_bytes(n, std::max(m, n), mixed), R ? sym_bytes(n, R) : 0)));
     if (ctx->capturing) return launch_direct(ctx, p, idx, m, out, mixed, buf.p, next, nullptr);
     Timing &t = ctx->timing;
     timing_begin(t, ctx->stream);

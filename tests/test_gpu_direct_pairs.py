@@ -133,3 +133,76 @@ def test_pair_sum_outputs_over_inputs_in_slabs(fsslib, orc, shift):
     got = [t.cpu().numpy() for t in fsslib.Context().velocity_direct(*d, *_dev(c[4]), out=out)]
     idx, ref = _sampled(orc, c)
     assert _err([g[idx] for g in got], ref) <= 1e-12
+
+
+@pytest.mark.parametrize("n", [5003, 20011, 70001])
+@pytest.mark.parametrize("first", ["apart", "over"])
+def test_captured_call_with_other_outputs(fsslib, n, first):
+    """An eager call sizes the workspace for a captured one of as many particles,
+    whether the outputs of either overlap the inputs (another kernel) or not."""
+    import torch
+    s = torch.cuda.Stream()
+    d = _dev(*_case(n, 6))
+    ctx = fsslib.Context(stream=s)
+    spare = [t.clone() for t in d[:4]]
+    want = [t.clone() for t in fsslib.Context().velocity_direct(*d)]
+    into = [torch.empty_like(t) for t in spare]
+    torch.cuda.synchronize()
+    print(f"direct pairs captured n={n} first={first}", flush=True)
+
+    def call(over):
+        # the inputs of a call over them are set again before each
+        x = spare if over else d[:4]
+        return ctx.velocity_direct(*x, d[4], out=spare if over else into)
+
+    call(first == "over")
+    torch.cuda.synchronize()
+    for a, b in zip(spare, d):
+        a.copy_(b)
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph, stream=s):
+        got = call(first != "over")
+    for _ in range(3):
+        for a, b in zip(spare, d):
+            a.copy_(b)
+        torch.cuda.synchronize()
+        graph.replay()
+        torch.cuda.synchronize()
+        assert _err([t.cpu().numpy() for t in got], [t.cpu().numpy() for t in want]) <= 1e-12
+
+
+@pytest.mark.parametrize("precision,eager,captured", [
+    (0, (20011, None), (15001, None)), (0, (60000, None), (45001, None)), (0, (2700, None), (2561, None)),
+    (0, (3350, None), (3250, None)), (1, (655361, None), (300001, None)), (1, (40000, None), (30011, None)),
+    (0, (20011, 100), (20011, 7001)), (0, (20011, 20011), (20011, 3001)), (0, (900001, None), (900001, 20011))])
+def test_captured_call_of_fewer_particles(fsslib, precision, eager, captured):
+    """An eager call sizes the workspace for every later one of as many particles or
+    fewer, whatever its targets: layouts differ, and a smaller sum may cut itself
+    into more runs."""
+    import torch
+    s = torch.cuda.Stream()
+    ctx = fsslib.Context(stream=s, precision=precision)
+    rng = np.random.default_rng(3)
+    print(f"direct captured precision={precision} eager={eager} captured={captured}", flush=True)
+
+    def case(n, m):
+        d = _dev(*_case(n, 6))
+        if m is None:
+            return lambda c: c.velocity_direct(*d)
+        idx = torch.from_numpy(rng.integers(0, n, m)).cuda()
+        return lambda c: c.velocity_direct_targets(*d, idx)
+
+    big, small = case(*eager), case(*captured)
+    want = [t.cpu().numpy() for t in small(fsslib.Context(precision=precision))]
+    torch.cuda.synchronize()
+    big(ctx)
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph, stream=s):
+        got = small(ctx)
+    for _ in range(3):
+        graph.replay()
+        torch.cuda.synchronize()
+        for g, w in zip(got, want):
+            np.testing.assert_array_equal(g.cpu().numpy(), w)
